@@ -421,7 +421,7 @@ def main():
                      "frac": achieved / HBM_PEAK_GBS,
                      "traffic": (LINE_SWEEP_TRAFFIC_RATIO * comp / max(cnt, 1)
                                  if LINE_SWEEP_TRAFFIC_RATIO else None),
-                     "kernel": "line sweep (k_line_solve*, k_line_pcr_solve, k_line_rhs*)",
+                     "kernel": "line sweep (k_line_solve*, k_line_rhs*)",
                      "bytes": "compulsory: a full sweep (4 colours) reads u and f and sigma-bar and writes u once, "
                               "3 Ne s + 3 Nc c; one colour launch a quarter",
                      "avg_launch_us": 1e3 * ms / max(cnt, 1), "launches": cnt,

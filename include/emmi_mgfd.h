@@ -236,9 +236,8 @@ int emmi_solver_blend_guess(emmi_solver_t *s, int n, const void *const *b, const
  * shape a solve of all the solver's slots issues -- precision, axis, line
  * length, lines per colour, right-hand sides per launch -- that the
  * process-wide table does not hold yet, times each substitution kernel
- * (one lane per line half; four lanes per line half with the right-hand
- * sides computed in the same launch; four lanes with a separate
- * right-hand-side launch) reps times on the slots' own vectors and records
+ * (16 lanes per line half on the matrix cores; one lane per line half) reps
+ * times on the slots' own vectors and records
  * the fastest; later launches of that shape use it (unless
  * emmi_set_line_kernel forces a kernel).  Overwrites the solver's vectors
  * (the next solve sets them) and drops its captured cycle graphs.  Returns
@@ -247,8 +246,8 @@ int emmi_solver_blend_guess(emmi_solver_t *s, int n, const void *const *b, const
  * in the last bits once the table holds entries. */
 int emmi_solver_autotune(emmi_solver_t *s, int reps);
 /* the table: rows[6k..6k+5] = value size (4 or 8), axis, line length (cells),
- * lines per colour, right-hand sides per launch, choice (0 one lane, 1 quad
- * fused, 2 quad separate); us[2k] = microseconds per launch of the choice,
+ * lines per colour, right-hand sides per launch, choice (0 one lane, 1
+ * matrix cores); us[2k] = microseconds per launch of the choice,
  * us[2k+1] of the built-in rule.  Returns the number of entries (may exceed
  * maxn) */
 int emmi_line_tuning(int *rows, double *us, int maxn);
@@ -389,11 +388,10 @@ int emmi_memcpy_d2h(void *dst, const void *src, size_t bytes);
 int emmi_memcpy_d2d(void *dst, const void *src, size_t bytes);
 int emmi_device_sync(void);
 /* Line-substitution kernel of the following launches (no counterpart in the
- * reference; for tests and tuning): 0 by line count (default), 1 one lane per
- * line half, 2 four lanes per line half, 3 four lanes with the right-hand
- * sides built by the substitution launch itself, 4 four lanes with the
- * right-hand sides built by a launch of their own.  All solve the same line
- * systems exactly.  Graphs a solver captured earlier keep the kernels they
+ * reference; for tests and tuning): 0 the matrix-core kernel wherever a line
+ * fits it (default; the autotuner's table is consulted), 1 one lane per line
+ * half, 2 to 4 the matrix-core kernel without the table.  All solve the same
+ * line systems exactly.  Graphs a solver captured earlier keep the kernels they
  * captured.  Returns the previous mode, or -1 for an unknown mode. */
 int emmi_set_line_kernel(int mode);
 /* kernel timing: accumulated milliseconds, launch counts and compulsory

@@ -4,13 +4,10 @@
 // (pb%2, pc%2); lines of one colour are independent.  Per colour the line
 // systems are factored once (k_line_factor: FREC values per node, depending
 // on grid, medium and frequency only) and every sweep then computes the
-// right-hand sides (k_line_rhs, SREC values per node) and runs a forward/back
-// substitution (k_line_solve).  Records hold values of type LineFac<T>::type
-// (factors) or LineScr<T>::type (line records) in 16-byte chunks: value k of node p of line l is element k % V of chunk
-// (p * nchunks + k / V) * nlines + l, V = 16 / sizeof(value), so a lane reads
-// its node with 16-byte loads and a wave's load covers contiguous memory.  A launch takes a pack of up to
-// LINE_PACK_MAX jobs (one per right-hand side or per level) that share the
-// axis and colour.
+// lines' right-hand sides and runs a forward/back substitution
+// (k_line_solve_m, or k_line_rhs* and k_line_solve).  A launch takes a pack of
+// up to LINE_PACK_MAX jobs (one per right-hand side or per level) that share
+// the axis and colour.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -35,8 +32,8 @@ struct LineJob {
   Level<T> L;
   typename cvec<T>::type* u;
   const typename cvec<T>::type* f;
-  typename LineFac<T>::type* fac;  // factor records of this colour, chunked: [n_a][FREC/V][nlines][V]
-  typename LineScr<T>::type* scr;  // right-hand side / substitution records, chunked: [n_a][SREC/V][nlines][V]
+  typename LineFac<T>::type* fac;  // factor records of this colour, line by line (HalfOrder)
+  typename LineScr<T>::type* scr;  // one-lane records, in 16-byte chunks: [n_a][SREC/V][nlines][V]
   int cb, cc;    // colour: parity of pb and pc (1 = odd)
   int nlo, nhi;  // lines of this colour along the low- and high-stride perpendicular axes
 };
@@ -64,11 +61,11 @@ inline void line_job_colour(LineJob<T>& J, int a, int colour) {
   line_colour_counts(J.L.n, a, colour, &J.nlo, &J.nhi);
 }
 
-// substitution kernel of later launches: 0 by line count (or by the
-// autotuner's table where it has the launch's shape), 1 one lane per line
-// half, 2 four lanes per line half, 3 four lanes building their own
-// right-hand sides, 4 four lanes after a right-hand-side launch; returns the
-// previous mode or -1
+// substitution kernel of later launches: 0 the matrix-core kernel where the
+// line fits its LDS records (or the autotuner's choice where its table has the
+// launch's shape), 1 the one-lane kernel, 2, 3, 4 as 0 without the table
+// (they named kernels that the matrix-core one replaced); returns the previous
+// mode or -1
 int set_line_kernel(int mode);
 
 // Autotuning: a launch shape (value size of the cycle precision, axis, line
@@ -76,7 +73,7 @@ int set_line_kernel(int mode);
 // fastest for it.  LINE_RULE: the built-in rule by line count.
 // LINE_RULE_ONLY (forced launches only): the rule, ignoring the table.
 enum LineChoice {
-  LINE_RULE_ONLY = -2, LINE_RULE = -1, LINE_ONE_LANE = 0, LINE_QUAD_FUSED = 1, LINE_QUAD_SEPARATE = 2, LINE_NCHOICE = 3
+  LINE_RULE_ONLY = -2, LINE_RULE = -1, LINE_ONE_LANE = 0, LINE_MATRIX = 1, LINE_NCHOICE = 2
 };
 struct LineShape {
   int esize, axis, n;
@@ -92,9 +89,6 @@ struct LineShape {
 };
 template <typename T>
 LineShape line_shape(const LinePack<T>& P, int axis);
-// single-line launches (cyclic reduction) have no choice to tune
-template <typename T>
-bool line_pcr_shape(const LinePack<T>& P, int axis);
 void set_line_choice(const LineShape& k, int choice, double us_choice, double us_rule);
 bool has_line_choice(const LineShape& k);
 void clear_line_choices();

@@ -14,19 +14,20 @@
 //     D_p = K_p - v v^T (1/d_{p-1} + 1/d_p),   B_p = diag(l_{p-1}) + v v^T / d_{p-1}
 //     W_1 = D_1,  W_p = D_p - B_p W_{p-1}^{-1} B_p
 // whose factors depend on the grid, the medium and the frequency only.
-// k_line_factor stores, per node, W_p^{-1} (symmetric, 10 entries) and
-// 1/d_p once; k_line_rhs computes the residuals sigma_p, rho_p of the lines
-// and k_line_solve then runs, per sweep,
+// k_line_factor stores, per node, W_p^{-1} (symmetric, 10 entries) and 1/d
+// once; a sweep then computes the residuals sigma_p, rho_p of the lines and
+// runs
 //     y_p = g_p - B_p z_{p-1},  z_p = W_p^{-1} y_p          (forward)
 //     da_p = z_p - W_p^{-1} B_{p+1} da_{p+1},
 //     dE_a(p) = rho_p/d_p + v.(da_{p+1} - da_p) / d_p        (backward)
-// with g_p = sigma_p + v (rho_{p-1}/d_{p-1} - rho_p/d_p) from the residual.
+// with g_p = sigma_p + v (rho_{p-1}/d_{p-1} - rho_p/d_p) from the residual:
+// k_line_solve_m does all of it in one launch on the matrix cores,
+// k_line_rhs* and k_line_solve (one lane per line half) take the lines too
+// long for its LDS and serve as its check.
 // Lines of one colour (pb%2, pc%2) are not coupled, so a launch sweeps one
-// colour; every kernel computes in FP64 whatever the storage precision.
-// Records hold LineFac<T> / LineScr<T> values in 16-byte chunks (layout in
-// line_kernels.h);
-// the substitution keeps a ring of the next D nodes' chunks in registers, so
-// D nodes of loads are in flight while a node is computed.
+// colour; every kernel computes in FP64 whatever the storage precision.  The
+// substitutions keep a ring of the next D nodes' factor records in registers,
+// so D nodes of loads are in flight while a node is computed.
 #include "line_kernels.h"
 
 #include <hip/hip_ext.h>
@@ -36,6 +37,7 @@
 #include <cstdint>
 #include <map>
 #include <mutex>
+#include <set>
 #include <utility>
 #include "stencil.h"
 #include "timing.h"
@@ -71,42 +73,6 @@ template <typename T> using ScrRec = typename LineScr<T>::type;
 #define EMMI_LINE_RING_F64 1
 #endif
 template <typename T> constexpr int ring_depth() { return sizeof(T) == 4 ? EMMI_LINE_RING_F32 : EMMI_LINE_RING_F64; }
-// Launches of at most this many lines per job (FP32-storage / FP64 cycles)
-// use the quad-lane substitution, whose ring holds EMMI_LINE_QUAD_RING nodes.
-#ifndef EMMI_LINE_QUAD_MAX_LINES_F32
-#define EMMI_LINE_QUAD_MAX_LINES_F32 4096
-#endif
-#ifndef EMMI_LINE_QUAD_MAX_LINES_F64
-#define EMMI_LINE_QUAD_MAX_LINES_F64 4096
-#endif
-#ifndef EMMI_LINE_QUAD_RING
-#define EMMI_LINE_QUAD_RING 3
-#endif
-// quad-lane launches of at most this many lines per job (FP32-storage /
-// FP64 cycles) compute their right-hand sides themselves (no k_line_rhs
-// launch)
-#ifndef EMMI_LINE_FUSE_MAX_LINES_F32
-#define EMMI_LINE_FUSE_MAX_LINES_F32 4096
-#endif
-#ifndef EMMI_LINE_FUSE_MAX_LINES_F64
-#define EMMI_LINE_FUSE_MAX_LINES_F64 4096
-#endif
-// threads of a block of the fused launches (a multiple of 128; the waves
-// beyond the first two only compute right-hand sides)
-#ifndef EMMI_LINE_FUSE_THREADS
-#define EMMI_LINE_FUSE_THREADS 512
-#endif
-// the same for lines of 64 nodes and more
-#ifndef EMMI_LINE_FUSE_THREADS_LONG
-#define EMMI_LINE_FUSE_THREADS_LONG 256
-#endif
-template <typename T> constexpr int fuse_max_lines() {
-  return sizeof(T) == 4 ? EMMI_LINE_FUSE_MAX_LINES_F32 : EMMI_LINE_FUSE_MAX_LINES_F64;
-}
-template <typename T> constexpr int quad_max_lines() {
-  return sizeof(T) == 4 ? EMMI_LINE_QUAD_MAX_LINES_F32 : EMMI_LINE_QUAD_MAX_LINES_F64;
-}
-
 // value k of a node's chunks, as double
 template <typename R, int NC>
 __device__ __forceinline__ double val(const Ch<R> (&c)[NC], int k) {
@@ -249,9 +215,41 @@ __device__ __forceinline__ void sub_bwb(cxd (&D)[4][4], const cxd (&Wi)[4][4], c
     for (int j = 0; j < 4; j++) D[i][j] -= Pm[i][j] * l[i] + (vP[j] * rd) * v[i];
 }
 
-// inverts D in place and stores the symmetric part with 1/d of node p
+// The factor records of a line stand in the order of the substitution: the
+// two halves one after the other, each from its boundary node towards the
+// meeting node m = N/2, then the meeting node,
+//     record t            (t < T)   node t - (T - m)       (top half)
+//     record T + t                  node N + (T - H) - t   (bottom half)
+//     record 2 T                    node m
+// with H = N - m.  A record holds the node's inverse block and 1/d of its
+// inner edge (towards m): edge p of a top node p, edge p - 1 of a bottom
+// node.  T is H rounded up to whole groups of line_ring nodes (the
+// substitution loads and unrolls by groups); the boundary nodes and the
+// records before them hold zero inverses, so that their corrections are zero.
+// The group is 8 nodes where that pads a half by no more than an eighth, else
+// 4, and 2 for halves of at most two nodes (a single group: the back pass
+// reloads a slot one step late, which a ring of two could not wait for).
+__host__ __device__ __forceinline__ int line_ring(int N) {
+  const int H = N - N / 2;
+  return (8 - H % 8) % 8 <= H / 8 ? 8 : H > 2 ? 4 : 2;
+}
+struct HalfOrder {
+  int N, m, T, o, ob;   // o, ob: t of the boundary node on top and below
+  __host__ __device__ explicit HalfOrder(int n) : N(n), m(n / 2) {
+    const int H = N - m, D = line_ring(N);
+    T = (H + D - 1) / D * D;
+    o = T - m;
+    ob = T - H;
+  }
+  __host__ __device__ int records() const { return 2 * T + 1; }
+  // record of node p (0..N) and the record that holds 1/d of edge e (0..N-1)
+  __host__ __device__ int node(int p) const { return p < m ? p + o : p > m ? T + N + ob - p : 2 * T; }
+  __host__ __device__ int edge(int e) const { return e < m ? e + o : T + N + ob - e - 1; }
+};
+
+// inverts D in place and stores the symmetric part with 1/d of the inner edge
 template <typename R>
-__device__ __forceinline__ void store_factor(Ch<R>* rec, long stride, int p, cxd (&D)[4][4], cxd rd) {
+__device__ __forceinline__ void store_factor(Ch<R>* r, cxd (&D)[4][4], cxd rd) {
   constexpr int FC = fchunks<R>();
   inv4(D);
   Ch<R> c[FC] = {};
@@ -266,9 +264,8 @@ __device__ __forceinline__ void store_factor(Ch<R>* rec, long stride, int p, cxd
     }
   put(c, 20, rd.re);
   put(c, 21, rd.im);
-  Ch<R>* r = rec + (long)p * FC * stride;
 #pragma unroll
-  for (int k = 0; k < FC; k++) r[k * stride] = c[k];
+  for (int k = 0; k < FC; k++) r[k] = c[k];
 }
 
 // Twisted factorization of each line, meeting at node m = N/2 of the nodes
@@ -276,12 +273,11 @@ __device__ __forceinline__ void store_factor(Ch<R>* rec, long stride, int p, cxd
 //   top     W_1 = D_1,  W_p = D_p - B_p W_{p-1}^-1 B_p        p = 2..m-1
 //   bottom  U_M = D_M,  U_p = D_p - B_{p+1} U_{p+1}^-1 B_{p+1}  p = M-1..m+1
 //   middle  S_m = D_m - B_m W_{m-1}^-1 B_m - B_{m+1} U_{m+1}^-1 B_{m+1}
-// Node p stores the inverse of its factor (W, S or U) and 1/d_p; node 0
-// stores 1/d_0.
+// The records (HalfOrder) take the inverse of each node's factor (W, S or U).
 template <typename T, int A>
 __global__ void __launch_bounds__(64) k_line_factor(LinePack<T> P) {
   using R = FacRec<T>;
-  constexpr int FC = fchunks<R>(), V = Ch<R>::V;
+  constexpr int FC = fchunks<R>();
   const LineJob<T>& J = P.job[blockIdx.y];
   const Level<T>& L = J.L;
   const int tid = blockIdx.x * blockDim.x + threadIdx.x;
@@ -291,16 +287,21 @@ __global__ void __launch_bounds__(64) k_line_factor(LinePack<T> P) {
   const int N = G.N;
   if (N < 2) return;
   const int M = N - 1, m = N / 2;
-  const long stride = (long)J.nlo * J.nhi;
-  Ch<R>* rec = reinterpret_cast<Ch<R>*>(J.fac) + tid;
-  const cxd rd0 = cinv(G.d_edge(L, 0));
-  {
-    // node 0 holds only 1/d_0 (values 20, 21: one chunk)
+  const HalfOrder O(N);
+  Ch<R>* rec = reinterpret_cast<Ch<R>*>(J.fac) + (long)tid * O.records() * FC;
+  const cxd rd0 = cinv(G.d_edge(L, 0)), rdM = cinv(G.d_edge(L, M));
+  // boundary nodes and the padding before them
+  auto zero_rec = [&](int r, cxd rd) {
     Ch<R> c[FC] = {};
-    put(c, 20, rd0.re);
-    put(c, 21, rd0.im);
-    rec[(20 / V) * stride] = c[20 / V];
-  }
+    put(c, 20, rd.re);
+    put(c, 21, rd.im);
+#pragma unroll
+    for (int k = 0; k < FC; k++) rec[r * FC + k] = c[k];
+  };
+  for (int t = 0; t < O.o; t++) zero_rec(t, cxd(0, 0));
+  for (int t = 0; t < O.ob; t++) zero_rec(O.T + t, cxd(0, 0));
+  zero_rec(O.o, rd0);
+  zero_rec(O.T + O.ob, rdM);
   cxd Wt[4][4], Wb[4][4], Dm[4][4];
   double l[4];
   cxd rd_prev = rd0;
@@ -311,7 +312,7 @@ __global__ void __launch_bounds__(64) k_line_factor(LinePack<T> P) {
       G.lcoef(L, p - 1, l);
       sub_bwb(Dm, Wt, l, rd_prev, G.v);
     }
-    store_factor(rec, stride, p, Dm, rd);
+    store_factor(rec + O.node(p) * FC, Dm, rd);
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
@@ -325,7 +326,7 @@ __global__ void __launch_bounds__(64) k_line_factor(LinePack<T> P) {
       G.lcoef(L, p, l);
       sub_bwb(Dm, Wb, l, rdp, G.v);
     }
-    store_factor(rec, stride, p, Dm, rdp);
+    store_factor(rec + O.node(p) * FC, Dm, rdm);
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
@@ -342,271 +343,7 @@ __global__ void __launch_bounds__(64) k_line_factor(LinePack<T> P) {
       G.lcoef(L, m, l);
       sub_bwb(Dm, Wb, l, rdp, G.v);
     }
-    store_factor(rec, stride, m, Dm, rdp);
-  }
-}
-
-// ---------------------------------------------------------------------------
-// single-line launches: parallel cyclic reduction
-// ---------------------------------------------------------------------------
-// The coarsest level of a semi-coarsening pattern is one line along the
-// kept axis (the full grid length), so the substitution would be one serial
-// chain of N/2 nodes per half.  With one line per launch, the node system
-//     B_p x_{p-1} + D_p x_p + B_{p+1} x_{p+1} = g_p,   p = 1..M, x_0 = x_N = 0
-// is reduced instead: at stride s = 1, 2, 4, ... each equation eliminates its
-// neighbours at distance s,
-//     alpha_p = -A_p D_{p-s}^-1,  gamma_p = -C_p D_{p+s}^-1
-//     D_p <- D_p + alpha_p C_{p-s} + gamma_p A_{p+s},  A_p <- alpha_p A_{p-s},
-//     C_p <- gamma_p C_{p+s},  g_p <- g_p + alpha_p g_{p-s} + gamma_p g_{p+s}
-// (A_p couples p to p-s, C_p to p+s, both start as the line's B), until no
-// coupling is left and x_p = D_p^-1 g_p.  k_line_pcr_factor builds alpha,
-// gamma and D^-1 once per frequency; k_line_pcr_solve then takes log2(M)
-// block-wide steps.  Launches of one line of up to PCR_MAX_NODES nodes use it.
-constexpr int PCR_MAX_NODES = 256;
-
-__host__ __device__ constexpr int pcr_levels(int M) {
-  int k = 0;
-  for (int s = 1; s < M; s *= 2) k++;
-  return k;
-}
-// complex entries of the factor buffer: alpha and gamma per level and node,
-// D^-1 and 1/d per node, two work copies of (D, A, C) per node
-__host__ __device__ constexpr long pcr_entries(int N) {
-  return (long)N * (32L * pcr_levels(N - 1) + 16 + 1 + 2 * 48);
-}
-
-struct PcrLayout {
-  cxd *alpha, *dinv, *rd, *work;
-  int N, nlev;
-  __device__ PcrLayout(void* base, int N_) : N(N_), nlev(pcr_levels(N_ - 1)) {
-    cxd* b = reinterpret_cast<cxd*>(base);
-    alpha = b;                                   // [lev][p][2][16]: alpha, gamma
-    dinv = alpha + (long)nlev * N * 32;          // [p][16]
-    rd = dinv + (long)N * 16;                    // [e]
-    work = rd + N;                               // [2][p][48]: D, A, C
-  }
-  __device__ cxd* ag(int lev, int p, int which) const { return alpha + (((long)lev * N + p) * 2 + which) * 16; }
-  __device__ cxd* w(int buf, int p) const { return work + ((long)buf * N + p) * 48; }
-};
-
-__device__ __forceinline__ void ld16(const cxd* s, cxd (&M)[4][4]) {
-#pragma unroll
-  for (int i = 0; i < 4; i++)
-#pragma unroll
-    for (int j = 0; j < 4; j++) M[i][j] = s[4 * i + j];
-}
-__device__ __forceinline__ void st16(cxd* d, const cxd (&M)[4][4]) {
-#pragma unroll
-  for (int i = 0; i < 4; i++)
-#pragma unroll
-    for (int j = 0; j < 4; j++) d[4 * i + j] = M[i][j];
-}
-// C = A B
-__device__ __forceinline__ void mm4(const cxd (&A)[4][4], const cxd (&B)[4][4], cxd (&C)[4][4]) {
-#pragma unroll
-  for (int i = 0; i < 4; i++)
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      cxd acc(0, 0);
-#pragma unroll
-      for (int k = 0; k < 4; k++) acc += A[i][k] * B[k][j];
-      C[i][j] = acc;
-    }
-}
-__device__ __forceinline__ void zero4(cxd (&M)[4][4]) {
-#pragma unroll
-  for (int i = 0; i < 4; i++)
-#pragma unroll
-    for (int j = 0; j < 4; j++) M[i][j] = cxd(0, 0);
-}
-// the coupling B = diag(l) + v v^T rd of two neighbouring nodes
-template <typename T, int A>
-__device__ __forceinline__ void coupling(const Level<T>& L, const LineGeo<T, A>& G, int e, cxd rd, cxd (&Bm)[4][4]) {
-  double l[4];
-  G.lcoef(L, e, l);
-#pragma unroll
-  for (int i = 0; i < 4; i++)
-#pragma unroll
-    for (int j = 0; j < 4; j++) Bm[i][j] = (G.v[i] * G.v[j]) * rd + cxd(i == j ? l[i] : 0.0, 0);
-}
-
-template <typename T, int A>
-__global__ void __launch_bounds__(PCR_MAX_NODES) k_line_pcr_factor(LinePack<T> P) {
-  const LineJob<T>& J = P.job[blockIdx.y];
-  const Level<T>& L = J.L;
-  int pb, pc;
-  if (!line_of<T, A>(J, 0, pb, pc)) return;   // uniform over the block
-  const LineGeo<T, A> G(L, pb, pc);
-  const int N = G.N;
-  if (N < 2 || N > PCR_MAX_NODES) return;     // uniform
-  const int M = N - 1, p = threadIdx.x;
-  const PcrLayout F(J.fac, N);
-  for (int e = p; e <= M; e += blockDim.x) F.rd[e] = cinv(G.d_edge(L, e));
-  __syncthreads();
-  const bool own = p >= 1 && p <= M;
-  if (own) {
-    cxd Dm[4][4], Am[4][4], Cm[4][4];
-    diag_block(L, G, p, F.rd[p - 1], F.rd[p], Dm);
-    if (p >= 2) coupling(L, G, p - 1, F.rd[p - 1], Am);
-    else zero4(Am);
-    if (p <= M - 1) coupling(L, G, p, F.rd[p], Cm);
-    else zero4(Cm);
-    cxd* w = F.w(0, p);
-    st16(w, Dm);
-    st16(w + 16, Am);
-    st16(w + 32, Cm);
-  }
-  __syncthreads();
-  int cur = 0, lev = 0;
-  for (int s = 1; s < M; s *= 2, lev++) {
-    if (own) {
-      cxd Dm[4][4], Am[4][4], Cm[4][4], al[4][4], ga[4][4], t[4][4], u[4][4];
-      const cxd* w = F.w(cur, p);
-      ld16(w, Dm);
-      ld16(w + 16, Am);
-      ld16(w + 32, Cm);
-      cxd An[4][4], Cn[4][4];
-      zero4(An);
-      zero4(Cn);
-      if (p - s >= 1) {
-        const cxd* wm = F.w(cur, p - s);
-        ld16(wm, t);
-        inv4(t);
-        mm4(Am, t, al);
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-          for (int j = 0; j < 4; j++) al[i][j] = -al[i][j];
-        ld16(wm + 32, t);   // C_{p-s}
-        mm4(al, t, u);
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-          for (int j = 0; j < 4; j++) Dm[i][j] += u[i][j];
-        ld16(wm + 16, t);   // A_{p-s}
-        mm4(al, t, An);
-      } else {
-        zero4(al);
-      }
-      if (p + s <= M) {
-        const cxd* wp = F.w(cur, p + s);
-        ld16(wp, t);
-        inv4(t);
-        mm4(Cm, t, ga);
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-          for (int j = 0; j < 4; j++) ga[i][j] = -ga[i][j];
-        ld16(wp + 16, t);   // A_{p+s}
-        mm4(ga, t, u);
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-          for (int j = 0; j < 4; j++) Dm[i][j] += u[i][j];
-        ld16(wp + 32, t);   // C_{p+s}
-        mm4(ga, t, Cn);
-      } else {
-        zero4(ga);
-      }
-      st16(F.ag(lev, p, 0), al);
-      st16(F.ag(lev, p, 1), ga);
-      cxd* wn = F.w(cur ^ 1, p);
-      st16(wn, Dm);
-      st16(wn + 16, An);
-      st16(wn + 32, Cn);
-    }
-    __syncthreads();
-    cur ^= 1;
-  }
-  if (own) {
-    cxd Dm[4][4];
-    ld16(F.w(cur, p), Dm);
-    inv4(Dm);
-    st16(F.dinv + (long)p * 16, Dm);
-  }
-}
-
-template <typename T, int A>
-__global__ void __launch_bounds__(4 * PCR_MAX_NODES) k_line_pcr_solve(LinePack<T> P) {
-  using RS = ScrRec<T>;
-  constexpr int SC = schunks<RS>();
-  // LDS holds the complex values as double2 (cxd has a constructor)
-  __shared__ double2 g_[2][PCR_MAX_NODES][4];
-  __shared__ double2 xs_[PCR_MAX_NODES + 1][4];
-  __shared__ double2 qs_[PCR_MAX_NODES];
-  auto get = [](const double2& a) { return cxd(a.x, a.y); };
-  auto set = [](double2& a, cxd v) { a.x = v.re; a.y = v.im; };
-  const LineJob<T>& J = P.job[blockIdx.y];
-  const Level<T>& L = J.L;
-  int pb, pc;
-  if (!line_of<T, A>(J, 0, pb, pc)) return;   // uniform over the block
-  const LineGeo<T, A> G(L, pb, pc);
-  const int N = G.N;
-  if (N < 2 || N > PCR_MAX_NODES) return;     // uniform
-  const int M = N - 1, tid = threadIdx.x;
-  const PcrLayout F(J.fac, N);
-  // residual records of the line's nodes (as k_line_rhs writes them)
-  for (int p = tid; p <= M; p += blockDim.x) node_rhs<T, A>(J, 0, pb, pc, p, 1);
-  __syncthreads();   // the records are complete (workgroup scope)
-  const Ch<RS>* rec = reinterpret_cast<const Ch<RS>*>(J.scr);
-  for (int e = tid; e <= M; e += blockDim.x) {
-    Ch<RS> c[SC];
-#pragma unroll
-    for (int k = 0; k < SC; k++) c[k] = rec[(long)e * SC + k];
-    set(qs_[e], cval(c, 8) * F.rd[e]);
-  }
-  __syncthreads();
-  const int p = tid / 4 + 1, r = tid % 4;
-  const bool own = p <= M;
-  if (own) {
-    Ch<RS> c[SC];
-#pragma unroll
-    for (int k = 0; k < SC; k++) c[k] = rec[(long)p * SC + k];
-    set(g_[0][p][r], cval(c, 2 * r) + (get(qs_[p - 1]) - get(qs_[p])) * G.v[r]);
-  }
-  __syncthreads();
-  int cur = 0, lev = 0;
-  for (int s = 1; s < M; s *= 2, lev++) {
-    if (own) {
-      cxd acc = get(g_[cur][p][r]);
-      if (p - s >= 1) {
-        const cxd* a = F.ag(lev, p, 0) + 4 * r;
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc += a[j] * get(g_[cur][p - s][j]);
-      }
-      if (p + s <= M) {
-        const cxd* a = F.ag(lev, p, 1) + 4 * r;
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc += a[j] * get(g_[cur][p + s][j]);
-      }
-      set(g_[cur ^ 1][p][r], acc);
-    }
-    __syncthreads();
-    cur ^= 1;
-  }
-  if (own) {
-    const cxd* di = F.dinv + (long)p * 16 + 4 * r;
-    cxd acc(0, 0);
-#pragma unroll
-    for (int j = 0; j < 4; j++) acc += di[j] * get(g_[cur][p][j]);
-    set(xs_[p][r], acc);
-  }
-  if (tid < 4) {
-    set(xs_[0][tid], cxd(0, 0));
-    set(xs_[N][tid], cxd(0, 0));
-  }
-  __syncthreads();
-  typename cvec<T>::type* __restrict__ u = J.u;
-  if (own) {
-    const long o = (r == 0 ? G.ob0 : r == 1 ? G.ob1 : r == 2 ? G.oc0 : G.oc1) + (long)p * G.sa;
-    st<T>(u, o, ld<T>(u, o) + get(xs_[p][r]));
-  }
-  for (int e = tid; e <= M; e += blockDim.x) {
-    cxd dv(0, 0);
-#pragma unroll
-    for (int i = 0; i < 4; i++) dv += (get(xs_[e + 1][i]) - get(xs_[e][i])) * G.v[i];
-    const long o = G.oa + (long)e * G.sa;
-    st<T>(u, o, ld<T>(u, o) + (get(qs_[e]) + dv * F.rd[e]));
+    store_factor(rec + O.node(m) * FC, Dm, cxd(0, 0));
   }
 }
 
@@ -634,9 +371,8 @@ __device__ __forceinline__ void symv(const Ch<R> (&w)[NC], const cxd (&y)[4], cx
 // solve of the colour starts from.
 // the records of node p of line `line` (at (pb, pc)) of job J
 // the ten values of that record (node 0: rho only, the rest zero)
-template <typename T, int A>
-__device__ __forceinline__ void node_rhs_rec(const LineJob<T>& J, int pb, int pc, int p,
-                                             Ch<ScrRec<T>> (&c)[schunks<ScrRec<T>>()]) {
+template <typename T, int A, typename RS>
+__device__ __forceinline__ void node_rhs_rec(const LineJob<T>& J, int pb, int pc, int p, Ch<RS> (&c)[schunks<RS>()]) {
   constexpr int B = (A + 1) % 3, C = (A + 2) % 3;
   const Level<T>& L = J.L;
   const typename cvec<T>::type* __restrict__ u = J.u;
@@ -773,10 +509,9 @@ __device__ __forceinline__ void win_row(const MarchWin& w, cxd (&v)[13]) {
 // rows' arithmetic is row_arith in both).  Every position read lies in the
 // level: nodes -1 .. N along the line are read only where node_rhs_rec reads
 // them (da = -1 from node 1 on).
-template <typename T, int A, typename Sink>
+template <typename T, int A, typename RS = ScrRec<T>, typename Sink>
 __device__ __forceinline__ void line_rhs_march(const LineJob<T>& J, int pb, int pc, int p0, int p1,
                                                const Sink& sink) {
-  using RS = ScrRec<T>;
   constexpr int B = (A + 1) % 3, C = (A + 2) % 3;
   const Level<T>& L = J.L;
   const typename cvec<T>::type* __restrict__ u = J.u;
@@ -1102,11 +837,14 @@ __global__ void __launch_bounds__(128) k_line_solve(LinePack<T> P) {
   LineGeo<T, A> G;
   if (live) G.init(L, pb, pc);
   const long stride = (long)J.nlo * J.nhi;
-  const Ch<RF>* __restrict__ fac = reinterpret_cast<const Ch<RF>*>(J.fac) + line;
+  const HalfOrder O(N);
+  const Ch<RF>* __restrict__ fac = reinterpret_cast<const Ch<RF>*>(J.fac) + (long)line * O.records() * FC;
+  auto fnode = [&](int p) { return fac + O.node(p) * FC; };            // the node's inverse, 1/d of its inner edge
+  auto fedge = [&](int e) { return fac[O.edge(e) * FC + CD]; };        // 1/d of an edge
   Ch<RS>* __restrict__ scr = reinterpret_cast<Ch<RS>*>(J.scr) + line;
   E* __restrict__ u = J.u;
   const double* __restrict__ iw = L.IW[A];
-  const long fstep = (long)FC * stride, sstep = (long)SC * stride;
+  const long sstep = (long)SC * stride;
   const long off_u[5] = {G.oa, G.ob0, G.ob1, G.oc0, G.oc1};
 
   // D nodes ahead are in flight: the load for node p + D goes into the slot
@@ -1125,11 +863,11 @@ __global__ void __launch_bounds__(128) k_line_solve(LinePack<T> P) {
 #pragma unroll
     for (int d = 0; d < D; d++) {
       const int pn = max(min(1 + d, last), 1);
-      load_node(rf[d], fac + pn * fstep, stride);
+      load_node(rf[d], fnode(pn), 1);
       load_node(rs[d], scr + pn * sstep, stride);
       riw[d] = iw[pn - 1];
     }
-    const Ch<RF> f0 = fac[CD * stride];
+    const Ch<RF> f0 = fedge(0);
     const Ch<RS> s0 = scr[CQ * stride];
     cxd rd_prev((double)f0.v[20 % VF], (double)f0.v[21 % VF]);
     cxd q_prev = cxd((double)s0.v[8 % VS], (double)s0.v[9 % VS]) * rd_prev;
@@ -1140,7 +878,7 @@ __global__ void __launch_bounds__(128) k_line_solve(LinePack<T> P) {
       const double iWe = (double)riw[d];
       {
         const int pn = min(p + D, last), dn = (d + D) % R;
-        load_node(rf[dn], fac + pn * fstep, stride);
+        load_node(rf[dn], fnode(pn), 1);
         load_node(rs[dn], scr + pn * sstep, stride);
         riw[dn] = iw[pn - 1];
       }
@@ -1178,16 +916,16 @@ __global__ void __launch_bounds__(128) k_line_solve(LinePack<T> P) {
       if (p0 + d <= last) step(p0 + d, d);
     if (m >= 2) bmul(G, z, (double)iw[m - 1], rd_prev, tm);   // B_m z_{m-1}
   } else if (live) {
-    // ring entries also carry rho_{p-1} and 1/d_{p-1} of the node above
+    // ring entries also carry rho_{p-1} of the node above and 1/d_p
     Ch<RF> rdn[R];
     Ch<RS> rqn[R];
     const int last = m + 1;
 #pragma unroll
     for (int d = 0; d < D; d++) {
       const int pn = min(max(M - d, last), M);
-      load_node(rf[d], fac + pn * fstep, stride);
+      load_node(rf[d], fnode(pn), 1);
       load_node(rs[d], scr + pn * sstep, stride);
-      rdn[d] = fac[(pn - 1) * fstep + CD * stride];
+      rdn[d] = fedge(pn);
       rqn[d] = scr[(pn - 1) * sstep + CQ * stride];
       riw[d] = iw[pn];
     }
@@ -1195,20 +933,20 @@ __global__ void __launch_bounds__(128) k_line_solve(LinePack<T> P) {
     auto step = [&](const int p, const int d) {
       const Ch<RF>(&cf)[FC] = rf[d];
       const Ch<RS>(&cr)[SC] = rs[d];
-      const Ch<RF>& cdm = rdn[d];
+      const Ch<RF>& cdp = rdn[d];
       const Ch<RS>& cqm = rqn[d];
       const double iWe = (double)riw[d];
       {
         const int pn = max(p - D, last), dn = (d + D) % R;
-        load_node(rf[dn], fac + pn * fstep, stride);
+        load_node(rf[dn], fnode(pn), 1);
         load_node(rs[dn], scr + pn * sstep, stride);
-        rdn[dn] = fac[(pn - 1) * fstep + CD * stride];
+        rdn[dn] = fedge(pn);
         rqn[dn] = scr[(pn - 1) * sstep + CQ * stride];
         riw[dn] = iw[pn];
       }
-      const cxd rd = cval(cf, 20);
+      const cxd rd((double)cdp.v[20 % VF], (double)cdp.v[21 % VF]);
       const cxd q = cval(cr, 8) * rd;
-      const cxd rdm((double)cdm.v[20 % VF], (double)cdm.v[21 % VF]);
+      const cxd rdm = cval(cf, 20);
       const cxd qm = cxd((double)cqm.v[8 % VS], (double)cqm.v[9 % VS]) * rdm;
       const cxd dq = qm - q;
       cxd g[4];
@@ -1254,11 +992,11 @@ __global__ void __launch_bounds__(128) k_line_solve(LinePack<T> P) {
   {
     Ch<RF> cf[FC];
           Ch<RS> cr[SC];
-    load_node(cf, fac + m * fstep, stride);
+    load_node(cf, fnode(m), 1);
     load_node(cr, scr + m * sstep, stride);
-    const Ch<RF> cdm = fac[(m - 1) * fstep + CD * stride];
+    const Ch<RF> cdm = fedge(m - 1), cdp = fedge(m);
     const Ch<RS> cqm = scr[(m - 1) * sstep + CQ * stride];
-    rdmid = cval(cf, 20);
+    rdmid = cxd((double)cdp.v[20 % VF], (double)cdp.v[21 % VF]);
     qmid = cval(cr, 8) * rdmid;
     const cxd rdm((double)cdm.v[20 % VF], (double)cdm.v[21 % VF]);
     const cxd dq = cxd((double)cqm.v[8 % VS], (double)cqm.v[9 % VS]) * rdm - qmid;
@@ -1284,7 +1022,7 @@ __global__ void __launch_bounds__(128) k_line_solve(LinePack<T> P) {
 #pragma unroll
     for (int d = 0; d < D; d++) {
       const int pn = max(last - d, 1);
-      load_node(rf[d], fac + pn * fstep, stride);
+      load_node(rf[d], fnode(pn), 1);
       load_node(rs[d], scr + pn * sstep, stride);
       riw[d] = iw[pn];
       if constexpr (A != 0) {
@@ -1302,7 +1040,7 @@ __global__ void __launch_bounds__(128) k_line_solve(LinePack<T> P) {
       const double iWe = (double)riw[d];
       {
         const int pn = max(p - D, 1), dn = (d + D) % R;
-        load_node(rf[dn], fac + pn * fstep, stride);
+        load_node(rf[dn], fnode(pn), 1);
         load_node(rs[dn], scr + pn * sstep, stride);
         riw[dn] = iw[pn];
         if constexpr (A != 0) {
@@ -1343,7 +1081,7 @@ __global__ void __launch_bounds__(128) k_line_solve(LinePack<T> P) {
     for (int d = 0; d < R - 1; d++)
       if (p0 - d >= 1) step(p0 - d, d);
     // along-line edge 0, between the boundary node and node 1
-    const Ch<RF> f0 = fac[CD * stride];
+    const Ch<RF> f0 = fedge(0);
     const Ch<RS> s0 = scr[CQ * stride];
     const cxd rd0((double)f0.v[20 % VF], (double)f0.v[21 % VF]);
     const cxd q0 = cxd((double)s0.v[8 % VS], (double)s0.v[9 % VS]) * rd0;
@@ -1353,10 +1091,12 @@ __global__ void __launch_bounds__(128) k_line_solve(LinePack<T> P) {
     st<T>(u, G.oa, ld<T>(u, G.oa) + (q0 + dv * rd0));
   } else {
     const int last = m + 1;
+    Ch<RF> rdn[R];   // 1/d_p of the ring nodes
 #pragma unroll
     for (int d = 0; d < D; d++) {
       const int pn = min(last + d, M);
-      load_node(rf[d], fac + pn * fstep, stride);
+      load_node(rf[d], fnode(pn), 1);
+      rdn[d] = fedge(pn);
       load_node(rs[d], scr + pn * sstep, stride);
       riw[d] = iw[pn - 1];
       if constexpr (A != 0) {
@@ -1376,7 +1116,8 @@ __global__ void __launch_bounds__(128) k_line_solve(LinePack<T> P) {
       const double iWe = (double)riw[d];
       {
         const int pn = min(p + D, M), dn = (d + D) % R;
-        load_node(rf[dn], fac + pn * fstep, stride);
+        load_node(rf[dn], fnode(pn), 1);
+        rdn[dn] = fedge(pn);
         load_node(rs[dn], scr + pn * sstep, stride);
         riw[dn] = iw[pn - 1];
         if constexpr (A != 0) {
@@ -1385,7 +1126,7 @@ __global__ void __launch_bounds__(128) k_line_solve(LinePack<T> P) {
           for (int k = 1; k < 5; k++) ru[dn][k] = u[off_u[k] + (long)pn * G.sa];
         }
       }
-      const cxd rd = cval(cf, 20);
+      const cxd rd((double)rdn[d].v[20 % VF], (double)rdn[d].v[21 % VF]);
       const cxd q = cval(cr, 8) * rd;
       cxd t[4], wt[4], ap[4];
       bmul(G, xp, iWe, rdm, t);
@@ -1429,533 +1170,378 @@ __global__ void __launch_bounds__(128) k_line_solve(LinePack<T> P) {
 }
 
 // ---------------------------------------------------------------------------
-// quad-lane substitution for launches with few lines
+// substitution on the FP64 matrix cores
 // ---------------------------------------------------------------------------
-// Lanes 4k..4k+3 of a wave hold the components 0..3 of one line's node
-// vector and the matching rows of W^-1, so the serial chain of a node is a
-// quarter of the arithmetic plus quad exchanges (DPP): on levels with few
-// lines the launch is bound by that chain, not by memory.
-template <int CTRL>
-__device__ __forceinline__ double qdpp(double x) {
+// One launch per colour: a block takes LPB neighbouring lines, builds their
+// residual records in LDS with all its threads, substitutes with 16 lanes per
+// line half, and adds the corrections to u with all its threads again.
+//
+// v_mfma_f64_4x4x4_4b multiplies four 4x4 pairs at once, with lanes
+//     A[i][k] at i + 4 b + 16 k,  B[k][j] at j + 4 b + 16 k,
+//     D[i][j] at j + 4 b + 16 i          (b = 0..3: the pair),
+// so a product's D is the next product's B without any exchange.  The pairs
+// are the two halves (b / 2) of two lines (b % 2): a wave runs both chains of
+// its two lines with one instruction stream, since the bottom half is the top
+// half mirrored (the sign of v changes, nothing else).  Column j % 2 of B and
+// D holds the real (0) and imaginary (1) parts of a node vector (columns 2
+// and 3 repeat 0 and 1), a complex product M y is
+//     Re M [y.re, y.im] + Im M [-y.im, y.re]
+// -- two matrix instructions and one exchange of neighbouring lanes -- and A
+// holds the node's 4x4 matrices, symmetric, one complex entry per lane.
+// A node of the forward pass is y = g - B z, z = W^-1 y (three matrix
+// instructions, the chain), one of the back pass x = z - W^-1 B x' (three) and
+// the along-line edge q + v.(x' - x) / d (one, off the chain).
+//
+// Why: four lanes per line half on the vector units took 120 (forward) and
+// 160 (back) instructions and about 0.45 us a node, two substituting waves per
+// CU; a step here takes 35 and 44 instructions around a chain of about 150 cycles
+// (62 ns).  Blocks of eight lines keep their records in 80 KiB of LDS at 128
+// nodes (in FP64; FP32-storage cycles round sigma, rho and z to FP32), so two blocks and eight
+// substituting waves share a CU.  Launches with few lines are bound by the
+// chain of N / 2 nodes, large ones by the two reads of the factor records and
+// the stencil traffic (128 nodes: about 5 TB/s).  Per launch of a colour, four
+// lanes per half and cyclic reduction for single lines -> here: 128 nodes,
+// FP64, one right-hand side 137 -> 107 us along y and z, 145 -> 83 along x;
+// FP32, three 245 -> 225 and 280 -> 196; 96 nodes, FP32, eight 370 -> 248 and
+// 330 -> 218; 64 nodes, FP64, one 37 -> 24; 16 nodes 12.5 -> 9.5; one line of 96
+// nodes, eight right-hand sides 26 -> 16.
+constexpr int M_LDS = 160 * 1024;          // LDS of a CU
+// LDS of a line: 2 T - 1 node vectors (4 complex) and 2 T edges (1 complex)
+__host__ __device__ __forceinline__ int line_m_bytes(int n) { return 160 * HalfOrder(n).T - 64; }
+static int line_m_lpb(int n) { return 8 * line_m_bytes(n) <= M_LDS ? 8 : 2; }
+static bool line_m_fits(int n) { return 2 * line_m_bytes(n) <= M_LDS; }
+
+// (re, im) -> (-im, re) across the columns of a node vector; sg flips the
+// sign of the even columns
+__device__ __forceinline__ double mswap(double x, unsigned sg) {
   const long long b = __double_as_longlong(x);
-  const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xF, 0xF, true);
-  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xF, 0xF, true);
+  const int lo = __builtin_amdgcn_mov_dpp((int)b, 0xB1, 0xF, 0xF, true);          // quad_perm [1,0,3,2]
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), 0xB1, 0xF, 0xF, true);
+  return __longlong_as_double(((long long)(int)((unsigned)hi ^ sg) << 32) | (unsigned int)lo);
+}
+// the other half's value (pairs b and b ^ 2: eight lanes on in the row of 16)
+__device__ __forceinline__ double mpeer(double x) {
+  const long long b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_mov_dpp((int)b, 0x128, 0xF, 0xF, true);         // row_ror:8
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), 0x128, 0xF, 0xF, true);
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
-// sum over the quad (every lane gets the same value)
-__device__ __forceinline__ cxd qsum(cxd a) {
-  a += cxd(qdpp<0xB1>(a.re), qdpp<0xB1>(a.im));   // quad_perm [1,0,3,2]
-  a += cxd(qdpp<0x4E>(a.re), qdpp<0x4E>(a.im));   // quad_perm [2,3,0,1]
-  return a;
+__device__ __forceinline__ double mma(double a, double b, double c) {
+  return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
 }
-// component J of the quad's vector
-template <int J>
-__device__ __forceinline__ cxd qget(cxd a) {
-  return cxd(qdpp<J * 0x55>(a.re), qdpp<J * 0x55>(a.im));
-}
-// row q of W^-1 (w) times the quad's vector y
-__device__ __forceinline__ cxd qsymv(const cxd (&w)[4], cxd y) {
-  const cxd y0 = qget<0>(y), y1 = qget<1>(y), y2 = qget<2>(y), y3 = qget<3>(y);
-  cxd acc(0, 0);
-  acc += w[0] * y0;
-  acc += w[1] * y1;
-  acc += w[2] * y2;
-  acc += w[3] * y3;
-  return acc;
-}
-
-// one node of one lane's records: row q of W^-1, 1/d, component q of the line
-// record (sigma or z) and rho
-template <typename RS>
-struct QNode {
-  double2 w[4];
-  double2 rd;
-  typename cvec<RS>::type s, rho;
-  typename cvec<RS>::type pad;
-};
-
-template <typename RS>
-__device__ __forceinline__ void qload_f(QNode<RS>& n, const Ch<double>* __restrict__ fnode, long stride, const int (&wch)[4]) {
-#pragma unroll
-  for (int j = 0; j < 4; j++) n.w[j] = *reinterpret_cast<const double2*>(&fnode[wch[j] * stride]);
-  n.rd = *reinterpret_cast<const double2*>(&fnode[10 * stride]);
-}
-
-// fused launches with lines of NT nodes keep the block's line records in LDS
-// when they take at most EMMI_QUAD_LDS_KB KiB (build-time tunable)
-#ifndef EMMI_QUAD_LDS_KB
-#define EMMI_QUAD_LDS_KB 80
-#endif
-// Block shape of the fused quad-lane launches (lines per block, threads;
-// build-time tunables).  The FP32 128-node instance holds 314 registers per
-// lane (one wave per SIMD) and, with 16 lines, 80 KiB of records plus the
-// 2 KiB meeting exchange in LDS: one 256-thread block per CU, whose two
-// further waves only help with the right-hand sides.  15 lines in
-// 128-thread blocks (75 + 2 KiB) let two blocks and four substituting waves
-// share a CU, and measured slower at 128^3 (three right-hand sides:
-// 257 -> 305 us per y/z launch; one: 78 -> 128 us): the right-hand sides,
-// built by two waves instead of four, cost more than the second block gains.
-// Single-wave blocks of 8 lines from line length EMMI_LINE_WAVE_MIN_NT on
-// (off by default) fit four to eight to a CU, but the one wave builds all
-// its records and runs both halves' loops under divergent masks: measured at
-// 128^3 they won on a few shapes (FP64 128-node lines, one right-hand side:
-// 143 -> 125 us; FP32 64-node x lines, three: 77 -> 70 us) and lost on most
-// (FP32 128-node y/z lines, three: 257 -> 357 us; FP32 64-node lines, one:
-// 36 -> 62 us).
-#ifndef EMMI_LINE_WAVE_MIN_NT
-#define EMMI_LINE_WAVE_MIN_NT 1000000
-#endif
-#ifndef EMMI_LINE_LPB_F32_128
-#define EMMI_LINE_LPB_F32_128 16
-#endif
-#ifndef EMMI_LINE_BT_F32_128
-#define EMMI_LINE_BT_F32_128 EMMI_LINE_FUSE_THREADS_LONG
-#endif
+// a value of the line records, rounded to the cycle's precision
 template <typename T>
-__host__ __device__ constexpr int quad_lpb(int nt) {
-  return nt >= EMMI_LINE_WAVE_MIN_NT ? 8 : (sizeof(T) == 4 && nt == 128 ? EMMI_LINE_LPB_F32_128 : 16);
+__device__ __forceinline__ double rec_val(double x) {
+  return (double)(ScrRec<T>)x;
 }
-template <typename T>
-__host__ __device__ constexpr int quad_bt(int nt) {
-  return nt >= EMMI_LINE_WAVE_MIN_NT                 ? 64
-         : sizeof(T) == 4 && nt == 128               ? EMMI_LINE_BT_F32_128
-         : nt >= 64                                  ? EMMI_LINE_FUSE_THREADS_LONG
-                                                     : EMMI_LINE_FUSE_THREADS;
-}
+// ends a node of the unrolled passes, and before that sets its reload of the
+// ring apart: left to itself the scheduler gathers the off-chain products of a
+// whole group at its start, and waits there for every load of the ring, or
+// issues a reload before the last use of its slot, into registers of its own
+// that are copied back (and waited for) at the end of the group
+__device__ __forceinline__ void node_end() { __builtin_amdgcn_sched_barrier(0); }
 
-// nodes per thread whose right-hand sides a fused launch builds together
-#ifndef EMMI_LINE_RHS_UNROLL
-#define EMMI_LINE_RHS_UNROLL 4
-#endif
-// 1: a fused launch of lines of 64 nodes or more builds its right-hand sides
-// by marching along the lines (line_rhs_march; shorter lines leave runs of a
-// node or two, with nothing to carry); 0: node by node.  Lines along x keep
-// the node-by-node loop: there a wave's lanes take runs 8 nodes apart in 16
-// rows, twice the cache lines per load of four neighbouring nodes (and in
-// FP64 the record stores scatter alike).  Measured at 128^3 per launch of a
-// colour with one right-hand side: along y and z the march takes 143 -> 137
-// and 145 -> 139 us (FP64, 128 nodes), along x 156 -> 296 us (FP64) and 100
-// -> 107 us (FP32).
-#ifndef EMMI_LINE_RHS_MARCH
-#define EMMI_LINE_RHS_MARCH 1
-#endif
-// nodes per thread of the separate right-hand-side launch that marches
-#ifndef EMMI_LINE_RHS_RUN
-#define EMMI_LINE_RHS_RUN 8
-#endif
-// fused launches along x build their node-by-node records with a wave on
-// this many neighbouring nodes of each of 64 / EMMI_LINE_RHS_XGROUP lines
-// (0: 4 nodes of 16 lines, as along y and z)
-#ifndef EMMI_LINE_RHS_XGROUP
-#define EMMI_LINE_RHS_XGROUP 16
-#endif
-template <typename T, int A>
-__host__ __device__ constexpr bool rhs_march(int nt) {
-  return EMMI_LINE_RHS_MARCH != 0 && nt >= 64 && A != 0;
-}
-
-template <typename T>
-__host__ __device__ constexpr bool quad_lds_records(int nt, int lpb = 16) {
-  return nt > 0 && lpb * nt * SREC * (int)sizeof(ScrRec<T>) <= EMMI_QUAD_LDS_KB * 1024;
-}
-
-// NT > 0: every job of the launch has lines of NT nodes; up to 64 nodes the
-// passes are unrolled completely (longer lines keep the loop: the code would
-// not fit the instruction cache).  The rolled loop's guard-free groups keep
-// the ring in place (see k_line_solve); the unrolled passes also drop the
-// loop overhead of these short chains.
-//
-// With RHS the block first computes the records of its own LPB lines (the
-// work of k_line_rhs, for launches too small to pay for a launch of their
-// own) with all its BT threads, and then substitutes.  BT >= 128: a wave per
-// line half side (top halves of the block's LPB <= 16 lines in wave 0,
-// bottom halves in wave 1; four lanes per line half, lanes beyond 4 LPB
-// idle), further waves only help with the right-hand sides, the halves meet
-// through LDS.  BT = 64 (LPB <= 8): one wave holds both halves (lanes 0-31
-// the top halves, 32-63 the bottom ones, each side under its own exec
-// mask) and the halves meet through a cross-lane shuffle.
-template <typename T, int A, int D, bool RHS, int BT, int NT, int LPB = 16>
-__global__ void __launch_bounds__(BT) k_line_solve_q(LinePack<T> P) {
-  constexpr bool ONEW = BT == 64;   // both sides in one wave
-  static_assert(ONEW ? LPB <= 8 : (LPB <= 16 && BT >= 128), "lines per block");
-  using E = typename cvec<T>::type;
-  using RS = ScrRec<T>;
-  using PS = typename cvec<RS>::type;
-  constexpr int FC = fchunks<double>(), SC = schunks<RS>(), VS = Ch<RS>::V;
-  __shared__ double xch[ONEW ? 1 : 2][2][ONEW ? 1 : 64];
+// D = line_ring(N): nodes of factor records in flight per half
+template <typename T, int A, int LPB, int D>
+__global__ void __launch_bounds__(32 * LPB, 2) k_line_solve_m(LinePack<T> P) {
+  constexpr int BT = 32 * LPB, FC = fchunks<double>(), SC = schunks<double>();
+  extern __shared__ double2 mlds[];
   const LineJob<T>& J = P.job[blockIdx.y];
   const Level<T>& L = J.L;
-  const int N = NT > 0 ? NT : L.n[A];
-  constexpr int UNR = NT > 0 && NT <= 64 ? 64 : 1;   // the passes' unroll count
-  if (N < 2) return;   // uniform over the block: no interior node
-  const int M = N - 1, m = N / 2;
-  // LR: the block's line records live in LDS (lrec[node][line][value]) and
-  // never go to memory, which takes a store and a dependent load off each end
-  // of the substitution
-  constexpr bool LR = RHS && quad_lds_records<T>(NT, LPB);
-  __shared__ RS lrec[LR ? LPB * NT * SREC : 1];
-  if (RHS) {
-    const long nl = (long)J.nlo * J.nhi;
-    if constexpr (rhs_march<T, A>(NT)) {
-      // each line's nodes in CH consecutive runs, a run per thread, lines
-      // fastest (a wave's loads cover LPB neighbouring lines), each run
-      // marching along its line
+  const int N = L.n[A];
+  const int nl = J.nlo * J.nhi;
+  const int l0 = (int)xcd_block(blockIdx.x, gridDim.x) * LPB;
+  if (N < 2 || l0 >= nl) return;   // uniform over the block
+  const HalfOrder O(N);
+  const int m = O.m, T2 = 2 * O.T, TT = O.T;
+  const int nle = min(LPB, nl - l0);   // lines of this block
+  // edges: rho, then dE, in the order of the records; node vectors: sigma,
+  // then z, then x, in the same order without each half's first (boundary or
+  // padding) record.  Neighbouring threads of the first and last phase walk
+  // along x, so x lines lie one after another and other lines side by side.
+  double2* __restrict__ Q = mlds;
+  double2* __restrict__ X = mlds + T2 * LPB;
+  auto qslot = [&](int t2, int l) { return A == 0 ? l * T2 + t2 : t2 * LPB + l; };
+  auto xslot = [&](int s, int l) { return 4 * (A == 0 ? l * (T2 - 1) + s : s * LPB + l); };
+  // slot of the vector of record r (r = 0 and T have none)
+  auto xrec = [&](int r) { return r - 1 - (r > TT ? 1 : 0); };
+
+  // ---------------- residual records ----------------
+  auto put_rec = [&](int p, int l, const Ch<double>(&c)[SC]) {
+    Q[qslot(O.edge(p), l)] = make_double2(rec_val<T>(c[4].v[0]), rec_val<T>(c[4].v[1]));
+    if (p >= 1) {
+      double2* x = X + xslot(xrec(O.node(p)), l);
+#pragma unroll
+      for (int i = 0; i < 4; i++) x[i] = make_double2(rec_val<T>(c[i].v[0]), rec_val<T>(c[i].v[1]));
+    }
+  };
+  // padding and boundary records
+  if (O.o > 0) {
+    const double2 zz = make_double2(0.0, 0.0);
+    for (int idx = threadIdx.x; idx < LPB * (O.o + 1); idx += BT) {
+      const int l = idx % LPB, t = idx / LPB;
+      if (t < O.o) Q[qslot(t, l)] = zz;
+      if (t < O.ob) Q[qslot(TT + t, l)] = zz;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        if (t >= 1) X[xslot(t - 1, l) + i] = zz;
+        if (t >= 1 && t <= O.ob) X[xslot(TT - 1 + t - 1, l) + i] = zz;
+      }
+    }
+  }
+  // Along y and z, lines of 64 nodes and more are marched by runs of N / 32
+  // nodes (128 nodes, per launch of a colour: 120 -> 107 us FP64 with one
+  // right-hand side, 252 -> 224 FP32 with three); a block with few lines would
+  // leave most of its threads without a run (one line of 96 nodes: 23 us
+  // marched, 16 node by node).
+  bool march = false;
+  if constexpr (A != 0 && D == 8) march = N >= 64 && nle > LPB / 2;
+  if (march) {
+    if constexpr (A != 0 && D == 8) {
+      // runs of consecutive nodes marching along the line, lines fastest
       constexpr int CH = BT / LPB;
-      const int ll = (int)threadIdx.x % LPB, ch = (int)threadIdx.x / LPB;
+      const int l = (int)threadIdx.x % LPB, ch = (int)threadIdx.x / LPB;
       const int run = (N + CH - 1) / CH;
       const int p0 = ch * run, p1 = min(N, p0 + run);
-      const int ln = blockIdx.x * LPB + ll;
-      int b2, c2;
-      if (ch < CH && p0 < p1 && line_of<T, A>(J, ln, b2, c2)) {
-        line_rhs_march<T, A>(J, b2, c2, p0, p1, [&](int p, const Ch<RS>(&c)[SC]) {
-          if constexpr (LR) {
-#pragma unroll
-            for (int v = 0; v < SREC; v++) lrec[(p * LPB + ll) * SREC + v] = (RS)val(c, v);
-          } else {
-            store_rhs_rec<T>(J, ln, p, nl, c);
-          }
-        });
+      if (l < nle && p0 < p1) {
+        int pb, pc;
+        line_of<T, A>(J, l0 + l, pb, pc);
+        line_rhs_march<T, A, double>(J, pb, pc, p0, p1, [&](int p, const Ch<double>(&c)[SC]) { put_rec(p, l, c); });
       }
-    } else {
-      // unrolled: several nodes' stencil loads in flight per thread (the
-      // substitution sets the kernel's register count, this loop fits in it)
-#pragma unroll EMMI_LINE_RHS_UNROLL
-      for (int idx = threadIdx.x; idx < LPB * N; idx += blockDim.x) {
-        // along x (lines in separate rows) a wave takes XN neighbouring
-        // nodes of 64 / XN lines instead of 4 nodes of 16 lines
-        constexpr int XN = EMMI_LINE_RHS_XGROUP;
-        constexpr bool XG = A == 0 && NT > 0 && XN > 0 && NT % XN == 0;
-        const int ll = XG ? (idx / XN) % LPB : idx % LPB;
-        const int p = XG ? idx / (XN * LPB) * XN + idx % XN : idx / LPB;
-        const int ln = blockIdx.x * LPB + ll;
-        int b2, c2;
-        if (line_of<T, A>(J, ln, b2, c2)) {
-          if constexpr (LR) {
-            Ch<RS> c[SC] = {};
-            node_rhs_rec<T, A>(J, b2, c2, p, c);
+    }
+  } else {
+    const int nn = nle * N;
+    for (int idx = threadIdx.x; idx < nn; idx += BT) {
+      const int l = A == 0 ? idx / N : idx % nle, p = A == 0 ? idx % N : idx / nle;
+      int pb, pc;
+      line_of<T, A>(J, l0 + l, pb, pc);
+      Ch<double> c[SC] = {};
+      node_rhs_rec<T, A>(J, pb, pc, p, c);
+      put_rec(p, l, c);
+    }
+  }
+  __syncthreads();
+
+  // ---------------- substitution ----------------
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  if (2 * wave < nle) {   // uniform over the wave
+    const int lane = threadIdx.x & 63;
+    const int row = lane >> 4, j = lane & 3, b = (lane >> 2) & 3, side = b >> 1;
+    // a wave without a second line runs its first line twice
+    const int l = min(2 * wave + (b & 1), nle - 1);
+    int pb, pc;
+    line_of<T, A>(J, l0 + l, pb, pc);
+    const LineGeo<T, A> G(L, pb, pc);
+    auto vk = [&](int k) { const double h = k < 2 ? G.Hc : G.Hb; return (k & 1) ? -h : h; };
+    const double vr = vk(row);                  // also entry (j, row) of an A operand whose rows are all v
+    const double vs = side ? -vr : vr;          // v of this half, component `row`
+    const double ncl = row == 0 ? G.Wb0 * G.Hc : row == 1 ? G.Wb1 * G.Hc : row == 2 ? G.Wc0 * G.Hb : G.Wc1 * G.Hb;   // -l W_a
+    const int jr = j & 1;
+    const unsigned sg = jr ? 0u : 0x80000000u;  // sign of the swapped operand's even columns
+    // factor records of the wave's lines from a uniform base, node d of the
+    // current group at a constant offset
+    const int rbytes = FC * 16;
+    const char* fb = reinterpret_cast<const char*>(J.fac) + (long)(l0 + 2 * wave) * O.records() * rbytes;
+    const unsigned fo = (unsigned)(((l - 2 * wave) * O.records() + side * TT) * rbytes);
+    const unsigned fw = fo + 16 * symidx(j, row), fr = fo + 160;
+    // 1/W of the inner edge: t - o on top, N + ob - 1 - t below (clamped: the
+    // padding's value meets z = 0)
+    const double* __restrict__ iwa = L.IW[A];
+    const int e0 = side ? N + O.ob - 1 : -O.o, de = side ? -1 : 1;
+    double2 rw[D], rr[D];
+    double ri[D];
+    auto load = [&](int d, const char* base, int t) {   // base: record t - d
+      rw[d] = *reinterpret_cast<const double2*>(base + d * rbytes + fw);
+      rr[d] = *reinterpret_cast<const double2*>(base + d * rbytes + fr);
+      ri[d] = iwa[min((unsigned)(e0 + de * t), (unsigned)(N - 1))];
+    };
+    // LDS: vector component and edge of node t of the half
+    constexpr int XS = A == 0 ? 8 : 8 * LPB, QS = A == 0 ? 2 : 2 * LPB;
+    double* xq = reinterpret_cast<double*>(X + xslot(side * (TT - 1), l)) - XS + 2 * row + jr;
+    double* qa = reinterpret_cast<double*>(Q + qslot(side * TT, l)) + jr;
+    const int qx = 1 - 2 * jr;   // from the component jr to the other one
+    auto neg = [&](double x) { return __longlong_as_double(__double_as_longlong(x) ^ ((unsigned long long)sg << 32)); };
+    // q = rho / d of an edge, component jr
+    auto qval = [&](double ra, double rb, double2 rd) { return fma(rb, neg(rd.y), ra * rd.x); };
+
 #pragma unroll
-            for (int v = 0; v < SREC; v++) lrec[(p * LPB + ll) * SREC + v] = (RS)val(c, v);
-          } else {
-            node_rhs<T, A>(J, ln, b2, c2, p, nl);
-          }
+    for (int d = 0; d < D; d++) load(d, fb, d);
+    const double2 wm = *reinterpret_cast<const double2*>(fb + (unsigned)(((l - 2 * wave) * O.records() + T2) * rbytes + 16 * symidx(j, row)));
+    // Software pipeline: a node's step runs its chain on operands prepared in
+    // the step before, and prepares the next node's (coupling -B, right-hand
+    // side g) and reads the LDS of the one after.
+    double z = 0.0, q, sig, ra, rb;
+    // a single line (the coarsest level) is solved in FP64 throughout
+    auto zrec = [&](double v) { return nl > 1 ? rec_val<T>(v) : v; };
+    // -B = -diag(l) - (v / d) v^T towards the node before, g of the node.  B all
+    // but cancels on the node's gradient, which W^-1 amplifies in air: v.z is
+    // summed first (one matrix instruction, rows all v) and then scaled, as an
+    // explicit B would round every entry on its own.
+    double nl1, vre, vim, g;
+    auto couple = [&](int d) {
+      nl1 = ncl * ri[d];
+      vre = -vr * rr[d].x;
+      vim = -vr * rr[d].y;
+    };
+    auto bsub = [&](double v, double g0) {   // g0 - B v
+      const double sv = mma(vr, v, 0.0);
+      return fma(vim, mswap(sv, sg), fma(vre, sv, fma(nl1, v, g0)));
+    };
+    auto fnext = [&](int d) {   // operands of the node after d (of group slot d)
+      couple(d);
+      const double q1 = qval(ra, rb, rr[(d + 1) % D]);
+      g = fma(vs, q - q1, sig);
+      q = q1;
+    };
+    auto fread = [&](int d) {   // LDS of node d
+      sig = xq[d * XS];
+      ra = qa[d * QS];
+      rb = qa[d * QS + qx];
+    };
+    auto fstep = [&](int d) {
+      const double y = bsub(z, g);
+      z = mma(rw[d].x, y, 0.0);
+      z = mma(rw[d].y, mswap(y, sg), z);
+      fnext(d);
+      fread(d + 2);
+      xq[d * XS] = zrec(z);
+    };
+    // the first node of a half (boundary or padding) only hands its inner
+    // edge on
+    q = qval(qa[0], qa[qx], rr[0]);
+    fread(1);
+    fnext(0);
+    fread(2);
+    node_end();
+    int t0 = 0;
+    if (TT > D) {
+      load(0, fb + D * rbytes, D);
+      node_end();
+#pragma unroll
+      for (int d = 1; d < D; d++) {
+        fstep(d);
+        node_end();
+        load(d, fb + D * rbytes, D + d);
+        node_end();
+      }
+      for (t0 = D; t0 < TT - D; t0 += D) {
+        xq += D * XS; qa += D * QS; fb += D * rbytes;
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+          fstep(d);
+          node_end();
+          load(d, fb + D * rbytes, t0 + D + d);
+          node_end();
         }
       }
+      // the last group's records stay for the back pass
+      xq += D * XS; qa += D * QS; fb += D * rbytes;
+      fstep(0);
+      node_end();
     }
-    __syncthreads();   // the block's records are complete (workgroup scope)
-  }
-  const int lane = threadIdx.x & 63, side = ONEW ? lane >> 5 : (int)threadIdx.x >> 6;
-  const int q = lane & 3;
-  const int lloc = ONEW ? (lane & 31) >> 2 : lane >> 2;   // the lane's line within the block
-  const int line = blockIdx.x * LPB + lloc;
-  int pb = 0, pc = 0;
-  const bool live = side < 2 && lloc < LPB && line_of<T, A>(J, line, pb, pc);
-  LineGeo<T, A> G;
-  if (live) G.init(L, pb, pc);
-  const long stride = (long)J.nlo * J.nhi;
-  const Ch<double>* __restrict__ fac = reinterpret_cast<const Ch<double>*>(J.fac) + line;
-  Ch<RS>* __restrict__ scr = reinterpret_cast<Ch<RS>*>(J.scr) + line;
-  E* __restrict__ u = J.u;
-  const double* __restrict__ iw = L.IW[A];
-  const long fstep = (long)FC * stride, sstep = (long)SC * stride;
-  // this lane's component: v_q, the coupling coefficient (l_q = cq / W_a), the
-  // chunks of row q of W^-1, and where component q of a line record sits
-  const double vq = q == 0 ? G.Hc : q == 1 ? -G.Hc : q == 2 ? G.Hb : -G.Hb;
-  const double cq = q == 0 ? -G.Wb0 * G.Hc : q == 1 ? -G.Wb1 * G.Hc : q == 2 ? -G.Wc0 * G.Hb : -G.Wc1 * G.Hb;
-  const int wch[4] = {symidx(q, 0), symidx(q, 1), symidx(q, 2), symidx(q, 3)};
-  const long soff = (long)((2 * q) / VS) * stride;
-  const int sel = (2 * q) % VS;
-  const long off_q = q == 0 ? G.ob0 : q == 1 ? G.ob1 : q == 2 ? G.oc0 : G.oc1;
-  // component q of sigma (z once written) and rho of node p of this lane's line
-  auto rec_s = [&](int p) -> PS {
-    if constexpr (LR) return *reinterpret_cast<const PS*>(&lrec[(p * LPB + lloc) * SREC + 2 * q]);
-    else return *reinterpret_cast<const PS*>(reinterpret_cast<const RS*>(scr + p * sstep + soff) + sel);
-  };
-  auto rec_rho = [&](int p) -> PS {
-    if constexpr (LR) return *reinterpret_cast<const PS*>(&lrec[(p * LPB + lloc) * SREC + 8]);
-    else return *reinterpret_cast<const PS*>(reinterpret_cast<const RS*>(scr + p * sstep + (8 / VS) * stride) + 8 % VS);
-  };
-  auto put_z = [&](int p, PS z) {
-    if constexpr (LR) *reinterpret_cast<PS*>(&lrec[(p * LPB + lloc) * SREC + 2 * q]) = z;
-    else *reinterpret_cast<PS*>(reinterpret_cast<RS*>(scr + p * sstep + soff) + sel) = z;
-  };
-  auto qnode = [&](QNode<RS>& n, int p) {
-    qload_f(n, fac + p * fstep, stride, wch);
-    n.s = rec_s(p);
-    n.rho = rec_rho(p);
-  };
+#pragma unroll
+    for (int d = 1; d < D; d++) {
+      fstep(d);
+      node_end();
+    }
 
-  // D nodes ahead are in flight: the load for node p + D goes into the slot
-  // node p - 1 used, so a slot is never copied before it is refilled
-  constexpr int R = D + 1;
-  QNode<RS> ring[R];
-  double riw[R];
-  cxd tm(0, 0);   // component q of this half's coupling term at the meeting node
-  auto cw = [](const QNode<RS>& n, cxd (&w)[4]) {
-#pragma unroll
-    for (int j = 0; j < 4; j++) w[j] = cxd(n.w[j].x, n.w[j].y);
-  };
-
-  // ---------------- forward elimination ----------------
-  if (live && side == 0) {
-    const int last = m - 1;
-#pragma unroll
-    for (int d = 0; d < D; d++) {
-      const int pn = max(min(1 + d, last), 1);
-      qnode(ring[d], pn);
-      riw[d] = iw[pn - 1];
-    }
-    const cxd rd0(fac[10 * stride].v[0], fac[10 * stride].v[1]);
-    const PS r0 = rec_rho(0);
-    cxd rd_prev = rd0;
-    cxd q_prev = cxd((double)r0.x, (double)r0.y) * rd0;
-    cxd z(0, 0);
-    auto step = [&](const int p, const int d) {
-      const QNode<RS>& nd = ring[d];
-      const double iWe = (double)riw[d];
-      {
-        const int pn = min(p + D, last), dn = (d + D) % R;
-        qnode(ring[dn], pn);
-        riw[dn] = iw[pn - 1];
-      }
-      cxd w[4];
-      cw(nd, w);
-      const cxd rd(nd.rd.x, nd.rd.y);
-      const cxd qp = cxd((double)nd.rho.x, (double)nd.rho.y) * rd;
-      cxd g = cxd((double)nd.s.x, (double)nd.s.y) + (q_prev - qp) * vq;
-      if (p >= 2) {
-        const cxd vz = qsum(z * vq);
-        g -= z * (cq * iWe) + (vz * rd_prev) * vq;
-      }
-      z = qsymv(w, g);
-      PS zs;
-      zs.x = (RS)z.re;
-      zs.y = (RS)z.im;
-      put_z(p, zs);
-      rd_prev = rd;
-      q_prev = qp;
-    };
-    // whole groups of R nodes without a guard per node (guards inside the
-    // group make the register allocator copy the ring), then the rest
-    int p0 = 1;
-#pragma unroll UNR
-    for (; p0 + (R - 1) <= last; p0 += R) {
-#pragma unroll
-      for (int d = 0; d < R; d++) step(p0 + d, d);
-    }
-#pragma unroll
-    for (int d = 0; d < R - 1; d++)
-      if (p0 + d <= last) step(p0 + d, d);
-    if (m >= 2) {
-      const cxd vz = qsum(z * vq);
-      tm = z * (cq * (double)iw[m - 1]) + (vz * rd_prev) * vq;   // B_m z_{m-1}
-    }
-  } else if (live) {
-    const int last = m + 1;
-    // 1/d and rho of the node above each ring entry, kept as loaded: a
-    // conversion at load time would wait for the load
-    Ch<double> rdn[R];
-    PS qn[R];
-#pragma unroll
-    for (int d = 0; d < D; d++) {
-      const int pn = min(max(M - d, last), M);
-      qnode(ring[d], pn);
-      riw[d] = iw[pn];
-      rdn[d] = fac[(pn - 1) * fstep + 10 * stride];
-      qn[d] = rec_rho(pn - 1);
-    }
-    cxd zn(0, 0), rd_last(0, 0);
-    auto step = [&](const int p, const int d) {
-      const QNode<RS>& nd = ring[d];
-      const double iWe = (double)riw[d];
-      const cxd rdm(rdn[d].v[0], rdn[d].v[1]), rhom((double)qn[d].x, (double)qn[d].y);
-      {
-        const int pn = max(p - D, last), dn = (d + D) % R;
-        qnode(ring[dn], pn);
-        riw[dn] = iw[pn];
-        rdn[dn] = fac[(pn - 1) * fstep + 10 * stride];
-        qn[dn] = rec_rho(pn - 1);
-      }
-      cxd w[4];
-      cw(nd, w);
-      const cxd rd(nd.rd.x, nd.rd.y);
-      const cxd qp = cxd((double)nd.rho.x, (double)nd.rho.y) * rd;
-      const cxd qm = rhom * rdm;
-      cxd g = cxd((double)nd.s.x, (double)nd.s.y) + (qm - qp) * vq;
-      if (p <= M - 1) {
-        const cxd vz = qsum(zn * vq);
-        g -= zn * (cq * iWe) + (vz * rd) * vq;
-      }
-      zn = qsymv(w, g);
-      PS zs;
-      zs.x = (RS)zn.re;
-      zs.y = (RS)zn.im;
-      put_z(p, zs);
-      rd_last = rdm;
-    };
-    // whole groups of R nodes without a guard per node (guards inside the
-    // group make the register allocator copy the ring), then the rest
-    int p0 = M;
-#pragma unroll UNR
-    for (; p0 - (R - 1) >= last; p0 -= R) {
-#pragma unroll
-      for (int d = 0; d < R; d++) step(p0 - d, d);
-    }
-#pragma unroll
-    for (int d = 0; d < R - 1; d++)
-      if (p0 - d >= last) step(p0 - d, d);
-    if (m + 1 <= M) {
-      const cxd vz = qsum(zn * vq);
-      tm = zn * (cq * (double)iw[m]) + (vz * rd_last) * vq;   // B_{m+1} z_{m+1}
-    }
-  }
-
-  // ---------------- meeting node ----------------
-  cxd tpeer(0, 0);   // one wave: the other side's coupling term, same line and component
-  if constexpr (!ONEW) {
-    if (side < 2) {
-      xch[side][0][lane] = tm.re;
-      xch[side][1][lane] = tm.im;
-    }
-    __syncthreads();
-  } else {
-    tpeer = cxd(__shfl_xor(tm.re, 32), __shfl_xor(tm.im, 32));
-  }
-  if (!live) return;
-  cxd xm, qmid, rdmid;
-  {
-    QNode<RS> nd;
-    qnode(nd, m);
-    const Ch<double> c = fac[(m - 1) * fstep + 10 * stride];
-    const PS r = rec_rho(m - 1);
-    cxd w[4];
-    cw(nd, w);
-    rdmid = cxd(nd.rd.x, nd.rd.y);
-    qmid = cxd((double)nd.rho.x, (double)nd.rho.y) * rdmid;
-    const cxd rdm(c.v[0], c.v[1]);
-    const cxd dq = cxd((double)r.x, (double)r.y) * rdm - qmid;
-    cxd ttop, tbot;
-    if constexpr (!ONEW) {
-      ttop = cxd(xch[0][0][lane], xch[0][1][lane]);
-      tbot = cxd(xch[1][0][lane], xch[1][1][lane]);
-    } else {
-      ttop = side == 0 ? tm : tpeer;
-      tbot = side == 0 ? tpeer : tm;
-    }
-    const cxd g = ((cxd((double)nd.s.x, (double)nd.s.y) + dq * vq) - ttop) - tbot;
-    xm = qsymv(w, g);
-  }
-
-  // ---------------- back substitution ----------------
-  E ru[R], ra[R];
-  if (side == 0) {
+    // meeting node: x_m = S_m^-1 (g_m - B_m z_{m-1} - B_{m+1} z_{m+1})
+    double x;
     {
-      const long o = off_q + (long)m * G.sa;
-      st<T>(u, o, ld<T>(u, o) + xm);
+      const double ql = qval(qa[(D - 1) * QS], qa[(D - 1) * QS + qx], rr[D - 1]);
+      double* xm = reinterpret_cast<double*>(X + xslot(T2 - 2, l)) + 2 * row + jr;
+      double y = bsub(z, vs * ql);
+      y = *xm + (y + mpeer(y));
+      x = mma(wm.x, y, 0.0);
+      x = mma(wm.y, mswap(y, sg), x);
+      *xm = x;
     }
-    const int last = m - 1;
-#pragma unroll
-    for (int d = 0; d < D; d++) {
-      const int pn = max(last - d, 1);
-      qnode(ring[d], pn);
-      riw[d] = iw[pn];
-      ru[d] = u[off_q + (long)pn * G.sa];
-      ra[d] = u[G.oa + (long)pn * G.sa];
-    }
-    cxd an = xm;   // component q of x_{p+1}
-    auto step = [&](const int p, const int d) {
-      const QNode<RS>& nd = ring[d];
-      const double iWe = (double)riw[d];
-      const E cu = ru[d], ca = ra[d];
-      {
-        const int pn = max(p - D, 1), dn = (d + D) % R;
-        qnode(ring[dn], pn);
-        riw[dn] = iw[pn];
-        ru[dn] = u[off_q + (long)pn * G.sa];
-        ra[dn] = u[G.oa + (long)pn * G.sa];
-      }
-      cxd w[4];
-      cw(nd, w);
-      const cxd rd(nd.rd.x, nd.rd.y);
-      const cxd qp = cxd((double)nd.rho.x, (double)nd.rho.y) * rd;
-      const cxd va = qsum(an * vq);
-      const cxd t = an * (cq * iWe) + (va * rd) * vq;
-      const cxd ap = cxd((double)nd.s.x, (double)nd.s.y) - qsymv(w, t);
-      const cxd dv = qsum((an - ap) * vq);
-      const long o = (long)p * G.sa;
-      if (q == 0) st<T>(u, G.oa + o, cxd((double)ca.x, (double)ca.y) + (qp + dv * rd));
-      st<T>(u, off_q + o, cxd((double)cu.x, (double)cu.y) + ap);
-      an = ap;
+    sig = zrec(z);
+    // the along-line edge of a node follows one step later, off the chain
+    double dx = 0.0, ere = 0.0, eim = 0.0, eq = 0.0;
+    auto edge = [&](double* to) {   // q + v.dx / d
+      const double sv = mma(vs, dx, 0.0);
+      *to = fma(eim, mswap(sv, sg), fma(ere, sv, eq));
     };
-    // whole groups of R nodes without a guard per node (guards inside the
-    // group make the register allocator copy the ring), then the rest
-    int p0 = last;
-#pragma unroll UNR
-    for (; p0 - (R - 1) >= 1; p0 -= R) {
-#pragma unroll
-      for (int d = 0; d < R; d++) step(p0 - d, d);
-    }
-#pragma unroll
-    for (int d = 0; d < R - 1; d++)
-      if (p0 - d >= 1) step(p0 - d, d);
-    // along-line edge 0, between the boundary node and node 1
-    const cxd rd0(fac[10 * stride].v[0], fac[10 * stride].v[1]);
-    const PS r0 = rec_rho(0);
-    const cxd q0 = cxd((double)r0.x, (double)r0.y) * rd0;
-    const cxd dv = qsum(an * vq);
-    if (q == 0) st<T>(u, G.oa, ld<T>(u, G.oa) + (q0 + dv * rd0));
-  } else {
-    const int last = m + 1;
-#pragma unroll
-    for (int d = 0; d < D; d++) {
-      const int pn = min(last + d, M);
-      qnode(ring[d], pn);
-      riw[d] = iw[pn - 1];
-      ru[d] = u[off_q + (long)pn * G.sa];
-      ra[d] = u[G.oa + (long)(pn - 1) * G.sa];
-    }
-    cxd xp = xm;   // component q of x_{p-1}
-    cxd rdm = rdmid, qm = qmid;
-    auto step = [&](const int p, const int d) {
-      const QNode<RS>& nd = ring[d];
-      const double iWe = (double)riw[d];
-      const E cu = ru[d], ca = ra[d];
-      {
-        const int pn = min(p + D, M), dn = (d + D) % R;
-        qnode(ring[dn], pn);
-        riw[dn] = iw[pn - 1];
-        ru[dn] = u[off_q + (long)pn * G.sa];
-        ra[dn] = u[G.oa + (long)(pn - 1) * G.sa];
-      }
-      cxd w[4];
-      cw(nd, w);
-      const cxd rd(nd.rd.x, nd.rd.y);
-      const cxd qp = cxd((double)nd.rho.x, (double)nd.rho.y) * rd;
-      const cxd vx = qsum(xp * vq);
-      const cxd t = xp * (cq * iWe) + (vx * rdm) * vq;
-      const cxd ap = cxd((double)nd.s.x, (double)nd.s.y) - qsymv(w, t);
-      const cxd dv = qsum((ap - xp) * vq);
-      const long o = (long)p * G.sa;
-      if (q == 0) st<T>(u, G.oa + o - G.sa, cxd((double)ca.x, (double)ca.y) + (qm + dv * rdm));
-      st<T>(u, off_q + o, cxd((double)cu.x, (double)cu.y) + ap);
-      xp = ap;
-      rdm = rd;
-      qm = qp;
+    auto bedge = [&](int d) {   // operands of that edge
+      ere = rr[d].x;
+      eim = rr[d].y;
+      eq = qval(ra, rb, rr[d]);
     };
-    // whole groups of R nodes without a guard per node (guards inside the
-    // group make the register allocator copy the ring), then the rest
-    int p0 = last;
-#pragma unroll UNR
-    for (; p0 + (R - 1) <= M; p0 += R) {
+    auto bread = [&](int d) {   // rho of node d's inner edge
+      ra = qa[d * QS];
+      rb = qa[d * QS + qx];
+    };
+    // to: where the pending edge goes
+    auto bstep = [&](int d, double* to) {
+      const double y = bsub(x, 0.0);
+      double xp = mma(rw[d].x, y, sig);
+      xp = mma(rw[d].y, mswap(y, sg), xp);
+      sig = xq[(d - 1) * XS];
+      edge(to);
+      bedge(d);
+      bread(d - 1);
+      couple((d + D - 1) % D);
+      dx = x - xp;
+      xq[d * XS] = xp;
+      x = xp;
+    };
+    couple(D - 1);
+    bread(D - 1);
+    // no edge is pending at first: that write lands on the edge whose rho has
+    // just been read and which the next step writes
+    double* qe = qa + (D - 1) * QS;
+    for (; t0 > 0; t0 -= D) {
 #pragma unroll
-      for (int d = 0; d < R; d++) step(p0 + d, d);
+      for (int d = D - 1; d >= 0; d--) {
+        bstep(d, d == D - 1 ? qe : qa + (d + 1) * QS);
+        node_end();
+        // a slot is reloaded one step after its node: that node's edge is
+        // still pending until then
+        if (d == D - 1) load(0, fb, t0);
+        else load(d + 1, fb - D * rbytes, t0 - D + d + 1);
+        node_end();
+      }
+      qe = qa;
+      xq -= D * XS; qa -= D * QS; fb -= D * rbytes;
     }
 #pragma unroll
-    for (int d = 0; d < R - 1; d++)
-      if (p0 + d <= M) step(p0 + d, d);
-    // along-line edge M = N-1, between node M and the boundary node
-    const cxd dv = qsum((cxd(0, 0) - xp) * vq);
-    const long o = G.oa + (long)M * G.sa;
-    if (q == 0) st<T>(u, o, ld<T>(u, o) + (qm + dv * rdm));
+    for (int d = D - 1; d >= 1; d--) {
+      bstep(d, d == D - 1 ? qe : qa + (d + 1) * QS);
+      node_end();
+      if (d == D - 1) load(0, fb, 0);
+      node_end();
+    }
+    edge(qa + QS);
+    // the first node's correction is zero: its inner edge alone
+    bedge(0);
+    dx = x;
+    edge(qa);
+  }
+  __syncthreads();
+
+  // ---------------- u += corrections ----------------
+  {
+    typename cvec<T>::type* __restrict__ u = J.u;
+    const int nn = nle * N;
+    for (int idx = threadIdx.x; idx < nn; idx += BT) {
+      const int l = A == 0 ? idx / N : idx % nle, p = A == 0 ? idx % N : idx / nle;
+      int pb, pc;
+      line_of<T, A>(J, l0 + l, pb, pc);
+      constexpr int B = (A + 1) % 3, C = (A + 2) % 3;
+      const long o = (long)pb * L.es[B] + (long)pc * L.es[C] + (long)p * L.es[A];
+      const double2 e = Q[qslot(O.edge(p), l)];
+      st<T>(u, A * L.nc + o, ld<T>(u, A * L.nc + o) + cxd(e.x, e.y));
+      if (p >= 1) {
+        const double2* x = X + xslot(xrec(O.node(p)), l);
+        const long offs[4] = {B * L.nc + o - L.es[B], B * L.nc + o, C * L.nc + o - L.es[C], C * L.nc + o};
+        cxd v[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = ld<T>(u, offs[i]);
+#pragma unroll
+        for (int i = 0; i < 4; i++) st<T>(u, offs[i], v[i] + cxd(x[i].x, x[i].y));
+      }
+    }
   }
 }
 
@@ -2044,10 +1630,7 @@ static size_t chunks_of(int values, size_t esize) {
 size_t line_factor_bytes(const int* n, int a, int colour, size_t esize) {
   int nlo, nhi;
   line_colour_counts(n, a, colour, &nlo, &nhi);
-  const size_t twisted = (size_t)nlo * nhi * (size_t)n[a] * chunks_of(FREC, esize) * 16;
-  if ((long)nlo * nhi == 1 && n[a] >= 2 && n[a] <= PCR_MAX_NODES)
-    return std::max(twisted, (size_t)pcr_entries(n[a]) * sizeof(cxd));
-  return twisted;
+  return (size_t)nlo * nhi * (size_t)HalfOrder(n[a]).records() * chunks_of(FREC, esize) * 16;
 }
 
 size_t line_scratch_bytes(const int* n, int a, int colour, size_t esize) {
@@ -2071,18 +1654,49 @@ static void launch_timed(K kernel, dim3 g, dim3 b, hipStream_t s, int cls, Bytes
   else hipLaunchKernelGGL(kernel, g, b, 0, s, args...);
 }
 
-template <typename T, int NT>
-static void launch_quad_fused(const LinePack<T>& P, int axis, int maxl, hipStream_t s, Bytes by) {
-  // the 128-node lines keep their loop (not unrolled): a deeper ring pays
-  // there in FP32 cycles (in FP64 it spills)
-  constexpr int QD = NT == 128 && sizeof(T) == 4 ? 5 : EMMI_LINE_QUAD_RING;
-  // block shape: see quad_lpb / quad_bt
-  constexpr int LPB = quad_lpb<T>(NT);
-  constexpr int FT = quad_bt<T>(NT);
-  const dim3 g((unsigned)((maxl + LPB - 1) / LPB), P.njobs), b(FT);
-  if (axis == 0) launch_timed(k_line_solve_q<T, 0, QD, true, FT, NT, LPB>, g, b, s, timing::LINE, by, P);
-  else if (axis == 1) launch_timed(k_line_solve_q<T, 1, QD, true, FT, NT, LPB>, g, b, s, timing::LINE, by, P);
-  else launch_timed(k_line_solve_q<T, 2, QD, true, FT, NT, LPB>, g, b, s, timing::LINE, by, P);
+// the same with dynamic LDS (more than the default 64 KiB is enabled once per
+// kernel and device)
+template <typename K, typename... Args>
+static void launch_lds(K kernel, dim3 g, dim3 b, size_t lds, hipStream_t s, int cls, Bytes bytes, Args... args) {
+  if (lds > 64 * 1024) {
+    static std::mutex mu;
+    static std::set<std::pair<const void*, int>> done;
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    std::lock_guard<std::mutex> lk(mu);
+    const void* fn = reinterpret_cast<const void*>(kernel);
+    if (done.insert({fn, dev}).second)
+      (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, M_LDS);
+  }
+  hipEvent_t e0, e1;
+  timing::kernel_events(cls, bytes.comp, &e0, &e1, bytes.layout);
+  if (e0) hipExtLaunchKernelGGL(kernel, g, b, lds, s, e0, e1, 0, args...);
+  else hipLaunchKernelGGL(kernel, g, b, lds, s, args...);
+}
+
+// the matrix-core substitution: lines per block by what the LDS holds, the
+// ring by the length of a half
+template <typename T, int A>
+static void launch_line_m_axis(const LinePack<T>& P, int maxl, int maxna, hipStream_t s, Bytes by) {
+  const int lpb = line_m_lpb(maxna), D = line_ring(maxna);
+  const dim3 g((unsigned)((maxl + lpb - 1) / lpb), P.njobs), b(32 * lpb);
+  const size_t lds = (size_t)lpb * line_m_bytes(maxna);
+  auto go = [&](auto kernel) { launch_lds(kernel, g, b, lds, s, timing::LINE, by, P); };
+  if (lpb == 2) {
+    if (D == 8) go(k_line_solve_m<T, A, 2, 8>);
+    else if (D == 4) go(k_line_solve_m<T, A, 2, 4>);
+    else go(k_line_solve_m<T, A, 2, 2>);
+  } else {
+    if (D == 8) go(k_line_solve_m<T, A, 8, 8>);
+    else if (D == 4) go(k_line_solve_m<T, A, 8, 4>);
+    else go(k_line_solve_m<T, A, 8, 2>);
+  }
+}
+template <typename T>
+static void launch_line_m(const LinePack<T>& P, int axis, int maxl, int maxna, hipStream_t s, Bytes by) {
+  if (axis == 0) launch_line_m_axis<T, 0>(P, maxl, maxna, s, by);
+  else if (axis == 1) launch_line_m_axis<T, 1>(P, maxl, maxna, s, by);
+  else launch_line_m_axis<T, 2>(P, maxl, maxna, s, by);
 }
 
 template <typename T>
@@ -2111,22 +1725,6 @@ static void launch_pack(const LinePack<T>& P, int axis, bool factor, hipStream_t
   if (maxl == 0 || P.njobs == 0) return;
   int maxna = 0;
   for (int j = 0; j < P.njobs; j++) maxna = std::max(maxna, P.job[j].L.n[axis]);
-  if (maxl == 1 && maxna <= PCR_MAX_NODES) {
-    const dim3 g(1, P.njobs);
-    if (factor) {
-      timing::Scope ts(timing::OTHER, s, 0);
-      if (axis == 0) hipLaunchKernelGGL((k_line_pcr_factor<T, 0>), g, dim3(PCR_MAX_NODES), 0, s, P);
-      else if (axis == 1) hipLaunchKernelGGL((k_line_pcr_factor<T, 1>), g, dim3(PCR_MAX_NODES), 0, s, P);
-      else hipLaunchKernelGGL((k_line_pcr_factor<T, 2>), g, dim3(PCR_MAX_NODES), 0, s, P);
-      return;
-    }
-    const Bytes by{comp, rhs_bytes + solve_bytes};
-    const dim3 b(4 * PCR_MAX_NODES);
-    if (axis == 0) launch_timed(k_line_pcr_solve<T, 0>, g, b, s, timing::LINE, by, P);
-    else if (axis == 1) launch_timed(k_line_pcr_solve<T, 1>, g, b, s, timing::LINE, by, P);
-    else launch_timed(k_line_pcr_solve<T, 2>, g, b, s, timing::LINE, by, P);
-    return;
-  }
   if (factor) {
     const dim3 g((maxl + 63) / 64, P.njobs), b(64);
     timing::Scope ts(timing::OTHER, s, 0);
@@ -2135,33 +1733,23 @@ static void launch_pack(const LinePack<T>& P, int axis, bool factor, hipStream_t
     else hipLaunchKernelGGL((k_line_factor<T, 2>), g, b, 0, s, P);
     return;
   }
-  // along x the quad-lane kernel's updates of u are scattered rows (see
-  // k_line_solve_x_apply): the finest FP32 x sweeps of several right-hand
-  // sides keep the one-lane kernel (3 slots at 128^3: 1% faster), a single
-  // right-hand side takes the quad-lane one (430 against 567 us per sweep)
+  // the matrix-core substitution takes every line that fits its LDS records;
+  // longer ones (and forced launches) take the one-lane kernel
   if (choice == LINE_RULE && g_line_kernel == 0) choice = tuned_choice(line_shape(P, axis));
-  if (choice == LINE_RULE && g_line_kernel == 3) choice = LINE_QUAD_FUSED;
-  if (choice == LINE_RULE && g_line_kernel == 4) choice = LINE_QUAD_SEPARATE;
-  bool quad, fuse;
-  if (choice == LINE_ONE_LANE || choice == LINE_QUAD_FUSED || choice == LINE_QUAD_SEPARATE) {
-    quad = choice != LINE_ONE_LANE;
-    fuse = choice == LINE_QUAD_FUSED;
-  } else {
-    quad = g_line_kernel == 2 || (g_line_kernel == 0 && maxl <= quad_max_lines<T>() &&
-                                  (axis != 0 || maxl <= 2048 || sizeof(T) == 8 || P.njobs == 1));
-    fuse = quad && maxl <= fuse_max_lines<T>();
+  const bool one_lane = choice == LINE_ONE_LANE || (choice == LINE_RULE && g_line_kernel == 1);
+  if (!one_lane && line_m_fits(maxna)) {
+    launch_line_m<T>(P, axis, maxl, maxna, s, Bytes{comp, rhs_bytes + solve_bytes - 2.0 * rec_bytes});
+    return;
   }
-  if (fuse) {
-    // the substitution kernel computes its own right-hand sides
-  } else if (axis == 0) {
+  if (axis == 0) {
     int maxn = 0;
     for (int j = 0; j < P.njobs; j++) maxn = std::max(maxn, P.job[j].L.n[0]);
     const int nlb = (maxl + XT - 1) / XT, npb = (maxn + XT - 1) / XT;
     const dim3 g((unsigned)(nlb * npb), P.njobs), b(XT * XT);
     launch_timed(k_line_rhs_x<T>, g, b, s, timing::LINE_RHS, Bytes{0.0, rhs_bytes}, P, nlb);
-  } else if (EMMI_LINE_RHS_MARCH != 0 && maxna >= 64) {
-    // lines of 64 nodes and more march (as the fused launches do)
-    const int run = EMMI_LINE_RHS_RUN;
+  } else if (maxna >= 64) {
+    // lines of 64 nodes and more march
+    constexpr int run = 8;
     const long nth = (long)maxl * ((maxna + run - 1) / run);
     const dim3 g((unsigned)((nth + 255) / 256), P.njobs), b(256);
     if (axis == 1) launch_timed(k_line_rhs_run<T, 1>, g, b, s, timing::LINE_RHS, Bytes{0.0, rhs_bytes}, P, run);
@@ -2171,35 +1759,7 @@ static void launch_pack(const LinePack<T>& P, int axis, bool factor, hipStream_t
     if (axis == 1) launch_timed(k_line_rhs<T, 1>, g, b, s, timing::LINE_RHS, Bytes{0.0, rhs_bytes}, P);
     else launch_timed(k_line_rhs<T, 2>, g, b, s, timing::LINE_RHS, Bytes{0.0, rhs_bytes}, P);
   }
-  if (quad) {
-    // few lines: four lanes per line half shorten the serial chain
-    constexpr int QD = EMMI_LINE_QUAD_RING;
-    const dim3 g((maxl + 15) / 16, P.njobs);
-    if (fuse) {
-      // a common line length with an instance of its own, else the generic one
-      int nt = P.job[0].L.n[axis];
-      for (int j = 1; j < P.njobs; j++)
-        if (P.job[j].L.n[axis] != nt) nt = 0;
-      if (nt != 4 && nt != 8 && nt != 16 && nt != 32 && nt != 64 && nt != 128) nt = 0;
-      // records kept in LDS are neither written to nor read from memory
-      const Bytes by{comp, rhs_bytes + solve_bytes - (quad_lds_records<T>(nt, quad_lpb<T>(nt)) ? 2.0 * rec_bytes : 0.0)};
-      switch (nt) {
-        case 4: launch_quad_fused<T, 4>(P, axis, maxl, s, by); break;
-        case 8: launch_quad_fused<T, 8>(P, axis, maxl, s, by); break;
-        case 16: launch_quad_fused<T, 16>(P, axis, maxl, s, by); break;
-        case 32: launch_quad_fused<T, 32>(P, axis, maxl, s, by); break;
-        case 64: launch_quad_fused<T, 64>(P, axis, maxl, s, by); break;
-        case 128: launch_quad_fused<T, 128>(P, axis, maxl, s, by); break;
-        default: launch_quad_fused<T, 0>(P, axis, maxl, s, by); break;
-      }
-    } else {
-      const dim3 b(128);
-      const Bytes by{comp, solve_bytes};
-      if (axis == 0) launch_timed(k_line_solve_q<T, 0, QD, false, 128, 0>, g, b, s, timing::LINE, by, P);
-      else if (axis == 1) launch_timed(k_line_solve_q<T, 1, QD, false, 128, 0>, g, b, s, timing::LINE, by, P);
-      else launch_timed(k_line_solve_q<T, 2, QD, false, 128, 0>, g, b, s, timing::LINE, by, P);
-    }
-  } else {
+  {
     const dim3 g((maxl + 63) / 64, P.njobs), b(128);
     if (axis == 0) {
       // the substitution's algorithmic bytes include the update of u, which
@@ -2223,12 +1783,6 @@ template <typename T>
 void launch_line_solve_as(const LinePack<T>& P, int axis, int choice, hipStream_t s) {
   launch_pack<T>(P, axis, false, s, choice);
 }
-template <typename T>
-bool line_pcr_shape(const LinePack<T>& P, int axis) {
-  const LineShape k = line_shape(P, axis);
-  return k.nl == 1 && k.n <= PCR_MAX_NODES;
-}
-
 template void launch_line_factor<double>(const LinePack<double>&, int, hipStream_t);
 template void launch_line_factor<float>(const LinePack<float>&, int, hipStream_t);
 template void launch_line_solve<double>(const LinePack<double>&, int, hipStream_t);
@@ -2237,7 +1791,5 @@ template void launch_line_solve_as<double>(const LinePack<double>&, int, int, hi
 template void launch_line_solve_as<float>(const LinePack<float>&, int, int, hipStream_t);
 template LineShape line_shape<double>(const LinePack<double>&, int);
 template LineShape line_shape<float>(const LinePack<float>&, int);
-template bool line_pcr_shape<double>(const LinePack<double>&, int);
-template bool line_pcr_shape<float>(const LinePack<float>&, int);
 
 }  // namespace emmi

@@ -159,8 +159,7 @@ class Solver {
   // Autotuning of the line sweeps: for every launch shape a solve of all
   // slots issues (levels, axes, colours, packs of up to LINE_PACK_MAX
   // slots) and that the process-wide table does not hold yet, times each
-  // substitution choice (one-lane, quad-lane fused, quad-lane with separate
-  // right-hand sides) reps times on the slots' own level vectors and records
+  // substitution choice (matrix cores, one lane) reps times on the slots' own level vectors and records
   // the fastest.  The vectors' contents are overwritten (the next solve sets
   // them again); captured cycle graphs are dropped.  Returns the number of
   // shapes tuned.

@@ -526,7 +526,6 @@ int Solver::autotune_t(int reps) {
               J.scr = (typename LineScr<T>::type*)S.lscr;
               line_job_colour(J, axis, colour);
             }
-            if (line_pcr_shape<T>(P, axis)) continue;
             const LineShape key = line_shape<T>(P, axis);
             if (key.nl < 1 || has_line_choice(key)) continue;
             double best = 0;

@@ -381,7 +381,7 @@ def timing_enable(on=True):
     lib().emmi_timing_enable(1 if on else 0)
 
 
-LINE_CHOICES = ["one_lane", "quad_fused", "quad_separate"]
+LINE_CHOICES = ["one_lane", "matrix"]
 
 
 def line_tuning():
