@@ -124,80 +124,154 @@ __global__ void __launch_bounds__(256) k_conv_fwd(const bf16* __restrict__ x, in
     }
 }
 
-// dw partials: block = 4 waves, one (tap, 16-channel input tile, 16-channel
-// output tile) per block, the voxels of slab blockIdx.y in tiles of 128.
-// A tile of dy (16 output channels) and of x at the tap's offset (16 input
-// channels, zero outside the grid) is loaded with 16-byte loads (a thread: 8
-// channels of one voxel) and stored channel-major in LDS, so that a lane's
-// 8 consecutive voxels of one channel -- its share of an MFMA operand -- are
-// one aligned 16-byte LDS read.  Rows are padded to 136 values so the 16
-// channel rows start in different banks.  The next tile's loads are in
-// flight while the current one is multiplied.  Wave w takes voxels
-// [32 w, 32 w + 32) of each tile.
-constexpr int DW_TV = 128, DW_ROW = DW_TV + 8;
-__global__ void __launch_bounds__(256) k_conv_dw(const bf16* __restrict__ x, const bf16* __restrict__ dy, int Z, int Y,
-                                                 int X, int Cin, int Cout, int zslab, float* __restrict__ part) {
-  __shared__ __align__(16) bf16 As[16 * DW_ROW];
-  __shared__ __align__(16) bf16 Bs[16 * DW_ROW];
-  __shared__ float red[4][64][4];
+// dw partials: a block takes the three taps of one (dz, dy) for up to NCI
+// 16-channel input tiles and one 16-channel output tile, over the voxels of
+// slab blockIdx.y; its waves take chunks of 32 voxels in turn, each in LDS of
+// its own and without barriers.  A chunk's dy (32 voxels) and x (the same
+// voxels displaced by dz and dy, and one more at either end) are loaded with
+// contiguous 16-byte loads, stored voxel by voxel, and read back transposed
+// (ds_read_b64_tr_b16), so that a lane holds 8 voxels of one channel, its
+// share of an MFMA operand: the three taps read the same x tile at row offsets
+// -1, 0 and 1.  Voxels whose tap falls outside the grid are masked in the
+// operand (a chunk inside a row skips that).  The next chunk's loads are in
+// flight while the current one is multiplied.
+//
+// What bounds it: with one tap and one input tile per block, every tile was
+// stored element by element (16 two-byte LDS stores a voxel) for one matrix
+// instruction per wave between two barriers; here five loads and five LDS
+// stores serve nine.  48 -> 16 channels at 96^3: 48 -> 16 channels at 96^3: 560 -> 203 us (180 TFLOP/s).
+constexpr int DW_WAVES = 16, DW_CHUNK = 32;
+
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+// transposed read of rows r0 .. r0 + 31 of a [voxel][16] tile: lane l receives
+// channel l % 16 of voxels 4 (l / 16) + j and 16 + 4 (l / 16) + j (j < 4), an
+// order of K that both operands share
+__device__ __forceinline__ bf16x8 read_tr(const bf16* tile, int r0, int lane) {
+  typedef __attribute__((address_space(3))) s16x4 lds4;
+  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4*)(tile + 16 * r0 + 4 * lane));
+  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4*)(tile + 16 * (r0 + 16) + 4 * lane));
+  return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+template <int NCI>
+__global__ void __launch_bounds__(64 * DW_WAVES) k_conv_dw(const bf16* __restrict__ x, const bf16* __restrict__ dy,
+                                                           int Z, int Y, int X, int Cin, int Cout, int zslab,
+                                                           float* __restrict__ part) {
+  constexpr int XR = DW_CHUNK + 2;             // voxels of an x tile
+  constexpr int WT = (DW_CHUNK + NCI * XR) * 16;   // values of a wave's tiles
+  constexpr int RED = DW_WAVES * NCI * 256;    // floats of one tap's sums
+  __shared__ __align__(16) char smem[DW_WAVES * WT * 2 > RED * 4 ? DW_WAVES * WT * 2 : RED * 4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int nci = Cin / 16, nco = Cout / 16;
+  const int nci = Cin / 16, nco = Cout / 16, ng = (nci + NCI - 1) / NCI;
   const int t = blockIdx.x;
-  const int tap = t / (nci * nco);
-  const int ci0 = ((t / nco) % nci) * 16, co0 = (t % nco) * 16;
-  const int dz = tap / 9 - 1, dyy = (tap / 3) % 3 - 1, dx = tap % 3 - 1;
+  const int zy = t / (ng * nco);   // 3 (dz + 1) + dy + 1
+  const int c0 = ((t / nco) % ng) * NCI, co0 = (t % nco) * 16;
+  const int nt = min(NCI, nci - c0);   // input tiles of this block
+  const int dz = zy / 3 - 1, dyy = zy % 3 - 1;
   const int z0 = blockIdx.y * zslab, z1 = min(Z, z0 + zslab);
   // voxels of a slab fit 32-bit indices (the launcher checks the volume)
-  const int nv = (z1 - z0) * Y * X;
-  const int base = z0 * Y * X;   // flat index of the slab's first voxel
-  // staging role: voxel vi of the tile, channels 8 h .. 8 h + 7
-  const int vi = threadIdx.x >> 1, h = threadIdx.x & 1;
-  auto load = [&](int v0, uint4& ra, uint4& rb) {
-    ra = make_uint4(0, 0, 0, 0);
-    rb = make_uint4(0, 0, 0, 0);
-    const int v = v0 + vi;
-    if (v < nv) {
-      const int g = base + v;
-      ra = *reinterpret_cast<const uint4*>(dy + (long)g * Cout + co0 + 8 * h);
-      const int xx = g % X, q = g / X, yy = q % Y, zz = q / Y;
-      const int sz = zz + dz, sy = yy + dyy, sx = xx + dx;
-      if (sz >= 0 && sz < Z && sy >= 0 && sy < Y && sx >= 0 && sx < X)
-        rb = *reinterpret_cast<const uint4*>(x + ((long)(sz * Y + sy) * X + sx) * Cin + ci0 + 8 * h);
-    }
-  };
-  auto put = [&](const uint4& ra, const uint4& rb) {
-    const bf16* pa = reinterpret_cast<const bf16*>(&ra);
-    const bf16* pb = reinterpret_cast<const bf16*>(&rb);
+  const unsigned nv = (unsigned)(z1 - z0) * Y * X;
+  const long base = (long)z0 * Y * X, vol = (long)Z * Y * X, shift = (long)(dz * Y + dyy) * X;
+  bf16* A = reinterpret_cast<bf16*>(smem) + wave * WT;
+  bf16* B = A + DW_CHUNK * 16;
+  // coordinates of this lane's voxel of the chunk (lane % 32); a wave's next
+  // chunk is DW_WAVES chunks on
+  constexpr unsigned STEP = DW_WAVES * DW_CHUNK;
+  unsigned v0 = wave * DW_CHUNK;   // the chunk's first voxel within the slab
+  const unsigned vl = v0 + (lane & 31), uX = X, uY = Y;
+  int xx = (int)(vl % uX), yy = (int)(vl / uX % uY), zz = z0 + (int)(vl / uX / uY);
+  const int sx = (int)(STEP % uX), sy = (int)(STEP / uX % uY), sz = (int)(STEP / uX / uY);
+  // loads: dy, voxel lane / 2; x, 16-byte piece i 64 + lane of the tile's
+  // 34 voxels x 2 nt pieces
+  constexpr int NX = (XR * 2 * NCI + 63) / 64;
+  uint4 ra, rx[NX];
+  unsigned m[3];   // voxels whose tap dx - 1 lies in the grid
+  const int np = 2 * nt;
+  int gx[NX], lx[NX], vx[NX];   // offset from the voxel before the chunk, place in the tiles, voxel
 #pragma unroll
-    for (int c = 0; c < 8; c++) {
-      As[(8 * h + c) * DW_ROW + vi] = pa[c];
-      Bs[(8 * h + c) * DW_ROW + vi] = pb[c];
-    }
-  };
-  const int col = lane & 15, kq = (lane >> 4) * 8;
-  f32x4 acc = {0, 0, 0, 0};
-  uint4 ra, rb;
-  load(0, ra, rb);
-  for (int v0 = 0; v0 < nv; v0 += DW_TV) {
-    __syncthreads();   // the previous tile's operands are read
-    put(ra, rb);
-    __syncthreads();
-    if (v0 + DW_TV < nv) load(v0 + DW_TV, ra, rb);
-    // A = dy^T (rows co, cols voxels), B = x_tap (rows voxels, cols ci)
-    const int o = col * DW_ROW + 32 * wave + kq;
-    const bf16x8 a = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&As[o]));
-    const bf16x8 b = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&Bs[o]));
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
+  for (int i = 0; i < NX; i++) {
+    const int c = 64 * i + lane, piece = c % np;
+    vx[i] = c / np;
+    gx[i] = vx[i] * Cin + 16 * c0 + 8 * piece;
+    lx[i] = (piece >> 1) * (XR * 16) + vx[i] * 16 + 8 * (piece & 1);
+    if (vx[i] >= XR) vx[i] = 1 << 20;
   }
+  auto load = [&]() {
+    const bool in = v0 + (lane & 31) < nv;
+    const int pz = zz + dz, py = yy + dyy;
+    const bool ok = in && pz >= 0 && pz < Z && py >= 0 && py < Y;
+    m[0] = (unsigned)__ballot(ok && xx > 0);
+    m[1] = (unsigned)__ballot(ok);
+    m[2] = (unsigned)__ballot(ok && xx < X - 1);
+    const unsigned va = v0 + (lane >> 1);
+    ra = va < nv ? *reinterpret_cast<const uint4*>(dy + (base + va) * Cout + co0 + 8 * (lane & 1)) : make_uint4(0, 0, 0, 0);
+    // voxels of the x tile inside the tensor (the rest is masked anyway)
+    const long f0 = base + shift - 1 + (long)__builtin_amdgcn_readfirstlane((int)v0);
+    const int vlo = (int)max(0L, min(-f0, 1L << 20)), vhi = (int)max(0L, min((long)XR, vol - f0));
+    const bf16* xp = x + f0 * Cin;
 #pragma unroll
-  for (int i = 0; i < 4; i++) red[wave][lane][i] = acc[i];
-  __syncthreads();
-  if (wave == 0) {
+    for (int i = 0; i < NX; i++)
+      rx[i] = vx[i] >= vlo && vx[i] < vhi ? *reinterpret_cast<const uint4*>(xp + gx[i]) : make_uint4(0, 0, 0, 0);
+    v0 += STEP;
+    xx += sx; yy += sy; zz += sz;
+    if (xx >= X) { xx -= X; yy++; }
+    if (yy >= Y) { yy -= Y; zz++; }
+  };
+  f32x4 acc[3][NCI];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const float s = red[0][lane][i] + red[1][lane][i] + red[2][lane][i] + red[3][lane][i];
-      const int co = co0 + 4 * (lane >> 4) + i, ci = ci0 + col;
-      part[((long)blockIdx.y * Cout + co) * (27L * Cin) + (long)tap * Cin + ci] = s;
+  for (int k = 0; k < 3; k++)
+#pragma unroll
+    for (int n = 0; n < NCI; n++) acc[k][n] = f32x4{0, 0, 0, 0};
+  if (v0 < nv) load();
+  for (unsigned c = wave * DW_CHUNK; c < nv; c += STEP) {
+    reinterpret_cast<uint4*>(A)[lane] = ra;
+#pragma unroll
+    for (int i = 0; i < NX; i++)
+      if (vx[i] < XR) *reinterpret_cast<uint4*>(B + lx[i]) = rx[i];
+    const unsigned mk[3] = {m[0], m[1], m[2]};
+    if (c + STEP < nv) load();
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    // A = dy^T (rows co, cols voxels), B = x at the tap (rows voxels, cols ci)
+    const bf16x8 a = read_tr(A, 0, lane);
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      if (mk[k] == 0) continue;   // uniform over the wave
+      // 0xffff for the halves of the operand's voxels inside the grid
+      uint4 keep = make_uint4(~0u, ~0u, ~0u, ~0u);
+      if (mk[k] != ~0u) {
+        const unsigned lo = mk[k] >> (4 * (lane >> 4)), hi = lo >> 16;
+        auto two = [](unsigned bits) { return ((bits & 1) ? 0xffffu : 0u) | ((bits & 2) ? 0xffff0000u : 0u); };
+        keep = make_uint4(two(lo), two(lo >> 2), two(hi), two(hi >> 2));
+      }
+#pragma unroll
+      for (int n = 0; n < NCI; n++) {
+        if (n >= nt) continue;   // uniform
+        uint4 o = __builtin_bit_cast(uint4, read_tr(B + n * XR * 16, k, lane));
+        if (mk[k] != ~0u) { o.x &= keep.x; o.y &= keep.y; o.z &= keep.z; o.w &= keep.w; }
+        acc[k][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf16x8, o), acc[k][n], 0, 0, 0);
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+  // the waves' sums in a fixed order, one tap at a time in the tiles' memory
+  float* red = reinterpret_cast<float*>(smem);
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < NCI; n++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) red[((wave * NCI + n) * 64 + lane) * 4 + i] = acc[k][n][i];
+    __syncthreads();
+    for (int e = threadIdx.x; e < nt * 256; e += 64 * DW_WAVES) {
+      const int n = e / 256, ln = (e % 256) / 4, i = e % 4;
+      float sum = 0.f;
+#pragma unroll
+      for (int w = 0; w < DW_WAVES; w++) sum += red[((w * NCI + n) * 64 + ln) * 4 + i];
+      const int co = co0 + 4 * (ln >> 4) + i, ci = 16 * (c0 + n) + (ln & 15);
+      part[((long)blockIdx.y * Cout + co) * (27L * Cin) + (long)(3 * zy + k) * Cin + ci] = sum;
     }
   }
 }
@@ -616,12 +690,19 @@ int emmi_x0_conv_dw(const void* x, const void* dy, int Z, int Y, int X, int Cin,
   if (Cin % 16 || Cout % 16 || Cout > 256 || zslab < 1 || Z < 1 || Y < 1 || X < 1) return -1;
   if ((long)Z * Y * X >= (1L << 31)) return -1;   // the kernel indexes voxels in 32 bits
   const int nslab = (Z + zslab - 1) / zslab;
-  const dim3 g(27 * (Cin / 16) * (Cout / 16), nslab), b(256);
+  // input tiles per block: up to three
+  const int nci = Cin / 16, NCI = nci == 4 ? 2 : std::min(nci, 3);
+  const dim3 g(9 * ((nci + NCI - 1) / NCI) * (Cout / 16), nslab), b(64 * DW_WAVES);
   hipEvent_t e0, e1;
   emmi::timing::kernel_events(emmi::timing::CONV_DW, 54.0 * Cin * Cout * (double)Z * Y * X, &e0, &e1);
-  if (e0) hipExtLaunchKernelGGL(k_conv_dw, g, b, 0, S(stream), e0, e1, 0, (const bf16*)x, (const bf16*)dy, Z, Y, X, Cin,
-                                Cout, zslab, part);
-  else hipLaunchKernelGGL(k_conv_dw, g, b, 0, S(stream), (const bf16*)x, (const bf16*)dy, Z, Y, X, Cin, Cout, zslab, part);
+  auto go = [&](auto kernel) {
+    if (e0) hipExtLaunchKernelGGL(kernel, g, b, 0, S(stream), e0, e1, 0, (const bf16*)x, (const bf16*)dy, Z, Y, X, Cin,
+                                  Cout, zslab, part);
+    else hipLaunchKernelGGL(kernel, g, b, 0, S(stream), (const bf16*)x, (const bf16*)dy, Z, Y, X, Cin, Cout, zslab, part);
+  };
+  if (NCI == 1) go(k_conv_dw<1>);
+  else if (NCI == 2) go(k_conv_dw<2>);
+  else go(k_conv_dw<3>);
   const long n = 27L * Cin * Cout;
   hipLaunchKernelGGL(k_reduce_slabs, dim3(blocks(n, 256)), dim3(256), 0, S(stream), part, nslab, n, dw);
   if (db) {
