@@ -46,6 +46,53 @@ __device__ __forceinline__ bf16x8 zero8() { return __builtin_bit_cast(bf16x8, ma
 
 enum Epilogue { EPI_LEAKY = 0, EPI_LINEAR = 1, EPI_DACT = 2, EPI_LINEAR_BF16 = 3 };
 
+// a wave's 16 MT voxels from x0 of row (z, y): with the weights as the first
+// operand a lane holds voxel x0 + 16 m + l % 16, channels 16 n + 4 (l / 16) + i,
+// so that it stores four channels at once and the wave's stores are contiguous
+template <int MT, int NT>
+__device__ __forceinline__ void conv_epilogue(const f32x4 (&acc)[MT][NT], int x0, int y, int z, int Y, int X,
+                                              const float* __restrict__ bias, int epi, float slope,
+                                              const bf16* __restrict__ act, bf16* __restrict__ out_bf,
+                                              float* __restrict__ out_f, int Cout_store) {
+  constexpr int Cout = 16 * NT;
+  const int lane = threadIdx.x & 63, c4 = 4 * (lane >> 4);
+  auto pack = [](const f32x4& r) {
+    return make_uint2((unsigned)f2bf(r[0]) | ((unsigned)f2bf(r[1]) << 16), (unsigned)f2bf(r[2]) | ((unsigned)f2bf(r[3]) << 16));
+  };
+#pragma unroll
+  for (int m = 0; m < MT; m++) {
+    const int xx = x0 + 16 * m + (lane & 15);
+    if (xx >= X) continue;
+    const long v = ((long)z * Y + y) * X + xx;
+#pragma unroll
+    for (int n = 0; n < NT; n++) {
+      f32x4 r = acc[m][n];
+      const int co = 16 * n + c4;
+      if (epi == EPI_LEAKY || (epi == EPI_LINEAR && bias)) {
+        const float4 bb = *reinterpret_cast<const float4*>(bias + co);
+        r[0] += bb.x; r[1] += bb.y; r[2] += bb.z; r[3] += bb.w;
+      }
+      if (epi == EPI_LEAKY) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) r[i] = r[i] > 0.f ? r[i] : slope * r[i];
+      } else if (epi == EPI_DACT) {
+        // gradient through the activation of the tensor this one feeds
+        const uint2 av = *reinterpret_cast<const uint2*>(act + v * Cout + co);
+        const bf16 a4[4] = {(bf16)av.x, (bf16)(av.x >> 16), (bf16)av.y, (bf16)(av.y >> 16)};
+#pragma unroll
+        for (int i = 0; i < 4; i++) r[i] = bf2f(a4[i]) > 0.f ? r[i] : slope * r[i];
+      }
+      if (epi == EPI_LINEAR) {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          if (co + i < Cout_store) out_f[v * Cout_store + co + i] = r[i];
+      } else {
+        *reinterpret_cast<uint2*>(out_bf + v * Cout + co) = pack(r);
+      }
+    }
+  }
+}
+
 // One wave: 16*MT consecutive voxels along x of row (z, y) and all 16*NT
 // output channels.  Block: 4 waves on rows y0..y0+3.
 template <int MT, int NT>
@@ -66,62 +113,175 @@ __global__ void __launch_bounds__(256) k_conv_fwd(const bf16* __restrict__ x, in
     for (int n = 0; n < NT; n++) acc[m][n] = f32x4{0, 0, 0, 0};
   const int K27 = 27 * Cin;
   const int row = lane & 15, kq = (lane >> 4) * 8;
-  for (int k0 = 0; k0 < Kpad; k0 += 32) {
+  // the next G steps' operands are in flight while a step is multiplied
+  constexpr int G = MT + NT <= 4 ? 6 : MT + NT <= 6 ? 4 : 3;
+  bf16x8 a[G][MT], b[G][NT];
+  auto fetch = [&](int q, int k0) {
+    if (k0 >= Kpad) return;   // uniform
     const int k = k0 + kq;
-    bf16x8 a[MT];
-    if (k < K27) {
-      const int tap = k / Cin, ci = k - tap * Cin;
-      const int dz = tap / 9 - 1, dy = (tap / 3) % 3 - 1, dx = tap % 3 - 1;
-      const int zz = z + dz, yy = y + dy;
-      const bool zy_ok = zz >= 0 && zz < Z && yy >= 0 && yy < Y;
+    const int tap = k / Cin, ci = k - tap * Cin;
+    const int dz = tap / 9 - 1, dy = (tap / 3) % 3 - 1, dx = tap % 3 - 1;
+    const int zz = z + dz, yy = y + dy;
+    const bool zy_ok = k < K27 && zz >= 0 && zz < Z && yy >= 0 && yy < Y;
 #pragma unroll
-      for (int m = 0; m < MT; m++) {
-        const int xx = x0 + 16 * m + row + dx;
-        if (zy_ok && xx >= 0 && xx < X)
-          a[m] = load8(x + (((long)zz * Y + yy) * X + xx) * Cin + ci);
-        else
-          a[m] = zero8();
-      }
-    } else {
-#pragma unroll
-      for (int m = 0; m < MT; m++) a[m] = zero8();
+    for (int m = 0; m < MT; m++) {
+      const int xx = x0 + 16 * m + row + dx;
+      if (zy_ok && xx >= 0 && xx < X)
+        a[q][m] = load8(x + (((long)zz * Y + yy) * X + xx) * Cin + ci);
+      else
+        a[q][m] = zero8();
     }
 #pragma unroll
-    for (int n = 0; n < NT; n++) {
-      const bf16x8 b = load8(w + (long)(16 * n + row) * Kpad + k);
+    for (int n = 0; n < NT; n++) b[q][n] = load8(w + (long)(16 * n + row) * Kpad + k);
+  };
 #pragma unroll
-      for (int m = 0; m < MT; m++) acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], b, acc[m][n], 0, 0, 0);
+  for (int q = 0; q < G; q++) fetch(q, 32 * q);
+  for (int k0 = 0; k0 < Kpad; k0 += 32 * G) {
+#pragma unroll
+    for (int q = 0; q < G; q++) {
+      if (k0 + 32 * q < Kpad) {   // uniform
+#pragma unroll
+        for (int n = 0; n < NT; n++)
+#pragma unroll
+          for (int m = 0; m < MT; m++) acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[q][n], a[q][m], acc[m][n], 0, 0, 0);
+      }
+      fetch(q, k0 + 32 * (G + q));
     }
   }
-  // epilogue: lane holds voxels x0+16m+4(l/16)+i, channel 16n+(l%16)
-  const int Cout = 16 * NT;
+  conv_epilogue<MT, NT>(acc, x0, y, z, Y, X, bias, epi, slope, act, out_bf, out_f, Cout_store);
+}
+
+// The same sums from LDS: a block takes a tile of 32 x TY voxels, a wave per
+// row of 32, and marches along z with three planes of the input (the tile and
+// a voxel around it, zero outside the grid) in LDS, so every input voxel is
+// loaded (TY + 2) 34 / (32 TY) times instead of 27, and with contiguous loads.
+// The plane after next is loaded while a plane is computed.  Voxels stand
+// 2 Cin + 16 bytes apart, so that the 16 voxels of an operand start in
+// different banks.  A table holds, for each phase of the ring and each group of
+// 8 k, the place of its tap and channels relative to the output voxel.  The
+// instructions and their order are those of k_conv_fwd: the results are equal
+// bit for bit.
+//
+// What bounds it: k_conv_fwd gathered every operand from 16 rows in L1 or L2
+// (one 16-byte load a lane for each NT matrix instructions); here an operand is
+// one LDS read.  At 96^3: 48 -> 16 channels 222 -> 118 us, 16 -> 48
+// 183 -> 97 us (310 to 380 TFLOP/s); the weights come from LDS where they fit
+// beside the planes -- read from memory, 16 rows apart, they were the bound
+// (170 and 241 us).
+template <int NT, int TY, int NP, bool WL>
+__global__ void __launch_bounds__(64 * TY) k_conv_fwd_lds(const bf16* __restrict__ x, int Z, int Y, int X, int Cin,
+                                                          const bf16* __restrict__ w, int Kpad,
+                                                          const float* __restrict__ bias, int epi, float slope,
+                                                          const bf16* __restrict__ act, bf16* __restrict__ out_bf,
+                                                          float* __restrict__ out_f, int Cout_store, int zper) {
+  constexpr int TX = 32, VX = TX + 2, NV = (TY + 2) * VX, BT = 64 * TY, MT = 2, G = WL ? 2 : NT <= 2 ? 8 : NT <= 4 ? 4 : 2;
+  extern __shared__ __align__(16) char smem[];
+  const int vs = 2 * Cin + 16, pb = NV * vs, pc = Cin / 8, np = NV * pc, ng = Kpad / 8;
+  char* planes = smem;                                    // [3][NV][vs]
+  int* tab = reinterpret_cast<int*>(smem + 3 * pb);       // [3][ng]
+  const int ws = 2 * Kpad + 16;                           // bytes of a weight row (rows in different banks)
+  char* wlds = smem + 3 * pb + (3 * ng * 4 + 15) / 16 * 16;   // WL: [16 NT][ws]
+  if constexpr (WL) {
+    for (int i = threadIdx.x; i < 16 * NT * ng; i += BT) {
+      const int co = i / ng, k8 = i - co * ng;
+      *reinterpret_cast<uint4*>(wlds + co * ws + 16 * k8) = *reinterpret_cast<const uint4*>(w + (long)co * Kpad + 8 * k8);
+    }
+  }
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int x0 = blockIdx.x * TX, y0 = blockIdx.y * TY, zs = blockIdx.z * zper, ze = min(Z, zs + zper);
+  for (int i = threadIdx.x; i < 3 * ng; i += BT) {
+    const int ph = i / ng, k = (i - ph * ng) * 8;
+    int off = 0;
+    if (k < 27 * Cin) {
+      const int tap = k / Cin, ci = k - tap * Cin;
+      const int dz = tap / 9, dy = (tap / 3) % 3, dx = tap % 3;
+      off = ((ph + dz) % 3) * pb + (dy * VX + dx) * vs + 2 * ci;
+    }
+    tab[i] = off;   // (padding of K: masked)
+  }
+  // this thread's 16-byte pieces of a plane
+  int go[NP], lo[NP];
 #pragma unroll
-  for (int m = 0; m < MT; m++)
+  for (int i = 0; i < NP; i++) {
+    const int idx = i * BT + (int)threadIdx.x, vox = idx / pc, piece = idx - vox * pc;
+    const int gx = x0 + vox % VX - 1, gy = y0 + vox / VX - 1;
+    lo[i] = idx < np ? vox * vs + 16 * piece : -1;
+    go[i] = idx < np && gx >= 0 && gx < X && gy >= 0 && gy < Y ? (gy * X + gx) * Cin + 8 * piece : -1;
+  }
+  uint4 pre[NP];
+  auto load = [&](int z) {
+    const bool in = z >= 0 && z < Z;   // uniform
+    const bf16* p = x + (long)z * Y * X * Cin;
 #pragma unroll
-    for (int n = 0; n < NT; n++) {
-      const int co = 16 * n + row;
+    for (int i = 0; i < NP; i++)
+      pre[i] = in && go[i] >= 0 ? *reinterpret_cast<const uint4*>(p + go[i]) : make_uint4(0, 0, 0, 0);
+  };
+  auto put = [&](int slot) {
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int xx = x0 + 16 * m + 4 * (lane >> 4) + i;
-        if (xx >= X) continue;
-        const long v = ((long)z * Y + y) * X + xx;
-        float r = acc[m][n][i];
-        if (epi == EPI_LEAKY) {
-          r += bias[co];
-          r = r > 0.f ? r : slope * r;
-          out_bf[v * Cout + co] = f2bf(r);
-        } else if (epi == EPI_LINEAR) {
-          r += bias ? bias[co] : 0.f;
-          if (co < Cout_store) out_f[v * Cout_store + co] = r;
-        } else if (epi == EPI_LINEAR_BF16) {
-          out_bf[v * Cout + co] = f2bf(r);
-        } else {
-          // gradient through the activation of the tensor this one feeds
-          const float av = bf2f(act[v * Cout + co]);
-          out_bf[v * Cout + co] = f2bf(av > 0.f ? r : slope * r);
+    for (int i = 0; i < NP; i++)
+      if (lo[i] >= 0) *reinterpret_cast<uint4*>(planes + slot * pb + lo[i]) = pre[i];
+  };
+  load(zs - 1);
+  put(0);
+  load(zs);
+  put(1);
+  load(zs + 1);
+  const int row = lane & 15, kq = (lane >> 4) * 8, y = y0 + wave, K27 = 27 * Cin;
+  const char* av = planes + (wave * VX + row) * vs;
+  const bf16* wl = w + (long)row * Kpad + kq;
+  int ph = 0;   // slot of plane z - 1
+  for (int z = zs; z < ze; z++) {
+    put(ph == 0 ? 2 : ph - 1);   // plane z + 1, where plane z - 2 was
+    __syncthreads();
+    if (z + 1 < ze) load(z + 2);
+    if (y < Y) {   // uniform over the wave
+      f32x4 acc[MT][NT];
+#pragma unroll
+      for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int n = 0; n < NT; n++) acc[m][n] = f32x4{0, 0, 0, 0};
+      const int* tp = tab + ph * ng + (lane >> 4);
+      // the next G steps' weights are in flight while a step is computed
+      bf16x8 bw[G][NT];
+      auto weights = [&](int q, int k0) {
+        const int k = min(k0, Kpad - 32);
+#pragma unroll
+        for (int n = 0; n < NT; n++) {
+          if constexpr (WL) bw[q][n] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(wlds + (16 * n + row) * ws + 2 * (k + kq)));
+          else bw[q][n] = load8(wl + (long)16 * n * Kpad + k);
+        }
+      };
+      auto step = [&](int q, int k0, bool tail) {
+        const int off = tp[k0 / 8];
+        bf16x8 a[MT];
+#pragma unroll
+        for (int m = 0; m < MT; m++) {
+          a[m] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(av + off + 16 * m * vs));
+          if (tail && k0 + kq >= K27) a[m] = zero8();   // the padding of K
+        }
+#pragma unroll
+        for (int n = 0; n < NT; n++)
+#pragma unroll
+          for (int m = 0; m < MT; m++) acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[q][n], a[m], acc[m][n], 0, 0, 0);
+      };
+#pragma unroll
+      for (int q = 0; q < G; q++) weights(q, 32 * q);
+      int k0 = 0;
+      for (; k0 + 32 * G <= K27; k0 += 32 * G) {
+#pragma unroll
+        for (int q = 0; q < G; q++) {
+          step(q, k0 + 32 * q, false);
+          weights(q, k0 + 32 * (G + q));
         }
       }
+#pragma unroll
+      for (int q = 0; q < G; q++)
+        if (k0 + 32 * q < Kpad) step(q, k0 + 32 * q, true);
+      conv_epilogue<MT, NT>(acc, x0, y, z, Y, X, bias, epi, slope, act, out_bf, out_f, Cout_store);
     }
+    __syncthreads();
+    ph = ph == 2 ? 0 : ph + 1;
+  }
 }
 
 // dw partials: a block takes the three taps of one (dz, dy) for up to NCI
@@ -667,6 +827,35 @@ void conv_fwd_mt(const bf16* x, int Z, int Y, int X, int Cin, const bf16* w, int
   }
 }
 
+// LDS bytes of k_conv_fwd_lds for rows TY
+size_t conv_lds(int TY, int Cin, int Kpad) {
+  return 3 * (size_t)((TY + 2) * 34) * (2 * Cin + 16) + (3 * (Kpad / 8) * sizeof(int) + 15) / 16 * 16;
+}
+
+template <int TY, int NP>
+void conv_fwd_lds(const bf16* x, int Z, int Y, int X, int Cin, const bf16* w, int Kpad, int Cout, const float* bias,
+                  int epi, float slope, const bf16* act, bf16* ob, float* of, int cstore, hipStream_t s) {
+  const int tiles = ((X + 31) / 32) * ((Y + TY - 1) / TY);
+  const int zper = std::max(2, (int)((long)Z * tiles / 512));
+  const dim3 g((X + 31) / 32, (Y + TY - 1) / TY, (Z + zper - 1) / zper), b(64 * TY);
+  // the weights join the planes where they fit
+  const size_t planes = conv_lds(TY, Cin, Kpad), wl = (size_t)Cout * (2 * Kpad + 16);
+  const bool in_lds = planes + wl <= 160 * 1024;
+  const size_t lds = in_lds ? planes + wl : planes;
+  hipEvent_t e0, e1;
+  emmi::timing::kernel_events(emmi::timing::CONV, 54.0 * Cin * Cout * (double)Z * Y * X, &e0, &e1);
+  auto go = [&](auto kernel) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    if (e0) hipExtLaunchKernelGGL(kernel, g, b, lds, s, e0, e1, 0, x, Z, Y, X, Cin, w, Kpad, bias, epi, slope, act, ob, of, cstore, zper);
+    else hipLaunchKernelGGL(kernel, g, b, lds, s, x, Z, Y, X, Cin, w, Kpad, bias, epi, slope, act, ob, of, cstore, zper);
+  };
+  switch (Cout / 16) {
+#define CASE(NT) case NT: if (in_lds) go(k_conv_fwd_lds<NT, TY, NP, true>); else go(k_conv_fwd_lds<NT, TY, NP, false>); break;
+    CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
+#undef CASE
+  }
+}
+
 }  // namespace
 
 extern "C" {
@@ -679,6 +868,18 @@ int emmi_x0_conv_fwd(const void* x, int Z, int Y, int X, int Cin, const void* w,
   const int Kpad = emmi_x0_kpad(Cin);
   const bf16* xb = (const bf16*)x;
   const bf16* wb = (const bf16*)w;
+  // Rows of 32 voxels and more, in planes of at least eight rows, from LDS: eight
+  // rows where the planes of the tile fit it, four for more channels (up to 112)
+  if (X >= 32 && Y >= 8 && (long)Y * X * Cin < (1L << 31)) {
+    if (Cin <= 64 && conv_lds(8, Cin, Kpad) <= 160 * 1024) {
+      conv_fwd_lds<8, 6>(xb, Z, Y, X, Cin, wb, Kpad, Cout, bias, epi, slope, (const bf16*)act, (bf16*)out_bf16, out_f32, cout_store, S(stream));
+      return hipGetLastError() == hipSuccess ? 0 : -1;
+    }
+    if (Cin <= 112 && conv_lds(4, Cin, Kpad) <= 160 * 1024) {
+      conv_fwd_lds<4, 12>(xb, Z, Y, X, Cin, wb, Kpad, Cout, bias, epi, slope, (const bf16*)act, (bf16*)out_bf16, out_f32, cout_store, S(stream));
+      return hipGetLastError() == hipSuccess ? 0 : -1;
+    }
+  }
   if (X % 64 == 0) conv_fwd_mt<4>(xb, Z, Y, X, Cin, wb, Kpad, Cout, bias, epi, slope, (const bf16*)act, (bf16*)out_bf16, out_f32, cout_store, S(stream));
   else if (X % 32 == 0) conv_fwd_mt<2>(xb, Z, Y, X, Cin, wb, Kpad, Cout, bias, epi, slope, (const bf16*)act, (bf16*)out_bf16, out_f32, cout_store, S(stream));
   else conv_fwd_mt<1>(xb, Z, Y, X, Cin, wb, Kpad, Cout, bias, epi, slope, (const bf16*)act, (bf16*)out_bf16, out_f32, cout_store, S(stream));
