@@ -404,6 +404,22 @@ __device__ __forceinline__ void node_rhs_rec(const LineJob<T>& J, int pb, int pc
   }
 }
 
+// one of the five values of that record: the residual of perpendicular edge
+// k = 0..3 or of the along-line edge (k = 4)
+template <typename T, int A>
+__device__ __forceinline__ cxd node_rhs_row(const LineJob<T>& J, int pb, int pc, int p, int k) {
+  constexpr int B = (A + 1) % 3, C = (A + 2) % 3;
+  const Level<T>& L = J.L;
+  const typename cvec<T>::type* __restrict__ u = J.u;
+  const typename cvec<T>::type* __restrict__ f = J.f;
+  if (k == 0) pb--;
+  if (k == 2) pc--;
+  const long o = (long)pb * L.es[B] + (long)pc * L.es[C] + (long)p * L.es[A];
+  if (k < 2) return ld<T>(f, B * L.nc + o) - apply_row<T, B>(L, u, pb, pc, p, o);
+  if (k < 4) return ld<T>(f, C * L.nc + o) - apply_row<T, C>(L, u, pc, p, pb, o);
+  return ld<T>(f, A * L.nc + o) - apply_row<T, A>(L, u, p, pb, pc, o);
+}
+
 // the records of node p of a line into its chunked scratch records
 template <typename T>
 __device__ __forceinline__ void store_rhs_rec(const LineJob<T>& J, int line, int p, long nl,
@@ -1206,8 +1222,9 @@ __global__ void __launch_bounds__(128) k_line_solve(LinePack<T> P) {
 // 330 -> 218; 64 nodes, FP64, one 37 -> 24; 16 nodes 12.5 -> 9.5; one line of 96
 // nodes, eight right-hand sides 26 -> 16.
 constexpr int M_LDS = 160 * 1024;          // LDS of a CU
-// LDS of a line: 2 T - 1 node vectors (4 complex) and 2 T edges (1 complex)
-__host__ __device__ __forceinline__ int line_m_bytes(int n) { return 160 * HalfOrder(n).T - 64; }
+// LDS of a line: 2 T edges (1 complex), 2 T - 1 node vectors (4 complex) and
+// room for one more, which the last step's read of the node after next meets
+__host__ __device__ __forceinline__ int line_m_bytes(int n) { return 160 * HalfOrder(n).T; }
 static int line_m_lpb(int n) { return 8 * line_m_bytes(n) <= M_LDS ? 8 : 2; }
 static bool line_m_fits(int n) { return 2 * line_m_bytes(n) <= M_LDS; }
 
@@ -1241,138 +1258,83 @@ __device__ __forceinline__ double rec_val(double x) {
 // that are copied back (and waited for) at the end of the group
 __device__ __forceinline__ void node_end() { __builtin_amdgcn_sched_barrier(0); }
 
-// D = line_ring(N): nodes of factor records in flight per half
-template <typename T, int A, int LPB, int D>
-__global__ void __launch_bounds__(32 * LPB, 2) k_line_solve_m(LinePack<T> P) {
-  constexpr int BT = 32 * LPB, FC = fchunks<double>(), SC = schunks<double>();
-  extern __shared__ double2 mlds[];
-  const LineJob<T>& J = P.job[blockIdx.y];
-  const Level<T>& L = J.L;
-  const int N = L.n[A];
-  const int nl = J.nlo * J.nhi;
-  const int l0 = (int)xcd_block(blockIdx.x, gridDim.x) * LPB;
-  if (N < 2 || l0 >= nl) return;   // uniform over the block
-  const HalfOrder O(N);
-  const int m = O.m, T2 = 2 * O.T, TT = O.T;
-  const int nle = min(LPB, nl - l0);   // lines of this block
-  // edges: rho, then dE, in the order of the records; node vectors: sigma,
-  // then z, then x, in the same order without each half's first (boundary or
-  // padding) record.  Neighbouring threads of the first and last phase walk
-  // along x, so x lines lie one after another and other lines side by side.
-  double2* __restrict__ Q = mlds;
-  double2* __restrict__ X = mlds + T2 * LPB;
-  auto qslot = [&](int t2, int l) { return A == 0 ? l * T2 + t2 : t2 * LPB + l; };
-  auto xslot = [&](int s, int l) { return 4 * (A == 0 ? l * (T2 - 1) + s : s * LPB + l); };
-  // slot of the vector of record r (r = 0 and T have none)
-  auto xrec = [&](int r) { return r - 1 - (r > TT ? 1 : 0); };
+// One lane of the substitution of two lines by a wave (see above).  ST: lines
+// side by side in the block's LDS (the stride between a line's slots).
+template <typename T, int A, int D, int ST>
+struct HalfLane {
+  static constexpr int XS = 8 * ST, QS = 2 * ST;   // doubles between the slots of a line
+  static constexpr int RB = fchunks<double>() * 16;   // bytes of a factor record
+  int row, j, side, jr;
+  unsigned sg;            // sign of the swapped operand's even columns
+  double vr, vs, ncl;     // v (entry (j, row) of an A operand whose rows are all v); v of this half; -l W_a
+  const char* fb;         // factor records of the wave's lines from a uniform base,
+  unsigned fw, fr, fm;    // node d of the current group at a constant offset
+  const double* iwa;
+  int e0, de, last, TT;   // inner edge of node t: e0 + de t
+  bool exact;             // z is kept in FP64 (a single line: the coarsest level)
+  double *xq, *qa, *xm;   // LDS: vector component and edge of node t of the half, meeting node
+  int qx;                 // from the component jr to the other one
+  double2 rw[D], rr[D], wm;
+  double ri[D];
 
-  // ---------------- residual records ----------------
-  auto put_rec = [&](int p, int l, const Ch<double>(&c)[SC]) {
-    Q[qslot(O.edge(p), l)] = make_double2(rec_val<T>(c[4].v[0]), rec_val<T>(c[4].v[1]));
-    if (p >= 1) {
-      double2* x = X + xslot(xrec(O.node(p)), l);
-#pragma unroll
-      for (int i = 0; i < 4; i++) x[i] = make_double2(rec_val<T>(c[i].v[0]), rec_val<T>(c[i].v[1]));
-    }
-  };
-  // padding and boundary records
-  if (O.o > 0) {
-    const double2 zz = make_double2(0.0, 0.0);
-    for (int idx = threadIdx.x; idx < LPB * (O.o + 1); idx += BT) {
-      const int l = idx % LPB, t = idx / LPB;
-      if (t < O.o) Q[qslot(t, l)] = zz;
-      if (t < O.ob) Q[qslot(TT + t, l)] = zz;
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        if (t >= 1) X[xslot(t - 1, l) + i] = zz;
-        if (t >= 1 && t <= O.ob) X[xslot(TT - 1 + t - 1, l) + i] = zz;
-      }
-    }
-  }
-  // Along y and z, lines of 64 nodes and more are marched by runs of N / 32
-  // nodes (128 nodes, per launch of a colour: 120 -> 107 us FP64 with one
-  // right-hand side, 252 -> 224 FP32 with three); a block with few lines would
-  // leave most of its threads without a run (one line of 96 nodes: 23 us
-  // marched, 16 node by node).
-  bool march = false;
-  if constexpr (A != 0 && D == 8) march = N >= 64 && nle > LPB / 2;
-  if (march) {
-    if constexpr (A != 0 && D == 8) {
-      // runs of consecutive nodes marching along the line, lines fastest
-      constexpr int CH = BT / LPB;
-      const int l = (int)threadIdx.x % LPB, ch = (int)threadIdx.x / LPB;
-      const int run = (N + CH - 1) / CH;
-      const int p0 = ch * run, p1 = min(N, p0 + run);
-      if (l < nle && p0 < p1) {
-        int pb, pc;
-        line_of<T, A>(J, l0 + l, pb, pc);
-        line_rhs_march<T, A, double>(J, pb, pc, p0, p1, [&](int p, const Ch<double>(&c)[SC]) { put_rec(p, l, c); });
-      }
-    }
-  } else {
-    const int nn = nle * N;
-    for (int idx = threadIdx.x; idx < nn; idx += BT) {
-      const int l = A == 0 ? idx / N : idx % nle, p = A == 0 ? idx % N : idx / nle;
-      int pb, pc;
-      line_of<T, A>(J, l0 + l, pb, pc);
-      Ch<double> c[SC] = {};
-      node_rhs_rec<T, A>(J, pb, pc, p, c);
-      put_rec(p, l, c);
-    }
-  }
-  __syncthreads();
-
-  // ---------------- substitution ----------------
-  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  if (2 * wave < nle) {   // uniform over the wave
+  __device__ __forceinline__ HalfLane() {
     const int lane = threadIdx.x & 63;
-    const int row = lane >> 4, j = lane & 3, b = (lane >> 2) & 3, side = b >> 1;
-    // a wave without a second line runs its first line twice
-    const int l = min(2 * wave + (b & 1), nle - 1);
-    int pb, pc;
-    line_of<T, A>(J, l0 + l, pb, pc);
+    row = lane >> 4;
+    j = lane & 3;
+    side = (lane >> 3) & 1;
+    jr = j & 1;
+  }
+  // 1 for the lanes of the wave's second line
+  __device__ __forceinline__ int second() const { return (threadIdx.x >> 2) & 1; }
+  // line (pb, pc), the `dl`-th of the wave's lines, whose first is line
+  // `first` of the colour; x0, q0: the line's first slots in LDS
+  __device__ __forceinline__ void init(const Level<T>& L, const HalfOrder& O, int pb, int pc, const double* fac,
+                                       int first, int dl, bool exact_, double2* x0, double2* q0) {
     const LineGeo<T, A> G(L, pb, pc);
-    auto vk = [&](int k) { const double h = k < 2 ? G.Hc : G.Hb; return (k & 1) ? -h : h; };
-    const double vr = vk(row);                  // also entry (j, row) of an A operand whose rows are all v
-    const double vs = side ? -vr : vr;          // v of this half, component `row`
-    const double ncl = row == 0 ? G.Wb0 * G.Hc : row == 1 ? G.Wb1 * G.Hc : row == 2 ? G.Wc0 * G.Hb : G.Wc1 * G.Hb;   // -l W_a
-    const int jr = j & 1;
-    const unsigned sg = jr ? 0u : 0x80000000u;  // sign of the swapped operand's even columns
-    // factor records of the wave's lines from a uniform base, node d of the
-    // current group at a constant offset
-    const int rbytes = FC * 16;
-    const char* fb = reinterpret_cast<const char*>(J.fac) + (long)(l0 + 2 * wave) * O.records() * rbytes;
-    const unsigned fo = (unsigned)(((l - 2 * wave) * O.records() + side * TT) * rbytes);
-    const unsigned fw = fo + 16 * symidx(j, row), fr = fo + 160;
-    // 1/W of the inner edge: t - o on top, N + ob - 1 - t below (clamped: the
-    // padding's value meets z = 0)
-    const double* __restrict__ iwa = L.IW[A];
-    const int e0 = side ? N + O.ob - 1 : -O.o, de = side ? -1 : 1;
-    double2 rw[D], rr[D];
-    double ri[D];
-    auto load = [&](int d, const char* base, int t) {   // base: record t - d
-      rw[d] = *reinterpret_cast<const double2*>(base + d * rbytes + fw);
-      rr[d] = *reinterpret_cast<const double2*>(base + d * rbytes + fr);
-      ri[d] = iwa[min((unsigned)(e0 + de * t), (unsigned)(N - 1))];
-    };
-    // LDS: vector component and edge of node t of the half
-    constexpr int XS = A == 0 ? 8 : 8 * LPB, QS = A == 0 ? 2 : 2 * LPB;
-    double* xq = reinterpret_cast<double*>(X + xslot(side * (TT - 1), l)) - XS + 2 * row + jr;
-    double* qa = reinterpret_cast<double*>(Q + qslot(side * TT, l)) + jr;
-    const int qx = 1 - 2 * jr;   // from the component jr to the other one
-    auto neg = [&](double x) { return __longlong_as_double(__double_as_longlong(x) ^ ((unsigned long long)sg << 32)); };
-    // q = rho / d of an edge, component jr
-    auto qval = [&](double ra, double rb, double2 rd) { return fma(rb, neg(rd.y), ra * rd.x); };
-
+    const double h = row < 2 ? G.Hc : G.Hb;
+    vr = (row & 1) ? -h : h;
+    vs = side ? -vr : vr;
+    ncl = row == 0 ? G.Wb0 * G.Hc : row == 1 ? G.Wb1 * G.Hc : row == 2 ? G.Wc0 * G.Hb : G.Wc1 * G.Hb;
+    sg = jr ? 0u : 0x80000000u;
+    TT = O.T;
+    exact = exact_;
+    fb = reinterpret_cast<const char*>(fac) + (long)first * O.records() * RB;
+    const unsigned fl = (unsigned)(dl * O.records() * RB), sym = 16 * symidx(j, row);
+    fw = fl + side * TT * RB + sym;
+    fr = fl + side * TT * RB + 160;
+    fm = fl + 2 * TT * RB + sym;
+    // t - o on top, N + ob - 1 - t below (clamped: the padding's value meets z = 0)
+    iwa = L.IW[A];
+    e0 = side ? O.N + O.ob - 1 : -O.o;
+    de = side ? -1 : 1;
+    last = O.N - 1;
+    xq = reinterpret_cast<double*>(x0) + (side * (TT - 1) - 1) * XS + 2 * row + jr;
+    xm = reinterpret_cast<double*>(x0) + (2 * TT - 2) * XS + 2 * row + jr;
+    qa = reinterpret_cast<double*>(q0) + side * TT * QS + jr;
+    qx = 1 - 2 * jr;
+  }
+  __device__ __forceinline__ void load(int d, const char* base, int t) {   // base: record t - d
+    rw[d] = *reinterpret_cast<const double2*>(base + d * RB + fw);
+    rr[d] = *reinterpret_cast<const double2*>(base + d * RB + fr);
+    ri[d] = iwa[min((unsigned)(e0 + de * t), (unsigned)last)];
+  }
+  __device__ __forceinline__ void first_loads() {
 #pragma unroll
     for (int d = 0; d < D; d++) load(d, fb, d);
-    const double2 wm = *reinterpret_cast<const double2*>(fb + (unsigned)(((l - 2 * wave) * O.records() + T2) * rbytes + 16 * symidx(j, row)));
+    wm = *reinterpret_cast<const double2*>(fb + fm);
+  }
+  // q = rho / d of an edge, component jr
+  __device__ __forceinline__ double qval(double ra, double rb, double2 rd) const {
+    const double s = __longlong_as_double(__double_as_longlong(rd.y) ^ ((unsigned long long)sg << 32));
+    return fma(rb, s, ra * rd.x);
+  }
+  // both passes, on the records that first_loads() has under way
+  __device__ __forceinline__ void run() {
     // Software pipeline: a node's step runs its chain on operands prepared in
     // the step before, and prepares the next node's (coupling -B, right-hand
     // side g) and reads the LDS of the one after.
     double z = 0.0, q, sig, ra, rb;
-    // a single line (the coarsest level) is solved in FP64 throughout
-    auto zrec = [&](double v) { return nl > 1 ? rec_val<T>(v) : v; };
+    auto zrec = [&](double v) { return exact ? v : rec_val<T>(v); };
     // -B = -diag(l) - (v / d) v^T towards the node before, g of the node.  B all
     // but cancels on the node's gradient, which W^-1 amplifies in air: v.z is
     // summed first (one matrix instruction, rows all v) and then scaled, as an
@@ -1415,27 +1377,27 @@ __global__ void __launch_bounds__(32 * LPB, 2) k_line_solve_m(LinePack<T> P) {
     node_end();
     int t0 = 0;
     if (TT > D) {
-      load(0, fb + D * rbytes, D);
+      load(0, fb + D * RB, D);
       node_end();
 #pragma unroll
       for (int d = 1; d < D; d++) {
         fstep(d);
         node_end();
-        load(d, fb + D * rbytes, D + d);
+        load(d, fb + D * RB, D + d);
         node_end();
       }
       for (t0 = D; t0 < TT - D; t0 += D) {
-        xq += D * XS; qa += D * QS; fb += D * rbytes;
+        xq += D * XS; qa += D * QS; fb += D * RB;
 #pragma unroll
         for (int d = 0; d < D; d++) {
           fstep(d);
           node_end();
-          load(d, fb + D * rbytes, t0 + D + d);
+          load(d, fb + D * RB, t0 + D + d);
           node_end();
         }
       }
       // the last group's records stay for the back pass
-      xq += D * XS; qa += D * QS; fb += D * rbytes;
+      xq += D * XS; qa += D * QS; fb += D * RB;
       fstep(0);
       node_end();
     }
@@ -1449,7 +1411,6 @@ __global__ void __launch_bounds__(32 * LPB, 2) k_line_solve_m(LinePack<T> P) {
     double x;
     {
       const double ql = qval(qa[(D - 1) * QS], qa[(D - 1) * QS + qx], rr[D - 1]);
-      double* xm = reinterpret_cast<double*>(X + xslot(T2 - 2, l)) + 2 * row + jr;
       double y = bsub(z, vs * ql);
       y = *xm + (y + mpeer(y));
       x = mma(wm.x, y, 0.0);
@@ -1468,79 +1429,202 @@ __global__ void __launch_bounds__(32 * LPB, 2) k_line_solve_m(LinePack<T> P) {
       eim = rr[d].y;
       eq = qval(ra, rb, rr[d]);
     };
+    // (from the slot before the group, as LDS offsets are not negative)
+    double *xb = xq - XS, *qb = qa - QS;
     auto bread = [&](int d) {   // rho of node d's inner edge
-      ra = qa[d * QS];
-      rb = qa[d * QS + qx];
+      ra = qb[(d + 1) * QS];
+      rb = qb[(d + 1) * QS + qx];
     };
     // to: where the pending edge goes
     auto bstep = [&](int d, double* to) {
       const double y = bsub(x, 0.0);
       double xp = mma(rw[d].x, y, sig);
       xp = mma(rw[d].y, mswap(y, sg), xp);
-      sig = xq[(d - 1) * XS];
+      sig = xb[d * XS];
       edge(to);
       bedge(d);
       bread(d - 1);
       couple((d + D - 1) % D);
       dx = x - xp;
-      xq[d * XS] = xp;
+      xb[(d + 1) * XS] = xp;
       x = xp;
     };
     couple(D - 1);
     bread(D - 1);
     // no edge is pending at first: that write lands on the edge whose rho has
     // just been read and which the next step writes
-    double* qe = qa + (D - 1) * QS;
+    double* qe = qb + D * QS;
     for (; t0 > 0; t0 -= D) {
 #pragma unroll
       for (int d = D - 1; d >= 0; d--) {
-        bstep(d, d == D - 1 ? qe : qa + (d + 1) * QS);
+        bstep(d, d == D - 1 ? qe : qb + (d + 2) * QS);
         node_end();
         // a slot is reloaded one step after its node: that node's edge is
         // still pending until then
         if (d == D - 1) load(0, fb, t0);
-        else load(d + 1, fb - D * rbytes, t0 - D + d + 1);
+        else load(d + 1, fb - D * RB, t0 - D + d + 1);
         node_end();
       }
-      qe = qa;
-      xq -= D * XS; qa -= D * QS; fb -= D * rbytes;
+      qe = qb + QS;
+      xb -= D * XS; qb -= D * QS; fb -= D * RB;
     }
 #pragma unroll
     for (int d = D - 1; d >= 1; d--) {
-      bstep(d, d == D - 1 ? qe : qa + (d + 1) * QS);
+      bstep(d, d == D - 1 ? qe : qb + (d + 2) * QS);
       node_end();
       if (d == D - 1) load(0, fb, 0);
       node_end();
     }
-    edge(qa + QS);
+    edge(qb + 2 * QS);
     // the first node's correction is zero: its inner edge alone
     bedge(0);
     dx = x;
-    edge(qa);
+    edge(qb + QS);
+  }
+};
+
+// D = line_ring(N): nodes of factor records in flight per half.  MODE: how the
+// residual records are built -- M_MARCH by marching along the lines, M_NODES
+// node by node, M_SHORT the same for blocks of at most a node per thread,
+// whose launch is a chain of memory latencies: it loads its first factor
+// records and the u that it will update ahead of the residual phase.
+enum { M_NODES = 0, M_MARCH = 1, M_SHORT = 2 };
+template <typename T, int A, int LPB, int D, int MODE>
+__global__ void __launch_bounds__(32 * LPB, 2) k_line_solve_m(LinePack<T> P) {
+  constexpr int BT = 32 * LPB, SC = schunks<double>();
+  extern __shared__ double2 mlds[];
+  const LineJob<T>& J = P.job[blockIdx.y];
+  const Level<T>& L = J.L;
+  const int N = L.n[A];
+  const int nl = J.nlo * J.nhi;
+  const int l0 = (int)xcd_block(blockIdx.x, gridDim.x) * LPB;
+  if (N < 2 || l0 >= nl) return;   // uniform over the block
+  const HalfOrder O(N);
+  const int T2 = 2 * O.T, TT = O.T;
+  const int nle = min(LPB, nl - l0);   // lines of this block
+  // edges: rho, then dE, in the order of the records; node vectors: sigma,
+  // then z, then x, in the same order without each half's first (boundary or
+  // padding) record.  Neighbouring threads of the first and last phase walk
+  // along x, so x lines lie one after another and other lines side by side.
+  double2* __restrict__ Q = mlds;
+  double2* __restrict__ X = mlds + T2 * LPB;
+  auto qslot = [&](int t2, int l) { return A == 0 ? l * T2 + t2 : t2 * LPB + l; };
+  auto xslot = [&](int s, int l) { return 4 * (A == 0 ? l * (T2 - 1) + s : s * LPB + l); };
+  // slot of the vector of record r (r = 0 and T have none)
+  auto xrec = [&](int r) { return r - 1 - (r > TT ? 1 : 0); };
+
+  // ---------------- the lane of the substitution ----------------
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const bool live = 2 * wave < nle;   // uniform over the wave
+  HalfLane<T, A, D, A == 0 ? 1 : LPB> H;
+  {
+    // a wave without a second line runs its first line twice
+    const int l = live ? min(2 * wave + H.second(), nle - 1) : 0, l2 = live ? 2 * wave : 0;
+    int pb, pc;
+    line_of<T, A>(J, l0 + l, pb, pc);
+    H.init(L, O, pb, pc, J.fac, l0 + l2, l - l2, nl == 1, X + xslot(0, l), Q + qslot(0, l));
+  }
+  if constexpr (MODE == M_SHORT) H.first_loads();
+
+  // ---------------- residual records ----------------
+  auto put_rec = [&](int p, int l, const Ch<double>(&c)[SC]) {
+    Q[qslot(O.edge(p), l)] = make_double2(rec_val<T>(c[4].v[0]), rec_val<T>(c[4].v[1]));
+    if (p >= 1) {
+      double2* x = X + xslot(xrec(O.node(p)), l);
+#pragma unroll
+      for (int i = 0; i < 4; i++) x[i] = make_double2(rec_val<T>(c[i].v[0]), rec_val<T>(c[i].v[1]));
+    }
+  };
+  // padding and boundary records
+  if (O.o > 0) {
+    const double2 zz = make_double2(0.0, 0.0);
+    for (int idx = threadIdx.x; idx < LPB * (O.o + 1); idx += BT) {
+      const int l = idx % LPB, t = idx / LPB;
+      if (t < O.o) Q[qslot(t, l)] = zz;
+      if (t < O.ob) Q[qslot(TT + t, l)] = zz;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        if (t >= 1) X[xslot(t - 1, l) + i] = zz;
+        if (t >= 1 && t <= O.ob) X[xslot(TT - 1 + t - 1, l) + i] = zz;
+      }
+    }
+  }
+  const int nn = nle * N;
+  auto node_of = [&](int idx, int& l, int& p) {
+    l = A == 0 ? idx / N : idx % nle;
+    p = A == 0 ? idx % N : idx / nle;
+  };
+  if constexpr (MODE == M_MARCH) {
+    // runs of consecutive nodes marching along the line, lines fastest
+    constexpr int CH = BT / LPB;
+    const int l = (int)threadIdx.x % LPB, ch = (int)threadIdx.x / LPB;
+    const int run = (N + CH - 1) / CH;
+    const int p0 = ch * run, p1 = min(N, p0 + run);
+    if (l < nle && p0 < p1) {
+      int pb, pc;
+      line_of<T, A>(J, l0 + l, pb, pc);
+      line_rhs_march<T, A, double>(J, pb, pc, p0, p1, [&](int p, const Ch<double>(&c)[SC]) { put_rec(p, l, c); });
+    }
+  } else if (MODE == M_SHORT && 4 * nn <= BT) {
+    // few nodes: a thread per row (rows in the order of the records, rho last)
+    for (int idx = threadIdx.x; idx < 5 * nn; idx += BT) {
+      const int k = idx / nn;
+      int l, p, pb, pc;
+      node_of(idx - k * nn, l, p);
+      line_of<T, A>(J, l0 + l, pb, pc);
+      if (k == 4 || p >= 1) {
+        const cxd r = node_rhs_row<T, A>(J, pb, pc, p, k);
+        double2* to = k == 4 ? Q + qslot(O.edge(p), l) : X + xslot(xrec(O.node(p)), l) + k;
+        *to = make_double2(rec_val<T>(r.re), rec_val<T>(r.im));
+      }
+    }
+  } else {
+    for (int idx = threadIdx.x; idx < nn; idx += BT) {
+      int l, p, pb, pc;
+      node_of(idx, l, p);
+      line_of<T, A>(J, l0 + l, pb, pc);
+      Ch<double> c[SC] = {};
+      node_rhs_rec<T, A>(J, pb, pc, p, c);
+      put_rec(p, l, c);
+    }
+  }
+  typename cvec<T>::type* __restrict__ u = J.u;
+  typename cvec<T>::type uv[5];
+  long uo[5];
+  auto u_of = [&](int idx, int& l, int& p) {
+    constexpr int B = (A + 1) % 3, C = (A + 2) % 3;
+    int pb, pc;
+    node_of(idx, l, p);
+    line_of<T, A>(J, l0 + l, pb, pc);
+    const long o = (long)pb * L.es[B] + (long)pc * L.es[C] + (long)p * L.es[A];
+    uo[0] = A * L.nc + o;
+    uo[1] = B * L.nc + o - L.es[B];
+    uo[2] = B * L.nc + o;
+    uo[3] = C * L.nc + o - L.es[C];
+    uo[4] = C * L.nc + o;
+#pragma unroll
+    for (int i = 0; i < 5; i++) uv[i] = u[i == 0 || p >= 1 ? uo[i] : uo[0]];
+  };
+  int ul = 0, up = 0;
+  if (MODE == M_SHORT && (int)threadIdx.x < nn) u_of(threadIdx.x, ul, up);
+  __syncthreads();
+
+  // ---------------- substitution ----------------
+  if (live) {
+    if constexpr (MODE != M_SHORT) H.first_loads();
+    H.run();
   }
   __syncthreads();
 
   // ---------------- u += corrections ----------------
-  {
-    typename cvec<T>::type* __restrict__ u = J.u;
-    const int nn = nle * N;
-    for (int idx = threadIdx.x; idx < nn; idx += BT) {
-      const int l = A == 0 ? idx / N : idx % nle, p = A == 0 ? idx % N : idx / nle;
-      int pb, pc;
-      line_of<T, A>(J, l0 + l, pb, pc);
-      constexpr int B = (A + 1) % 3, C = (A + 2) % 3;
-      const long o = (long)pb * L.es[B] + (long)pc * L.es[C] + (long)p * L.es[A];
-      const double2 e = Q[qslot(O.edge(p), l)];
-      st<T>(u, A * L.nc + o, ld<T>(u, A * L.nc + o) + cxd(e.x, e.y));
-      if (p >= 1) {
-        const double2* x = X + xslot(xrec(O.node(p)), l);
-        const long offs[4] = {B * L.nc + o - L.es[B], B * L.nc + o, C * L.nc + o - L.es[C], C * L.nc + o};
-        cxd v[4];
+  for (int idx = threadIdx.x; idx < nn; idx += BT) {
+    if (MODE != M_SHORT) u_of(idx, ul, up);
+    auto add = [&](int i, double2 d) { st<T>(u, uo[i], cxd((double)uv[i].x, (double)uv[i].y) + cxd(d.x, d.y)); };
+    add(0, Q[qslot(O.edge(up), ul)]);
+    if (up >= 1) {
+      const double2* x = X + xslot(xrec(O.node(up)), ul);
 #pragma unroll
-        for (int i = 0; i < 4; i++) v[i] = ld<T>(u, offs[i]);
-#pragma unroll
-        for (int i = 0; i < 4; i++) st<T>(u, offs[i], v[i] + cxd(x[i].x, x[i].y));
-      }
+      for (int i = 0; i < 4; i++) add(i + 1, x[i]);
     }
   }
 }
@@ -1682,14 +1766,31 @@ static void launch_line_m_axis(const LinePack<T>& P, int maxl, int maxna, hipStr
   const dim3 g((unsigned)((maxl + lpb - 1) / lpb), P.njobs), b(32 * lpb);
   const size_t lds = (size_t)lpb * line_m_bytes(maxna);
   auto go = [&](auto kernel) { launch_lds(kernel, g, b, lds, s, timing::LINE, by, P); };
+  // Along y and z, lines of 64 nodes and more are marched by runs of N / 32
+  // nodes (128 nodes, per launch of a colour: 120 -> 107 us FP64 with one
+  // right-hand side, 252 -> 224 FP32 with three); a launch with few lines would
+  // leave most threads of its block without a run (one line of 96 nodes: 23 us
+  // marched, 16 node by node).
+  if constexpr (A != 0) {
+    if (D == 8 && maxna >= 64 && maxl > 4) {
+      if (lpb == 2) go(k_line_solve_m<T, A, 2, 8, M_MARCH>);
+      else go(k_line_solve_m<T, A, 8, 8, M_MARCH>);
+      return;
+    }
+  }
   if (lpb == 2) {
-    if (D == 8) go(k_line_solve_m<T, A, 2, 8>);
-    else if (D == 4) go(k_line_solve_m<T, A, 2, 4>);
-    else go(k_line_solve_m<T, A, 2, 2>);
+    if (D == 8) go(k_line_solve_m<T, A, 2, 8, M_NODES>);
+    else go(k_line_solve_m<T, A, 2, 4, M_NODES>);
+  } else if (maxna <= 32 && D < 8 && (long)g.x * P.njobs <= 256) {
+    // at most a block per CU (the look-ahead takes the registers of a second:
+    // solves of one slot 64^3 10.3 -> 10.1 ms, 12x10x16 13.1 -> 12.8; eight slots
+    // on 96^3 without this limit 55.6 -> 56.4)
+    if (D == 4) go(k_line_solve_m<T, A, 8, 4, M_SHORT>);
+    else go(k_line_solve_m<T, A, 8, 2, M_SHORT>);
   } else {
-    if (D == 8) go(k_line_solve_m<T, A, 8, 8>);
-    else if (D == 4) go(k_line_solve_m<T, A, 8, 4>);
-    else go(k_line_solve_m<T, A, 8, 2>);
+    if (D == 8) go(k_line_solve_m<T, A, 8, 8, M_NODES>);
+    else if (D == 4) go(k_line_solve_m<T, A, 8, 4, M_NODES>);
+    else go(k_line_solve_m<T, A, 8, 2, M_NODES>);
   }
 }
 template <typename T>
