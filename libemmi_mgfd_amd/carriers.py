@@ -100,18 +100,21 @@ class Tables:
         return a.ctypes.data_as(FP)
 
     def _tables(self, base_addr, shape, itemsize, elem_ptr, levels):
-        # rows of the innermost dimension, then each outer level
+        # rows of the innermost dimension, then each outer level; the tables are
+        # address arrays seen as pointers (made one by one in Python, the tables
+        # of a 101 x 101 x 81 model took 50 ms)
         shape = tuple(shape)
-        nrows = int(np.prod(shape[:-1]))
-        rows = (elem_ptr * nrows)(*[C.cast(base_addr + r * shape[-1] * itemsize, elem_ptr) for r in range(nrows)])
-        self.keep.append(rows)
-        cur, cur_type = rows, elem_ptr
+
+        def table(n, base, stride, ptype):
+            t = (ptype * n).from_buffer(np.uint64(base) + np.arange(n, dtype=np.uint64) * np.uint64(stride))
+            self.keep.append(t)
+            return t
+
+        cur, cur_type = table(int(np.prod(shape[:-1])), base_addr, shape[-1] * itemsize, elem_ptr), elem_ptr
         for d in range(len(shape) - 2, 0, -1):
-            n = int(np.prod(shape[:d]))
             ptype = C.POINTER(cur_type)
-            tab = (ptype * n)(*[C.cast(C.addressof(cur) + i * shape[d] * C.sizeof(cur_type), ptype) for i in range(n)])
-            self.keep.append(tab)
-            cur, cur_type = tab, ptype
+            cur = table(int(np.prod(shape[:d])), C.addressof(cur), shape[d] * C.sizeof(cur_type), ptype)
+            cur_type = ptype
         return C.cast(C.addressof(cur), C.POINTER(cur_type))
 
     def f3(self, a) -> FPPP:

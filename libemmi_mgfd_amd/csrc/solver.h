@@ -42,6 +42,25 @@ struct SolveStats {
 
 void check_hip(hipError_t e, const char* what);
 
+// Device memory of one owner, carved from blocks that double up to 64 MiB
+// (requests of 16 MiB and more get blocks of their own) and are all freed with
+// it.  A solver of four 64^3 slots holds some 900 buffers, most of them a few
+// KiB; one hipFree each took 53 ms of the 190 of a whole survey call, now 6.
+class Arena {
+ public:
+  Arena() = default;
+  Arena(const Arena&) = delete;
+  Arena& operator=(const Arena&) = delete;
+  ~Arena() { release(); }
+  void* get(size_t bytes);
+  void release();
+
+ private:
+  std::vector<void*> blocks_;
+  char* cur_ = nullptr;
+  size_t left_ = 0, next_ = size_t(1) << 20;
+};
+
 struct HostAxis {
   std::vector<double> x, xs, d, ds;
   void from_nodes(const std::vector<double>& nodes);  // src/gmg.c:1672-1685
@@ -219,7 +238,7 @@ class Solver {
   double* blend_part_ = nullptr;   // blend_guess: partial sums and their total (allocated on first use)
   double* blend_dots_ = nullptr;
   double* hnorm_ = nullptr;   // pinned host, one per slot
-  std::vector<void*> owned_;
+  Arena owned_;
   // state of the running batch
   std::vector<int> act_;      // active slots
   int icycle_ = 0;

@@ -86,12 +86,41 @@ static int depth_of(int n) {
   return l;
 }
 
-static void* dalloc(size_t bytes, std::vector<void*>& owned) {
+void* Arena::get(size_t bytes) {
+  constexpr size_t ALIGN = 256, OWN = size_t(16) << 20, MOST = size_t(64) << 20;
+  bytes = (std::max<size_t>(bytes, 1) + ALIGN - 1) / ALIGN * ALIGN;
+  const bool own = bytes >= OWN;
+  if (!own && bytes <= left_) {
+    void* p = cur_;
+    cur_ += bytes;
+    left_ -= bytes;
+    return p;
+  }
+  const size_t size = own ? bytes : std::max(bytes, next_);
+  blocks_.push_back(nullptr);   // (grows before the memory is ours)
   void* p = nullptr;
-  HIPCHECK(hipMalloc(&p, bytes ? bytes : 16));
-  owned.push_back(p);
+  const hipError_t e = hipMalloc(&p, size);
+  if (e != hipSuccess) {
+    blocks_.pop_back();
+    check_hip(e, "hipMalloc");
+  }
+  blocks_.back() = p;
+  if (!own) {
+    cur_ = (char*)p + bytes;
+    left_ = size - bytes;
+    next_ = std::min(MOST, 2 * next_);
+  }
   return p;
 }
+
+void Arena::release() {
+  for (void* p : blocks_) (void)hipFree(p);
+  blocks_.clear();
+  cur_ = nullptr;
+  left_ = 0;
+}
+
+static void* dalloc(size_t bytes, Arena& owned) { return owned.get(bytes); }
 
 template <> Hier<double>& Solver::hier<double>(int m) { return meds_[m].h64; }
 template <> Hier<float>& Solver::hier<float>(int m) { return meds_[m].h32; }
@@ -178,7 +207,7 @@ void Solver::init(int n1, int n2, int n3, int nmed, const float* const* x1, cons
 
     // ---- medium: sigma*vol cells on the device, all levels and patterns ----
     const long ncell0 = (long)n1 * n2 * n3;
-    std::vector<void*> tmp;
+    Arena tmp;
     std::vector<std::vector<double*>> cells(npat_ * lmax_);  // [pat*lmax+lev][3]
     double* W[3];
     for (int a = 0; a < 3; a++) {
@@ -222,7 +251,7 @@ void Solver::init(int n1, int n2, int n3, int nmed, const float* const* x1, cons
       M.l0_64 = one.pat[0][0];
     }
     HIPCHECK(hipStreamSynchronize(s_));
-    for (void* t : tmp) HIPCHECK(hipFree(t));
+    tmp.release();
   }
 
   // records of the line solves: max over levels, patterns, axes and colours
@@ -263,7 +292,7 @@ void Solver::init(int n1, int n2, int n3, int nmed, const float* const* x1, cons
 Solver::~Solver() {
   hipStreamSynchronize(s_);
   drop_graphs();
-  for (void* p : owned_) hipFree(p);
+  owned_.release();
   if (hnorm_) hipHostFree(hnorm_);
 }
 
