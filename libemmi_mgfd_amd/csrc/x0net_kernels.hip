@@ -56,6 +56,8 @@ __device__ __forceinline__ void conv_epilogue(const f32x4 (&acc)[MT][NT], int x0
                                               float* __restrict__ out_f, int Cout_store) {
   constexpr int Cout = 16 * NT;
   const int lane = threadIdx.x & 63, c4 = 4 * (lane >> 4);
+  // four channels at once where the tensors' bases allow it (uniform)
+  const bool vec = ((reinterpret_cast<uintptr_t>(out_bf) | reinterpret_cast<uintptr_t>(act)) & 7) == 0;
   auto pack = [](const f32x4& r) {
     return make_uint2((unsigned)f2bf(r[0]) | ((unsigned)f2bf(r[1]) << 16), (unsigned)f2bf(r[2]) | ((unsigned)f2bf(r[3]) << 16));
   };
@@ -69,16 +71,22 @@ __device__ __forceinline__ void conv_epilogue(const f32x4 (&acc)[MT][NT], int x0
       f32x4 r = acc[m][n];
       const int co = 16 * n + c4;
       if (epi == EPI_LEAKY || (epi == EPI_LINEAR && bias)) {
-        const float4 bb = *reinterpret_cast<const float4*>(bias + co);
-        r[0] += bb.x; r[1] += bb.y; r[2] += bb.z; r[3] += bb.w;
+#pragma unroll
+        for (int i = 0; i < 4; i++) r[i] += bias[co + i];
       }
       if (epi == EPI_LEAKY) {
 #pragma unroll
         for (int i = 0; i < 4; i++) r[i] = r[i] > 0.f ? r[i] : slope * r[i];
       } else if (epi == EPI_DACT) {
         // gradient through the activation of the tensor this one feeds
-        const uint2 av = *reinterpret_cast<const uint2*>(act + v * Cout + co);
-        const bf16 a4[4] = {(bf16)av.x, (bf16)(av.x >> 16), (bf16)av.y, (bf16)(av.y >> 16)};
+        bf16 a4[4];
+        if (vec) {
+          const uint2 av = *reinterpret_cast<const uint2*>(act + v * Cout + co);
+          a4[0] = (bf16)av.x; a4[1] = (bf16)(av.x >> 16); a4[2] = (bf16)av.y; a4[3] = (bf16)(av.y >> 16);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; i++) a4[i] = act[v * Cout + co + i];
+        }
 #pragma unroll
         for (int i = 0; i < 4; i++) r[i] = bf2f(a4[i]) > 0.f ? r[i] : slope * r[i];
       }
@@ -86,8 +94,11 @@ __device__ __forceinline__ void conv_epilogue(const f32x4 (&acc)[MT][NT], int x0
 #pragma unroll
         for (int i = 0; i < 4; i++)
           if (co + i < Cout_store) out_f[v * Cout_store + co + i] = r[i];
-      } else {
+      } else if (vec) {
         *reinterpret_cast<uint2*>(out_bf + v * Cout + co) = pack(r);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++) out_bf[v * Cout + co + i] = f2bf(r[i]);
       }
     }
   }

@@ -83,3 +83,34 @@ def test_convolution_matches_64_bit(shape, ci, co):
         torch.cuda.synchronize()
         ref = (g.double().t() @ t.reshape(nv, -1))
         assert rel(dw.cpu().double(), ref) < 1e-5 and rel(db.cpu().double(), g.double().sum(0)) < 1e-5
+
+
+@pytest.mark.parametrize("shape", [(2, 9, 33), (2, 5, 7)], ids=["rows_of_33", "rows_of_7"])
+def test_outputs_at_any_element_offset(shape):
+    """bias, act and the outputs may start at any element of a buffer: the
+    results are those of aligned ones, bit for bit, and nothing beside them is
+    written."""
+    from libemmi_mgfd_amd import x0net
+    Z, Y, X = shape
+    nv, ci, co = Z * Y * X, 16, 32
+    gen = torch.Generator().manual_seed(3)
+    x = torch.randn((nv, ci), generator=gen).to(torch.bfloat16).cuda()
+    act = torch.randn(nv * co + 1, generator=gen).to(torch.bfloat16).cuda()
+    w = torch.randn((co, 27 * ci), generator=gen).cuda()
+    bias = torch.randn(co + 1, generator=gen).cuda()
+    L = x0net._lib()
+    wf = torch.empty((co, x0net.kpad(ci)), dtype=torch.bfloat16, device="cuda")
+    wt = torch.empty((ci, x0net.kpad(co)), dtype=torch.bfloat16, device="cuda")
+    assert L.emmi_x0_prep_weights(w.data_ptr(), ci, co, wf.data_ptr(), wt.data_ptr(), None) == 0
+    ab, bb = act[1:].clone(), bias[1:].clone()
+    for epi in (0, 2, 3):
+        print(f"conv {shape} epilogue {epi}, outputs one element on", flush=True)
+        outs = []
+        for a, b, off in ((ab.data_ptr(), bb.data_ptr(), 0), (act.data_ptr() + 2, bias.data_ptr() + 4, 1)):
+            ob = torch.full((nv * co + 2,), 7.0, dtype=torch.bfloat16, device="cuda")
+            assert L.emmi_x0_conv_fwd(x.data_ptr(), Z, Y, X, ci, wf.data_ptr(), co, b, epi, x0net.SLOPE, a,
+                                      ob.data_ptr() + 2 * off, None, 0, None) == 0
+            torch.cuda.synchronize()
+            assert float(ob[nv * co + off]) == 7.0 and (off == 0 or float(ob[0]) == 7.0)
+            outs.append(ob[off:off + nv * co].clone())
+        assert torch.equal(outs[0], outs[1])
