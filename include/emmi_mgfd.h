@@ -394,6 +394,10 @@ int emmi_device_sync(void);
  * line systems exactly.  Graphs a solver captured earlier keep the kernels they
  * captured.  Returns the previous mode, or -1 for an unknown mode. */
 int emmi_set_line_kernel(int mode);
+/* the substitution that a launch over njobs jobs (1 to 16), job j with lines of
+ * cells[j] cells, takes in the current mode (without the autotuner's table): 0
+ * one lane per line half, 1 matrix cores.  Host only.  -1: njobs out of range */
+int emmi_line_route(int njobs, const int *cells);
 /* kernel timing: accumulated milliseconds, launch counts and compulsory
  * bytes (each input read once, each output written once per launch at its
  * level's shape; a full line sweep, all four colours, counts 3 Ne s + 3 Nc c)

@@ -289,6 +289,11 @@ int emmi_device_sync(void) { return hipDeviceSynchronize() == hipSuccess ? 0 : -
 
 int emmi_set_line_kernel(int mode) { return emmi::set_line_kernel(mode); }
 
+int emmi_line_route(int njobs, const int* cells) {
+  if (njobs < 1 || njobs > emmi::LINE_PACK_MAX || !cells) return -1;
+  return emmi::line_route_now(njobs, cells);
+}
+
 int emmi_solver_kernel_rates(emmi_solver_t* h, int reps, double* ms, double* bytes, int n) {
   if (!h || !h->s) { set_err("null solver"); return EMMI_ERROR; }
   try {

@@ -6,8 +6,8 @@
 // on grid, medium and frequency only) and every sweep then computes the
 // lines' right-hand sides and runs a forward/back substitution
 // (k_line_solve_m, or k_line_rhs* and k_line_solve).  A launch takes a pack of
-// up to LINE_PACK_MAX jobs (one per right-hand side or per level) that share
-// the axis and colour.
+// up to LINE_PACK_MAX jobs (one per right-hand side) that share the axis and
+// colour; jobs whose lines differ in length take the one-lane kernel.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -67,6 +67,14 @@ inline void line_job_colour(LineJob<T>& J, int a, int colour) {
 // (they named kernels that the matrix-core one replaced); returns the previous
 // mode or -1
 int set_line_kernel(int mode);
+
+// The substitution that a launch takes: the matrix-core kernel lays out its
+// records, LDS and groups for one length, so every job's lines must have it
+// (and fit the LDS); one_lane: that kernel is asked for.
+enum LineRoute { LINE_ROUTE_ONE_LANE = 0, LINE_ROUTE_MATRIX = 1 };
+LineRoute line_route(int njobs, const int* cells, bool one_lane);
+// the route under the current mode, without the autotuner's table
+LineRoute line_route_now(int njobs, const int* cells);
 
 // Autotuning: a launch shape (value size of the cycle precision, axis, line
 // length, lines per job, jobs per pack) and the substitution choice measured

@@ -1640,7 +1640,16 @@ void line_colour_counts(const int* n, int a, int colour, int* nlo, int* nhi) {
   if (b < c) { *nlo = nbv; *nhi = ncv; } else { *nlo = ncv; *nhi = nbv; }
 }
 
+LineRoute line_route(int njobs, const int* cells, bool one_lane) {
+  if (one_lane || njobs < 1) return LINE_ROUTE_ONE_LANE;
+  for (int j = 1; j < njobs; j++)
+    if (cells[j] != cells[0]) return LINE_ROUTE_ONE_LANE;
+  return line_m_fits(cells[0]) ? LINE_ROUTE_MATRIX : LINE_ROUTE_ONE_LANE;
+}
+
 static int g_line_kernel = 0;
+
+LineRoute line_route_now(int njobs, const int* cells) { return line_route(njobs, cells, g_line_kernel == 1); }
 
 int set_line_kernel(int mode) {
   if (mode < 0 || mode > 4) return -1;
@@ -1824,8 +1833,11 @@ static void launch_pack(const LinePack<T>& P, int axis, bool factor, hipStream_t
     rec_bytes += (double)nl * na * SREC * sizeof(ScrRec<T>);
   }
   if (maxl == 0 || P.njobs == 0) return;
-  int maxna = 0;
-  for (int j = 0; j < P.njobs; j++) maxna = std::max(maxna, P.job[j].L.n[axis]);
+  int maxna = 0, cells[LINE_PACK_MAX];
+  for (int j = 0; j < P.njobs; j++) {
+    cells[j] = P.job[j].L.n[axis];
+    maxna = std::max(maxna, cells[j]);
+  }
   if (factor) {
     const dim3 g((maxl + 63) / 64, P.njobs), b(64);
     timing::Scope ts(timing::OTHER, s, 0);
@@ -1834,11 +1846,11 @@ static void launch_pack(const LinePack<T>& P, int axis, bool factor, hipStream_t
     else hipLaunchKernelGGL((k_line_factor<T, 2>), g, b, 0, s, P);
     return;
   }
-  // the matrix-core substitution takes every line that fits its LDS records;
-  // longer ones (and forced launches) take the one-lane kernel
+  // the matrix-core substitution takes lines of one length that fit its LDS
+  // records; longer ones (and forced launches) take the one-lane kernel
   if (choice == LINE_RULE && g_line_kernel == 0) choice = tuned_choice(line_shape(P, axis));
   const bool one_lane = choice == LINE_ONE_LANE || (choice == LINE_RULE && g_line_kernel == 1);
-  if (!one_lane && line_m_fits(maxna)) {
+  if (line_route(P.njobs, cells, one_lane) == LINE_ROUTE_MATRIX) {
     launch_line_m<T>(P, axis, maxl, maxna, s, Bytes{comp, rhs_bytes + solve_bytes - 2.0 * rec_bytes});
     return;
   }
