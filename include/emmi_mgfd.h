@@ -388,16 +388,17 @@ int emmi_memcpy_d2h(void *dst, const void *src, size_t bytes);
 int emmi_memcpy_d2d(void *dst, const void *src, size_t bytes);
 int emmi_device_sync(void);
 /* Line-substitution kernel of the following launches (no counterpart in the
- * reference; for tests and tuning): 0 the matrix-core kernel wherever a line
- * fits it (default; the autotuner's table is consulted), 1 one lane per line
- * half, 2 to 4 the matrix-core kernel without the table.  All solve the same
- * line systems exactly.  Graphs a solver captured earlier keep the kernels they
- * captured.  Returns the previous mode, or -1 for an unknown mode. */
+ * reference; for tests and tuning): 0 the matrix-core kernel (default; the
+ * autotuner's table is consulted), 1 one lane per line half, 2 to 4 the
+ * matrix-core kernel without the table.  All solve the same line systems
+ * exactly.  Graphs a solver captured earlier keep the kernels they captured.  Returns the previous mode, or -1 for an unknown mode. */
 int emmi_set_line_kernel(int mode);
-/* the substitution that a launch over njobs jobs (1 to 16), job j with lines of
- * cells[j] cells, takes in the current mode (without the autotuner's table): 0
- * one lane per line half, 1 matrix cores.  Host only.  -1: njobs out of range */
-int emmi_line_route(int njobs, const int *cells);
+/* the substitution that a launch over njobs jobs (1 to 16) along an axis takes
+ * in the current mode (without the autotuner's table), job j having lines[j]
+ * lines of cells[j] cells in cycles of esize-byte (4 or 8) values: 0 one lane
+ * per line half, 1 matrix cores, 2 matrix cores with the line records in
+ * memory.  Host only.  -1: an argument out of range */
+int emmi_line_route(int esize, int axis, int njobs, const int *cells, const long *lines);
 /* kernel timing: accumulated milliseconds, launch counts and compulsory
  * bytes (each input read once, each output written once per launch at its
  * level's shape; a full line sweep, all four colours, counts 3 Ne s + 3 Nc c)

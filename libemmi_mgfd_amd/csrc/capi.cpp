@@ -289,9 +289,10 @@ int emmi_device_sync(void) { return hipDeviceSynchronize() == hipSuccess ? 0 : -
 
 int emmi_set_line_kernel(int mode) { return emmi::set_line_kernel(mode); }
 
-int emmi_line_route(int njobs, const int* cells) {
-  if (njobs < 1 || njobs > emmi::LINE_PACK_MAX || !cells) return -1;
-  return emmi::line_route_now(njobs, cells);
+int emmi_line_route(int esize, int axis, int njobs, const int* cells, const long* lines) {
+  if (njobs < 1 || njobs > emmi::LINE_PACK_MAX || !cells || !lines || axis < 0 || axis > 2 || (esize != 4 && esize != 8))
+    return -1;
+  return emmi::line_route_now(esize, axis, njobs, cells, lines);
 }
 
 int emmi_solver_kernel_rates(emmi_solver_t* h, int reps, double* ms, double* bytes, int n) {

@@ -5,9 +5,9 @@
 // systems are factored once (k_line_factor: FREC values per node, depending
 // on grid, medium and frequency only) and every sweep then computes the
 // lines' right-hand sides and runs a forward/back substitution
-// (k_line_solve_m, or k_line_rhs* and k_line_solve).  A launch takes a pack of
-// up to LINE_PACK_MAX jobs (one per right-hand side) that share the axis and
-// colour; jobs whose lines differ in length take the one-lane kernel.
+// (k_line_solve_m, k_line_long_*, or k_line_rhs* and k_line_solve: line_route).
+// A launch takes a pack of up to LINE_PACK_MAX jobs (one per right-hand side)
+// that share the axis and colour.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -32,8 +32,9 @@ struct LineJob {
   Level<T> L;
   typename cvec<T>::type* u;
   const typename cvec<T>::type* f;
-  typename LineFac<T>::type* fac;  // factor records of this colour, line by line (HalfOrder)
-  typename LineScr<T>::type* scr;  // one-lane records, in 16-byte chunks: [n_a][SREC/V][nlines][V]
+  typename LineFac<T>::type* fac;  // factor records of this colour (HalfOrder, FacLine)
+  typename LineScr<T>::type* scr;  // one-lane records, in 16-byte chunks: [n_a][SREC/V][nlines][V]; or those
+                                   // of k_line_long_* (LongLine)
   int cb, cc;    // colour: parity of pb and pc (1 = odd)
   int nlo, nhi;  // lines of this colour along the low- and high-stride perpendicular axes
 };
@@ -49,8 +50,8 @@ static_assert(sizeof(LinePack<double>) <= 4096 && sizeof(LinePack<float>) <= 409
 
 // number of lines of a colour, split by perpendicular axis (low stride first)
 void line_colour_counts(const int* n, int a, int colour, int* nlo, int* nhi);
-// bytes of one colour's factor records / substitution records for values of
-// esize bytes (4 or 8)
+// bytes of one colour's factor records / of its line records in memory (LineJob::scr)
+// for values of esize bytes (4 or 8)
 size_t line_factor_bytes(const int* n, int a, int colour, size_t esize);
 size_t line_scratch_bytes(const int* n, int a, int colour, size_t esize);
 // fills the colour and counts of a job from its level shape
@@ -61,20 +62,21 @@ inline void line_job_colour(LineJob<T>& J, int a, int colour) {
   line_colour_counts(J.L.n, a, colour, &J.nlo, &J.nhi);
 }
 
-// substitution kernel of later launches: 0 the matrix-core kernel where the
-// line fits its LDS records (or the autotuner's choice where its table has the
+// substitution kernel of later launches: 0 the matrix-core kernel (or the
+// autotuner's choice where its table has the
 // launch's shape), 1 the one-lane kernel, 2, 3, 4 as 0 without the table
 // (they named kernels that the matrix-core one replaced); returns the previous
 // mode or -1
 int set_line_kernel(int mode);
 
-// The substitution that a launch takes: the matrix-core kernel lays out its
-// records, LDS and groups for one length, so every job's lines must have it
-// (and fit the LDS); one_lane: that kernel is asked for.
-enum LineRoute { LINE_ROUTE_ONE_LANE = 0, LINE_ROUTE_MATRIX = 1 };
-LineRoute line_route(int njobs, const int* cells, bool one_lane);
+// The substitution that a launch takes.  The matrix-core kernels lay out their
+// records, LDS and groups for one length, so every job's lines must have it;
+// colours whose factor records lie across the lines (line_across) take the
+// one-lane kernel, as does one_lane.
+enum LineRoute { LINE_ROUTE_ONE_LANE = 0, LINE_ROUTE_MATRIX = 1, LINE_ROUTE_MATRIX_MEM = 2 };
+LineRoute line_route(int esize, int axis, int njobs, const int* cells, const long* lines, bool one_lane);
 // the route under the current mode, without the autotuner's table
-LineRoute line_route_now(int njobs, const int* cells);
+LineRoute line_route_now(int esize, int axis, int njobs, const int* cells, const long* lines);
 
 // Autotuning: a launch shape (value size of the cycle precision, axis, line
 // length, lines per job, jobs per pack) and the substitution choice measured

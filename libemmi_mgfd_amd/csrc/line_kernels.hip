@@ -22,8 +22,9 @@
 //     dE_a(p) = rho_p/d_p + v.(da_{p+1} - da_p) / d_p        (backward)
 // with g_p = sigma_p + v (rho_{p-1}/d_{p-1} - rho_p/d_p) from the residual:
 // k_line_solve_m does all of it in one launch on the matrix cores,
-// k_line_rhs* and k_line_solve (one lane per line half) take the lines too
-// long for its LDS and serve as its check.
+// k_line_long_* in two for lines whose records are in memory; k_line_rhs* and
+// k_line_solve (one lane per line half) take colours of many long lines and
+// packs whose lines differ in length, and serve as the others' check.
 // Lines of one colour (pb%2, pc%2) are not coupled, so a launch sweeps one
 // colour; every kernel computes in FP64 whatever the storage precision.  The
 // substitutions keep a ring of the next D nodes' factor records in registers,
@@ -247,9 +248,44 @@ struct HalfOrder {
   __host__ __device__ int edge(int e) const { return e < m ? e + o : T + N + ob - e - 1; }
 };
 
+// Colours of many long lines keep their records across the lines (chunk k of
+// record r of line l at (r FC + k) nl + l) for the one-lane kernel, which then
+// reads them contiguously; the others line by line for the matrix cores.
+// Where lines no longer fit the LDS by the half-dozen, more than 4096 of them
+// are bound by memory traffic, of which one lane per line half has the least.
+// One launch of a colour, matrix cores (the better of k_line_solve_m and
+// k_line_long_*) against one lane: 160 x 160 lines of 1024 nodes along z, FP64
+// 2165 and 1961 us, FP32 1376 and 1313; along x 2275 and 2058, 1801 and 1514;
+// 224 x 224 lines of 288 nodes along z, FP64 1088 and 908, FP32 668 and 566; of
+// 256 nodes FP32 590 and 525 (160 x 160: 336 and 332).  Along x the records in
+// LDS win for longer lines, as its loads and stores of u run along the lines:
+// 160 x 160 of 512 nodes FP64 893 and 1000, FP32 841 and 759; of 288 nodes FP32
+// 360 and 407.
+__host__ __device__ __forceinline__ bool line_across(int esize, int axis, int N, long nl) {
+  if (nl <= 4096) return false;
+  if (axis == 0) return N > (esize == 4 ? 384 : 512);
+  return N > 256 || (esize == 4 && N > 128 && nl > 8192);
+}
+// the records of one line
+template <typename T, int A>
+struct FacLine {
+  using C = Ch<FacRec<T>>;
+  static constexpr int FC = fchunks<FacRec<T>>();
+  C* base;
+  long rs, cs;   // strides of the records and of their chunks
+  __device__ __forceinline__ FacLine(const LineJob<T>& J, const HalfOrder& O, int line) {
+    const long nl = (long)J.nlo * J.nhi;
+    const bool across = line_across(sizeof(T), A, O.N, nl);
+    cs = across ? nl : 1;
+    rs = FC * cs;
+    base = reinterpret_cast<C*>(J.fac) + (across ? line : (long)line * O.records() * FC);
+  }
+  __device__ __forceinline__ C* at(int r) const { return base + r * rs; }
+};
+
 // inverts D in place and stores the symmetric part with 1/d of the inner edge
 template <typename R>
-__device__ __forceinline__ void store_factor(Ch<R>* r, cxd (&D)[4][4], cxd rd) {
+__device__ __forceinline__ void store_factor(Ch<R>* r, long cs, cxd (&D)[4][4], cxd rd) {
   constexpr int FC = fchunks<R>();
   inv4(D);
   Ch<R> c[FC] = {};
@@ -265,7 +301,7 @@ __device__ __forceinline__ void store_factor(Ch<R>* r, cxd (&D)[4][4], cxd rd) {
   put(c, 20, rd.re);
   put(c, 21, rd.im);
 #pragma unroll
-  for (int k = 0; k < FC; k++) r[k] = c[k];
+  for (int k = 0; k < FC; k++) r[k * cs] = c[k];
 }
 
 // Twisted factorization of each line, meeting at node m = N/2 of the nodes
@@ -288,7 +324,7 @@ __global__ void __launch_bounds__(64) k_line_factor(LinePack<T> P) {
   if (N < 2) return;
   const int M = N - 1, m = N / 2;
   const HalfOrder O(N);
-  Ch<R>* rec = reinterpret_cast<Ch<R>*>(J.fac) + (long)tid * O.records() * FC;
+  const FacLine<T, A> F(J, O, tid);
   const cxd rd0 = cinv(G.d_edge(L, 0)), rdM = cinv(G.d_edge(L, M));
   // boundary nodes and the padding before them
   auto zero_rec = [&](int r, cxd rd) {
@@ -296,7 +332,7 @@ __global__ void __launch_bounds__(64) k_line_factor(LinePack<T> P) {
     put(c, 20, rd.re);
     put(c, 21, rd.im);
 #pragma unroll
-    for (int k = 0; k < FC; k++) rec[r * FC + k] = c[k];
+    for (int k = 0; k < FC; k++) F.at(r)[k * F.cs] = c[k];
   };
   for (int t = 0; t < O.o; t++) zero_rec(t, cxd(0, 0));
   for (int t = 0; t < O.ob; t++) zero_rec(O.T + t, cxd(0, 0));
@@ -312,7 +348,7 @@ __global__ void __launch_bounds__(64) k_line_factor(LinePack<T> P) {
       G.lcoef(L, p - 1, l);
       sub_bwb(Dm, Wt, l, rd_prev, G.v);
     }
-    store_factor(rec + O.node(p) * FC, Dm, rd);
+    store_factor(F.at(O.node(p)), F.cs, Dm, rd);
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
@@ -326,7 +362,7 @@ __global__ void __launch_bounds__(64) k_line_factor(LinePack<T> P) {
       G.lcoef(L, p, l);
       sub_bwb(Dm, Wb, l, rdp, G.v);
     }
-    store_factor(rec + O.node(p) * FC, Dm, rdm);
+    store_factor(F.at(O.node(p)), F.cs, Dm, rdm);
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
@@ -343,7 +379,7 @@ __global__ void __launch_bounds__(64) k_line_factor(LinePack<T> P) {
       G.lcoef(L, m, l);
       sub_bwb(Dm, Wb, l, rdp, G.v);
     }
-    store_factor(rec + O.node(m) * FC, Dm, cxd(0, 0));
+    store_factor(F.at(O.node(m)), F.cs, Dm, cxd(0, 0));
   }
 }
 
@@ -854,9 +890,10 @@ __global__ void __launch_bounds__(128) k_line_solve(LinePack<T> P) {
   if (live) G.init(L, pb, pc);
   const long stride = (long)J.nlo * J.nhi;
   const HalfOrder O(N);
-  const Ch<RF>* __restrict__ fac = reinterpret_cast<const Ch<RF>*>(J.fac) + (long)line * O.records() * FC;
-  auto fnode = [&](int p) { return fac + O.node(p) * FC; };            // the node's inverse, 1/d of its inner edge
-  auto fedge = [&](int e) { return fac[O.edge(e) * FC + CD]; };        // 1/d of an edge
+  const FacLine<T, A> F(J, O, line);
+  const long fs = F.cs;
+  auto fnode = [&](int p) -> const Ch<RF>* { return F.at(O.node(p)); };   // the node's inverse, 1/d of its inner edge
+  auto fedge = [&](int e) { return F.at(O.edge(e))[CD * fs]; };           // 1/d of an edge
   Ch<RS>* __restrict__ scr = reinterpret_cast<Ch<RS>*>(J.scr) + line;
   E* __restrict__ u = J.u;
   const double* __restrict__ iw = L.IW[A];
@@ -879,7 +916,7 @@ __global__ void __launch_bounds__(128) k_line_solve(LinePack<T> P) {
 #pragma unroll
     for (int d = 0; d < D; d++) {
       const int pn = max(min(1 + d, last), 1);
-      load_node(rf[d], fnode(pn), 1);
+      load_node(rf[d], fnode(pn), fs);
       load_node(rs[d], scr + pn * sstep, stride);
       riw[d] = iw[pn - 1];
     }
@@ -894,7 +931,7 @@ __global__ void __launch_bounds__(128) k_line_solve(LinePack<T> P) {
       const double iWe = (double)riw[d];
       {
         const int pn = min(p + D, last), dn = (d + D) % R;
-        load_node(rf[dn], fnode(pn), 1);
+        load_node(rf[dn], fnode(pn), fs);
         load_node(rs[dn], scr + pn * sstep, stride);
         riw[dn] = iw[pn - 1];
       }
@@ -939,7 +976,7 @@ __global__ void __launch_bounds__(128) k_line_solve(LinePack<T> P) {
 #pragma unroll
     for (int d = 0; d < D; d++) {
       const int pn = min(max(M - d, last), M);
-      load_node(rf[d], fnode(pn), 1);
+      load_node(rf[d], fnode(pn), fs);
       load_node(rs[d], scr + pn * sstep, stride);
       rdn[d] = fedge(pn);
       rqn[d] = scr[(pn - 1) * sstep + CQ * stride];
@@ -954,7 +991,7 @@ __global__ void __launch_bounds__(128) k_line_solve(LinePack<T> P) {
       const double iWe = (double)riw[d];
       {
         const int pn = max(p - D, last), dn = (d + D) % R;
-        load_node(rf[dn], fnode(pn), 1);
+        load_node(rf[dn], fnode(pn), fs);
         load_node(rs[dn], scr + pn * sstep, stride);
         rdn[dn] = fedge(pn);
         rqn[dn] = scr[(pn - 1) * sstep + CQ * stride];
@@ -1008,7 +1045,7 @@ __global__ void __launch_bounds__(128) k_line_solve(LinePack<T> P) {
   {
     Ch<RF> cf[FC];
           Ch<RS> cr[SC];
-    load_node(cf, fnode(m), 1);
+    load_node(cf, fnode(m), fs);
     load_node(cr, scr + m * sstep, stride);
     const Ch<RF> cdm = fedge(m - 1), cdp = fedge(m);
     const Ch<RS> cqm = scr[(m - 1) * sstep + CQ * stride];
@@ -1038,7 +1075,7 @@ __global__ void __launch_bounds__(128) k_line_solve(LinePack<T> P) {
 #pragma unroll
     for (int d = 0; d < D; d++) {
       const int pn = max(last - d, 1);
-      load_node(rf[d], fnode(pn), 1);
+      load_node(rf[d], fnode(pn), fs);
       load_node(rs[d], scr + pn * sstep, stride);
       riw[d] = iw[pn];
       if constexpr (A != 0) {
@@ -1056,7 +1093,7 @@ __global__ void __launch_bounds__(128) k_line_solve(LinePack<T> P) {
       const double iWe = (double)riw[d];
       {
         const int pn = max(p - D, 1), dn = (d + D) % R;
-        load_node(rf[dn], fnode(pn), 1);
+        load_node(rf[dn], fnode(pn), fs);
         load_node(rs[dn], scr + pn * sstep, stride);
         riw[dn] = iw[pn];
         if constexpr (A != 0) {
@@ -1111,7 +1148,7 @@ __global__ void __launch_bounds__(128) k_line_solve(LinePack<T> P) {
 #pragma unroll
     for (int d = 0; d < D; d++) {
       const int pn = min(last + d, M);
-      load_node(rf[d], fnode(pn), 1);
+      load_node(rf[d], fnode(pn), fs);
       rdn[d] = fedge(pn);
       load_node(rs[d], scr + pn * sstep, stride);
       riw[d] = iw[pn - 1];
@@ -1132,7 +1169,7 @@ __global__ void __launch_bounds__(128) k_line_solve(LinePack<T> P) {
       const double iWe = (double)riw[d];
       {
         const int pn = min(p + D, M), dn = (d + D) % R;
-        load_node(rf[dn], fnode(pn), 1);
+        load_node(rf[dn], fnode(pn), fs);
         rdn[dn] = fedge(pn);
         load_node(rs[dn], scr + pn * sstep, stride);
         riw[dn] = iw[pn - 1];
@@ -1227,6 +1264,8 @@ constexpr int M_LDS = 160 * 1024;          // LDS of a CU
 __host__ __device__ __forceinline__ int line_m_bytes(int n) { return 160 * HalfOrder(n).T; }
 static int line_m_lpb(int n) { return 8 * line_m_bytes(n) <= M_LDS ? 8 : 2; }
 static bool line_m_fits(int n) { return 2 * line_m_bytes(n) <= M_LDS; }
+// lines whose records are in memory: lines of a block, nodes in flight per half
+constexpr int LONG_LPB = 8, LONG_RING = 8;
 
 // (re, im) -> (-im, re) across the columns of a node vector; sg flips the
 // sign of the even columns
@@ -1259,8 +1298,11 @@ __device__ __forceinline__ double rec_val(double x) {
 __device__ __forceinline__ void node_end() { __builtin_amdgcn_sched_barrier(0); }
 
 // One lane of the substitution of two lines by a wave (see above).  ST: lines
-// side by side in the block's LDS (the stride between a line's slots).
-template <typename T, int A, int D, int ST>
+// side by side in the block's records (the stride between a line's slots).
+// MEM: these records are in memory, in the cycle's precision, and the back pass
+// adds to u itself; the ring holds a node's part of them beside its factor
+// records, as a read of memory takes the time of many nodes.
+template <typename T, int A, int D, int ST, bool MEM>
 struct HalfLane {
   static constexpr int XS = 8 * ST, QS = 2 * ST;   // doubles between the slots of a line
   static constexpr int RB = fchunks<double>() * 16;   // bytes of a factor record
@@ -1276,6 +1318,11 @@ struct HalfLane {
   int qx;                 // from the component jr to the other one
   double2 rw[D], rr[D], wm;
   double ri[D];
+  // MEM: sigma (then z), rho and u (node edge, inner edge) of the node
+  ScrRec<T> rs[D], ra_[D], rb_[D], *xr, *qr, *xmr;
+  T un[D], ue[D], *u0, *ue0, *um;
+  long su, sue;
+  int t1;                 // first node of the half that is not padding (the boundary node)
 
   __device__ __forceinline__ HalfLane() {
     const int lane = threadIdx.x & 63;
@@ -1308,15 +1355,46 @@ struct HalfLane {
     e0 = side ? O.N + O.ob - 1 : -O.o;
     de = side ? -1 : 1;
     last = O.N - 1;
-    xq = reinterpret_cast<double*>(x0) + (side * (TT - 1) - 1) * XS + 2 * row + jr;
-    xm = reinterpret_cast<double*>(x0) + (2 * TT - 2) * XS + 2 * row + jr;
-    qa = reinterpret_cast<double*>(q0) + side * TT * QS + jr;
+    if constexpr (!MEM) {
+      xq = reinterpret_cast<double*>(x0) + (side * (TT - 1) - 1) * XS + 2 * row + jr;
+      xm = reinterpret_cast<double*>(x0) + (2 * TT - 2) * XS + 2 * row + jr;
+      qa = reinterpret_cast<double*>(q0) + side * TT * QS + jr;
+    } else {
+      xq = xm = qa = nullptr;   // init_mem
+    }
     qx = 1 - 2 * jr;
+  }
+  // MEM: the records of the line and the u of node 0 of the half
+  __device__ __forceinline__ void init_mem(const Level<T>& L, const HalfOrder& O, int pb, int pc, ScrRec<T>* x0,
+                                           ScrRec<T>* q0, typename cvec<T>::type* u) {
+    const LineGeo<T, A> G(L, pb, pc);
+    xr = x0 + (side * (TT - 1) - 1) * XS + 2 * row + jr;
+    xmr = x0 + (2 * TT - 2) * XS + 2 * row + jr;
+    qr = q0 + side * TT * QS + jr;
+    t1 = side ? O.ob : O.o;
+    su = (side ? -2 : 2) * G.sa;
+    T* uc = reinterpret_cast<T*>(u) + jr;
+    u0 = uc + 2 * (row == 0 ? G.ob0 : row == 1 ? G.ob1 : row == 2 ? G.oc0 : G.oc1);
+    um = u0 + 2 * O.m * G.sa;
+    u0 += side ? 2L * (O.N + O.ob) * G.sa : -2L * O.o * G.sa;
+    ue0 = uc + 2 * (G.oa + (long)e0 * G.sa);
+  }
+  // (node 0 has no vector: the value before it is not used)
+  __device__ __forceinline__ void load_rec(int d, int t) {
+    rs[d] = xr[(long)t * XS];
+    ra_[d] = qr[(long)t * QS];
+    rb_[d] = qr[(long)t * QS + qx];
+  }
+  __device__ __forceinline__ void load_u(int d, int t) {   // the padding reads the boundary's
+    const long tc = max(t, t1);
+    un[d] = u0[tc * su];
+    ue[d] = ue0[tc * su];
   }
   __device__ __forceinline__ void load(int d, const char* base, int t) {   // base: record t - d
     rw[d] = *reinterpret_cast<const double2*>(base + d * RB + fw);
     rr[d] = *reinterpret_cast<const double2*>(base + d * RB + fr);
     ri[d] = iwa[min((unsigned)(e0 + de * t), (unsigned)last)];
+    if constexpr (MEM) load_rec(d, t);
   }
   __device__ __forceinline__ void first_loads() {
 #pragma unroll
@@ -1330,6 +1408,7 @@ struct HalfLane {
   }
   // both passes, on the records that first_loads() has under way
   __device__ __forceinline__ void run() {
+    int t0 = 0;   // first node of the group
     // Software pipeline: a node's step runs its chain on operands prepared in
     // the step before, and prepares the next node's (coupling -B, right-hand
     // side g) and reads the LDS of the one after.
@@ -1351,11 +1430,17 @@ struct HalfLane {
     };
     auto fnext = [&](int d) {   // operands of the node after d (of group slot d)
       couple(d);
+      if constexpr (MEM) {
+        sig = rs[(d + 1) % D];
+        ra = ra_[(d + 1) % D];
+        rb = rb_[(d + 1) % D];
+      }
       const double q1 = qval(ra, rb, rr[(d + 1) % D]);
       g = fma(vs, q - q1, sig);
       q = q1;
     };
     auto fread = [&](int d) {   // LDS of node d
+      if constexpr (MEM) return;
       sig = xq[d * XS];
       ra = qa[d * QS];
       rb = qa[d * QS + qx];
@@ -1366,16 +1451,20 @@ struct HalfLane {
       z = mma(rw[d].y, mswap(y, sg), z);
       fnext(d);
       fread(d + 2);
-      xq[d * XS] = zrec(z);
+      if constexpr (MEM) {
+        rs[d] = (ScrRec<T>)z;
+        xr[(long)(t0 + d) * XS] = rs[d];
+      } else {
+        xq[d * XS] = zrec(z);
+      }
     };
     // the first node of a half (boundary or padding) only hands its inner
     // edge on
-    q = qval(qa[0], qa[qx], rr[0]);
+    q = MEM ? qval(ra_[0], rb_[0], rr[0]) : qval(qa[0], qa[qx], rr[0]);
     fread(1);
     fnext(0);
     fread(2);
     node_end();
-    int t0 = 0;
     if (TT > D) {
       load(0, fb + D * RB, D);
       node_end();
@@ -1398,6 +1487,10 @@ struct HalfLane {
       }
       // the last group's records stay for the back pass
       xq += D * XS; qa += D * QS; fb += D * RB;
+      if constexpr (MEM) {
+#pragma unroll
+        for (int d = 0; d < D; d++) load_u(d, t0 + d);
+      }
       fstep(0);
       node_end();
     }
@@ -1410,43 +1503,48 @@ struct HalfLane {
     // meeting node: x_m = S_m^-1 (g_m - B_m z_{m-1} - B_{m+1} z_{m+1})
     double x;
     {
-      const double ql = qval(qa[(D - 1) * QS], qa[(D - 1) * QS + qx], rr[D - 1]);
+      const double ql = MEM ? qval(ra_[D - 1], rb_[D - 1], rr[D - 1])
+                            : qval(qa[(D - 1) * QS], qa[(D - 1) * QS + qx], rr[D - 1]);
       double y = bsub(z, vs * ql);
-      y = *xm + (y + mpeer(y));
+      y = (MEM ? (double)*xmr : *xm) + (y + mpeer(y));
       x = mma(wm.x, y, 0.0);
       x = mma(wm.y, mswap(y, sg), x);
-      *xm = x;
+      if constexpr (!MEM) *xm = x;
+      else if (side == 0 && j < 2) *um = (T)((double)*um + x);
     }
     sig = zrec(z);
     // the along-line edge of a node follows one step later, off the chain
     double dx = 0.0, ere = 0.0, eim = 0.0, eq = 0.0;
-    auto edge = [&](double* to) {   // q + v.dx / d
-      const double sv = mma(vs, dx, 0.0);
-      *to = fma(eim, mswap(sv, sg), fma(ere, sv, eq));
+    auto edge = [&](double* to, int t, int k) {   // q + v.dx / d; k: the node's slot of the ring
+      const double sv = mma(vs, dx, 0.0), de_ = fma(eim, mswap(sv, sg), fma(ere, sv, eq));
+      if constexpr (!MEM) *to = de_;
+      else if (t >= t1 && t < TT && row == 0 && j < 2) ue0[t * su] = (T)((double)ue[k] + de_);
     };
     auto bedge = [&](int d) {   // operands of that edge
       ere = rr[d].x;
       eim = rr[d].y;
-      eq = qval(ra, rb, rr[d]);
+      eq = MEM ? qval(ra_[d], rb_[d], rr[d]) : qval(ra, rb, rr[d]);
     };
     // (from the slot before the group, as LDS offsets are not negative)
     double *xb = xq - XS, *qb = qa - QS;
     auto bread = [&](int d) {   // rho of node d's inner edge
+      if constexpr (MEM) return;
       ra = qb[(d + 1) * QS];
       rb = qb[(d + 1) * QS + qx];
     };
     // to: where the pending edge goes
     auto bstep = [&](int d, double* to) {
       const double y = bsub(x, 0.0);
-      double xp = mma(rw[d].x, y, sig);
+      double xp = mma(rw[d].x, y, MEM ? rs[d] : sig);
       xp = mma(rw[d].y, mswap(y, sg), xp);
-      sig = xb[d * XS];
-      edge(to);
+      if constexpr (!MEM) sig = xb[d * XS];
+      edge(to, t0 + d + 1, (d + 1) % D);
       bedge(d);
       bread(d - 1);
       couple((d + D - 1) % D);
       dx = x - xp;
-      xb[(d + 1) * XS] = xp;
+      if constexpr (!MEM) xb[(d + 1) * XS] = xp;
+      else if (t0 + d > t1 && j < 2) u0[(t0 + d) * su] = (T)((double)un[d] + xp);
       x = xp;
     };
     couple(D - 1);
@@ -1461,8 +1559,13 @@ struct HalfLane {
         node_end();
         // a slot is reloaded one step after its node: that node's edge is
         // still pending until then
-        if (d == D - 1) load(0, fb, t0);
-        else load(d + 1, fb - D * RB, t0 - D + d + 1);
+        if (d == D - 1) {
+          load(0, fb, t0);
+          if constexpr (MEM) load_u(0, t0);
+        } else {
+          load(d + 1, fb - D * RB, t0 - D + d + 1);
+          if constexpr (MEM) load_u(d + 1, t0 - D + d + 1);
+        }
         node_end();
       }
       qe = qb + QS;
@@ -1472,14 +1575,17 @@ struct HalfLane {
     for (int d = D - 1; d >= 1; d--) {
       bstep(d, d == D - 1 ? qe : qb + (d + 2) * QS);
       node_end();
-      if (d == D - 1) load(0, fb, 0);
+      if (d == D - 1) {
+        load(0, fb, 0);
+        if constexpr (MEM) load_u(0, 0);
+      }
       node_end();
     }
-    edge(qb + 2 * QS);
+    edge(qb + 2 * QS, 1, 1);
     // the first node's correction is zero: its inner edge alone
     bedge(0);
     dx = x;
-    edge(qb + QS);
+    edge(qb + QS, 0, 0);
   }
 };
 
@@ -1516,7 +1622,7 @@ __global__ void __launch_bounds__(32 * LPB, 2) k_line_solve_m(LinePack<T> P) {
   // ---------------- the lane of the substitution ----------------
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const bool live = 2 * wave < nle;   // uniform over the wave
-  HalfLane<T, A, D, A == 0 ? 1 : LPB> H;
+  HalfLane<T, A, D, A == 0 ? 1 : LPB, false> H;
   {
     // a wave without a second line runs its first line twice
     const int l = live ? min(2 * wave + H.second(), nle - 1) : 0, l2 = live ? 2 * wave : 0;
@@ -1629,6 +1735,108 @@ __global__ void __launch_bounds__(32 * LPB, 2) k_line_solve_m(LinePack<T> P) {
   }
 }
 
+// Long lines: the same substitution with the line records in memory (J.scr),
+// in two launches: residual records; substitution and u += corrections.  The
+// records of x lines lie line after line; those of y and z lines lie side by
+// side, eight lines together.
+//
+// What bounds it: with many lines the traffic (both passes read the factor
+// records, 352 bytes a node; the line records are written twice and read twice,
+// 288 bytes in FP64; u), for few the chain.  One launch of a colour, four lanes
+// per line half -> here: 64 x 64 lines of 1100 nodes, FP64, along z 950 -> 518
+// us, along x 1199 -> 518; FP32 752 -> 315 and 1028 -> 391; 128 x 128 lines 1289
+// -> 1290 and 1483 -> 1312, FP32 936 -> 821 and 1287 -> 1024; a single line 590
+// -> 172.  All in one launch, with the records in FP64 and the update of u as a
+// phase of its own, took 621, 534, 527 and 482 us (64 x 64); three waves per
+// SIMD and four nodes in flight measured level.
+template <typename T, int A>
+struct LongLine {
+  using R = ScrRec<T>;
+  static constexpr int ST = A == 0 ? 1 : LONG_LPB;   // stride between a line's slots
+  R *Q, *X;   // edges (2 values) and node vectors (8 values), as in k_line_solve_m
+  __device__ __forceinline__ LongLine(const LineJob<T>& J, const HalfOrder& O, int line) {
+    const long per = 20L * O.T;   // values of a line
+    if constexpr (A == 0) {
+      Q = J.scr + line * per;
+      X = Q + 4 * O.T;
+    } else {
+      const int l = line % LONG_LPB;
+      R* base = J.scr + (line - l) * per;
+      Q = base + 2 * l;
+      X = base + 4 * O.T * LONG_LPB + 8 * l;
+    }
+  }
+  __device__ __forceinline__ typename cvec<R>::type* edge(int t) const {
+    return reinterpret_cast<typename cvec<R>::type*>(Q + 2L * ST * t);
+  }
+  // vector of record r (r = 0 and T have none)
+  __device__ __forceinline__ typename cvec<R>::type* vec(const HalfOrder& O, int r) const {
+    return reinterpret_cast<typename cvec<R>::type*>(X + 8L * ST * (r - 1 - (r > O.T ? 1 : 0)));
+  }
+};
+
+// residual records: a thread per run of nodes of a line, lines fastest
+// (marching) along y and z, nodes fastest (runs of one) along x
+template <typename T, int A>
+__global__ void __launch_bounds__(256) k_line_long_rhs(LinePack<T> P, int run) {
+  constexpr int SC = schunks<double>();
+  const LineJob<T>& J = P.job[blockIdx.y];
+  const int N = J.L.n[A];
+  const long nl = (long)J.nlo * J.nhi, nr = (N + run - 1) / run;
+  const long t = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  if (N < 2 || t >= nl * nr) return;
+  const int line = (int)(A == 0 ? t / nr : t % nl), p0 = (int)(A == 0 ? t % nr : t / nl) * run, p1 = min(N, p0 + run);
+  int pb, pc;
+  line_of<T, A>(J, line, pb, pc);
+  const HalfOrder O(N);
+  const LongLine<T, A> R(J, O, line);
+  auto put_rec = [&](int p, const Ch<double>(&c)[SC]) {
+    st<T>(R.edge(O.edge(p)), 0, cxd(c[4].v[0], c[4].v[1]));
+    if (p >= 1) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) st<T>(R.vec(O, O.node(p)), i, cxd(c[i].v[0], c[i].v[1]));
+    }
+  };
+  if constexpr (A == 0) {
+    Ch<double> c[SC] = {};
+    node_rhs_rec<T, A>(J, pb, pc, p0, c);
+    put_rec(p0, c);
+  } else {
+    line_rhs_march<T, A, double>(J, pb, pc, p0, p1, put_rec);
+  }
+  if (p0 == 0) {   // padding and boundary records
+    const cxd zz(0.0, 0.0);
+    for (int q = 0; q <= O.o; q++) {
+      if (q < O.o) st<T>(R.edge(q), 0, zz);
+      if (q < O.ob) st<T>(R.edge(O.T + q), 0, zz);
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        if (q >= 1) st<T>(R.vec(O, q), i, zz);
+        if (q >= 1 && q <= O.ob) st<T>(R.vec(O, O.T + q), i, zz);
+      }
+    }
+  }
+}
+
+template <typename T, int A>
+__global__ void __launch_bounds__(32 * LONG_LPB, 2) k_line_long_solve(LinePack<T> P) {
+  const LineJob<T>& J = P.job[blockIdx.y];
+  const int N = J.L.n[A], nl = J.nlo * J.nhi;
+  const int l2 = (int)xcd_block(blockIdx.x, gridDim.x) * LONG_LPB + 2 * __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  if (N < 2 || l2 >= nl) return;   // uniform over the wave
+  const HalfOrder O(N);
+  HalfLane<T, A, LONG_RING, LongLine<T, A>::ST, true> H;
+  // a wave without a second line runs its first line twice
+  const int line = min(l2 + H.second(), nl - 1);
+  int pb, pc;
+  line_of<T, A>(J, line, pb, pc);
+  const LongLine<T, A> R(J, O, line);
+  H.init(J.L, O, pb, pc, J.fac, l2, line - l2, false, nullptr, nullptr);
+  H.init_mem(J.L, O, pb, pc, R.X, R.Q, J.u);
+  H.first_loads();
+  H.run();
+}
+
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
@@ -1640,16 +1848,32 @@ void line_colour_counts(const int* n, int a, int colour, int* nlo, int* nhi) {
   if (b < c) { *nlo = nbv; *nhi = ncv; } else { *nlo = ncv; *nhi = nbv; }
 }
 
-LineRoute line_route(int njobs, const int* cells, bool one_lane) {
+// Lines of more than 256 nodes have their records in LDS two lines at a time,
+// at most six lines (three waves) a CU: with many lines their
+// residual and update phases no longer fill the chip.  Per launch of a colour in
+// LDS and in memory, along z: 64 x 64 lines (1024 a colour) of 512 nodes FP64
+// 165 and 209 us, FP32 127 and 132; of 1024 nodes 589 and 439, 512 and 275;
+// 96 x 96 of 288 nodes 232 and 278, 180 and 166; of 512 nodes 513 and 501, 423
+// and 312; 128 x 128 of 288 nodes 378 and 363, 300 and 216.  Along x, where the
+// LDS form loads and stores u along the lines, 128 x 128 of 512 nodes 530 and
+// 649, 494 and 475; 96 x 96 of 1024 nodes 1146 and 1019, 1131 and 829.
+LineRoute line_route(int esize, int axis, int njobs, const int* cells, const long* lines, bool one_lane) {
   if (one_lane || njobs < 1) return LINE_ROUTE_ONE_LANE;
-  for (int j = 1; j < njobs; j++)
-    if (cells[j] != cells[0]) return LINE_ROUTE_ONE_LANE;
-  return line_m_fits(cells[0]) ? LINE_ROUTE_MATRIX : LINE_ROUTE_ONE_LANE;
+  const int N = cells[0];
+  double nodes = 0;
+  for (int j = 0; j < njobs; j++) {
+    if (cells[j] != N || line_across(esize, axis, N, lines[j])) return LINE_ROUTE_ONE_LANE;
+    nodes += (double)N * (double)lines[j];
+  }
+  const bool many = N > 256 && nodes > 0.9e6 && (axis != 0 || N > 512);
+  return line_m_fits(N) && !many ? LINE_ROUTE_MATRIX : LINE_ROUTE_MATRIX_MEM;
 }
 
 static int g_line_kernel = 0;
 
-LineRoute line_route_now(int njobs, const int* cells) { return line_route(njobs, cells, g_line_kernel == 1); }
+LineRoute line_route_now(int esize, int axis, int njobs, const int* cells, const long* lines) {
+  return line_route(esize, axis, njobs, cells, lines, g_line_kernel == 1);
+}
 
 int set_line_kernel(int mode) {
   if (mode < 0 || mode > 4) return -1;
@@ -1729,7 +1953,10 @@ size_t line_factor_bytes(const int* n, int a, int colour, size_t esize) {
 size_t line_scratch_bytes(const int* n, int a, int colour, size_t esize) {
   int nlo, nhi;
   line_colour_counts(n, a, colour, &nlo, &nhi);
-  return (size_t)nlo * nhi * (size_t)n[a] * chunks_of(SREC, esize) * 16;
+  const size_t one_lane = (size_t)nlo * nhi * (size_t)n[a] * chunks_of(SREC, esize) * 16;
+  if (n[a] <= 256) return one_lane;   // always in the LDS
+  const size_t blocks = ((size_t)nlo * nhi + LONG_LPB - 1) / LONG_LPB;
+  return std::max(one_lane, blocks * LONG_LPB * 20 * HalfOrder(n[a]).T * esize);
 }
 
 // A launch; when timing is on, its events are recorded by the dispatch itself
@@ -1770,7 +1997,15 @@ static void launch_lds(K kernel, dim3 g, dim3 b, size_t lds, hipStream_t s, int 
 // the matrix-core substitution: lines per block by what the LDS holds, the
 // ring by the length of a half
 template <typename T, int A>
-static void launch_line_m_axis(const LinePack<T>& P, int maxl, int maxna, hipStream_t s, Bytes by) {
+static void launch_line_m_axis(const LinePack<T>& P, bool mem, int maxl, int maxna, hipStream_t s, Bytes by) {
+  if (mem) {
+    const int run = A == 0 || maxl < 64 ? 1 : 8;
+    auto blocks = [&](long n, int per) { return dim3((unsigned)((n + per - 1) / per), P.njobs); };
+    launch_timed(k_line_long_rhs<T, A>, blocks((long)maxl * ((maxna + run - 1) / run), 256), dim3(256), s, timing::LINE_RHS,
+                 Bytes{0.0, 0.0}, P, run);
+    launch_timed(k_line_long_solve<T, A>, blocks(maxl, LONG_LPB), dim3(32 * LONG_LPB), s, timing::LINE, by, P);
+    return;
+  }
   const int lpb = line_m_lpb(maxna), D = line_ring(maxna);
   const dim3 g((unsigned)((maxl + lpb - 1) / lpb), P.njobs), b(32 * lpb);
   const size_t lds = (size_t)lpb * line_m_bytes(maxna);
@@ -1803,10 +2038,10 @@ static void launch_line_m_axis(const LinePack<T>& P, int maxl, int maxna, hipStr
   }
 }
 template <typename T>
-static void launch_line_m(const LinePack<T>& P, int axis, int maxl, int maxna, hipStream_t s, Bytes by) {
-  if (axis == 0) launch_line_m_axis<T, 0>(P, maxl, maxna, s, by);
-  else if (axis == 1) launch_line_m_axis<T, 1>(P, maxl, maxna, s, by);
-  else launch_line_m_axis<T, 2>(P, maxl, maxna, s, by);
+static void launch_line_m(const LinePack<T>& P, int axis, bool mem, int maxl, int maxna, hipStream_t s, Bytes by) {
+  if (axis == 0) launch_line_m_axis<T, 0>(P, mem, maxl, maxna, s, by);
+  else if (axis == 1) launch_line_m_axis<T, 1>(P, mem, maxl, maxna, s, by);
+  else launch_line_m_axis<T, 2>(P, mem, maxl, maxna, s, by);
 }
 
 template <typename T>
@@ -1834,8 +2069,10 @@ static void launch_pack(const LinePack<T>& P, int axis, bool factor, hipStream_t
   }
   if (maxl == 0 || P.njobs == 0) return;
   int maxna = 0, cells[LINE_PACK_MAX];
+  long lines[LINE_PACK_MAX];
   for (int j = 0; j < P.njobs; j++) {
     cells[j] = P.job[j].L.n[axis];
+    lines[j] = (long)P.job[j].nlo * P.job[j].nhi;
     maxna = std::max(maxna, cells[j]);
   }
   if (factor) {
@@ -1846,12 +2083,12 @@ static void launch_pack(const LinePack<T>& P, int axis, bool factor, hipStream_t
     else hipLaunchKernelGGL((k_line_factor<T, 2>), g, b, 0, s, P);
     return;
   }
-  // the matrix-core substitution takes lines of one length that fit its LDS
-  // records; longer ones (and forced launches) take the one-lane kernel
   if (choice == LINE_RULE && g_line_kernel == 0) choice = tuned_choice(line_shape(P, axis));
   const bool one_lane = choice == LINE_ONE_LANE || (choice == LINE_RULE && g_line_kernel == 1);
-  if (line_route(P.njobs, cells, one_lane) == LINE_ROUTE_MATRIX) {
-    launch_line_m<T>(P, axis, maxl, maxna, s, Bytes{comp, rhs_bytes + solve_bytes - 2.0 * rec_bytes});
+  const LineRoute route = line_route(sizeof(T), axis, P.njobs, cells, lines, one_lane);
+  if (route != LINE_ROUTE_ONE_LANE) {
+    const bool mem = route == LINE_ROUTE_MATRIX_MEM;
+    launch_line_m<T>(P, axis, mem, maxl, maxna, s, Bytes{comp, rhs_bytes + solve_bytes - (mem ? 0.0 : 2.0 * rec_bytes)});
     return;
   }
   if (axis == 0) {

@@ -132,7 +132,7 @@ def lib() -> C.CDLL:
         L.emmi_set_line_kernel.restype = C.c_int
         L.emmi_set_line_kernel.argtypes = [C.c_int]
         L.emmi_line_route.restype = C.c_int
-        L.emmi_line_route.argtypes = [C.c_int, C.POINTER(C.c_int)]
+        L.emmi_line_route.argtypes = [C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_long)]
         L.emmi_timing_enable.argtypes = [C.c_int]
         L.emmi_solver_kernel_rates.restype = C.c_int
         L.emmi_solver_kernel_rates.argtypes = [C.c_void_p, C.c_int, C.POINTER(C.c_double), C.POINTER(C.c_double),
