@@ -338,6 +338,10 @@ const char *emmi_path_last_error(void);
 int emmi_x0_kpad(int cin);
 int emmi_x0_conv_fwd(const void *x, int Z, int Y, int X, int Cin, const void *w, int Cout, const float *bias, int epi,
                      float slope, const void *act, void *out_bf16, float *out_f32, int cout_store, void *stream);
+/* the kernel such a convolution takes: the rows (8 or 4) of a block that marches
+ * through LDS, 0 the one that gathers from memory.  Host only.  -1: a size out
+ * of range */
+int emmi_x0_conv_route(int Z, int Y, int X, int Cin, int Cout);
 /* weight gradient [Cout][27*Cin] (and bias gradient, db may be NULL) of a
  * convolution with input x [V][Cin] and output gradient dy [V][Cout];
  * part: scratch of ceil(Z/zslab)*27*Cin*Cout floats; Cin and Cout multiples

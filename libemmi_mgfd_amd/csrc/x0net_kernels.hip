@@ -106,8 +106,10 @@ __device__ __forceinline__ void conv_epilogue(const f32x4 (&acc)[MT][NT], int x0
 
 // One wave: 16*MT consecutive voxels along x of row (z, y) and all 16*NT
 // output channels.  Block: 4 waves on rows y0..y0+3.
+// (Four waves per SIMD for one tile into 48 to 80 channels: at three, 33^3 needs
+// a second, nearly empty round of blocks, 48 -> 48 channels 46 -> 54 us.)
 template <int MT, int NT>
-__global__ void __launch_bounds__(256) k_conv_fwd(const bf16* __restrict__ x, int Z, int Y, int X, int Cin,
+__global__ void __launch_bounds__(256, MT == 1 && NT >= 3 && NT <= 5 ? 4 : 1) k_conv_fwd(const bf16* __restrict__ x, int Z, int Y, int X, int Cin,
                                                   const bf16* __restrict__ w, int Kpad,
                                                   const float* __restrict__ bias, int epi, float slope,
                                                   const bf16* __restrict__ act, bf16* __restrict__ out_bf,
@@ -125,7 +127,7 @@ __global__ void __launch_bounds__(256) k_conv_fwd(const bf16* __restrict__ x, in
   const int K27 = 27 * Cin;
   const int row = lane & 15, kq = (lane >> 4) * 8;
   // the next G steps' operands are in flight while a step is multiplied
-  constexpr int G = MT + NT <= 4 ? 6 : MT + NT <= 6 ? 4 : 3;
+  constexpr int G = MT + NT <= 4 ? 6 : MT + NT <= 6 && NT != 5 ? 4 : 3;
   bf16x8 a[G][MT], b[G][NT];
   auto fetch = [&](int q, int k0) {
     if (k0 >= Kpad) return;   // uniform
@@ -838,25 +840,67 @@ void conv_fwd_mt(const bf16* x, int Z, int Y, int X, int Cin, const bf16* w, int
   }
 }
 
+constexpr size_t CONV_LDS = 160 * 1024;   // of a CU
+
 // LDS bytes of k_conv_fwd_lds for rows TY
 size_t conv_lds(int TY, int Cin, int Kpad) {
   return 3 * (size_t)((TY + 2) * 34) * (2 * Cin + 16) + (3 * (Kpad / 8) * sizeof(int) + 15) / 16 * 16;
 }
 
+// planes that a block of k_conv_fwd_lds marches through: one where all tiles of
+// all planes fill no more than the 256 CUs (two would double the serial time of
+// a launch that leaves CUs idle: 8 x 9 x 33, 16 -> 16 channels 8.8 and 5.9 us),
+// else enough for about two blocks a CU
+int conv_planes(int Z, int Y, int X, int TY) {
+  const long tiles = (long)((X + 31) / 32) * ((Y + TY - 1) / TY), n = Z * tiles;
+  return n <= 256 ? 1 : (int)std::max(2L, n / 512);
+}
+
+// The rows that k_conv_fwd_lds takes, eight where the planes of the tile fit the
+// LDS beside the table, four for more channels; 0: k_conv_fwd is the faster one.
+// With the weights in LDS, or 16 outputs, the march wins (1.0x for a single 8 x 32
+// plane of 16 -> 32 channels to 2.8x; the least of all sizes measured is 0.93,
+// 32 -> 16 on 1000 planes of 9 x 33).  With weights from memory it is bound by their loads:
+//  - where tiles leave CUs idle both are chains of latencies, and the march is
+//    ahead with four rows and up to 48 outputs (128 x 128 plane, 80 -> 32
+//    channels 32 and 24 us, 48 -> 64 28 and 33);
+//  - where k_conv_fwd's waves hold one tile of 16 voxels (X no multiple of 32),
+//    the march is about 1.9 (80 channels 1.8, 64, 96 and 112 2.1) times as fast
+//    per voxel of its tiles, but wastes more of them at the grid's edges and in the last
+//    round of blocks: it is taken by the ratio of the two fills (64 -> 64 at
+//    80^3, ratio 0.65: 940 and 639 us; 48 -> 48 at 40^3, 0.59: 55 and 47, at 48^3,
+//    0.42: 75 and 92);
+//  - where they hold two or four tiles k_conv_fwd is ahead (48 -> 48 channels at
+//    96^3 326 and 393 us, 64 -> 64 at 32^3 41 and 110) but for 96 channels and
+//    more into up to 48 (112 -> 48 at 96^3 932 and 807).
+int conv_rows(int Z, int Y, int X, int Cin, int Kpad, int Cout) {
+  if (X < 32 || Y < 8 || Cin > 112 || (long)Y * X * Cin >= (1L << 31)) return 0;
+  const int TY = Cin <= 64 && conv_lds(8, Cin, Kpad) <= CONV_LDS ? 8 : 4;
+  if (conv_lds(TY, Cin, Kpad) > CONV_LDS) return 0;
+  if (Cout == 16 || conv_lds(TY, Cin, Kpad) + (size_t)Cout * (2 * Kpad + 16) <= CONV_LDS) return TY;
+  const int tx = (X + 31) / 32, ty = (Y + TY - 1) / TY, zper = conv_planes(Z, Y, X, TY);
+  if (zper == 1) return TY == 4 && Cout <= 48 ? TY : 0;
+  const double rounds = (double)(((long)tx * ty * ((Z + zper - 1) / zper) + 255) / 256);
+  // voxels of the grid over those of the tile rows that the CUs' rounds hold, the same of k_conv_fwd's tiles
+  const double fill = (double)Z * Y * X / (rounds * 256 * zper * 32 * TY);
+  const double fill_fwd = (double)X / ((X + 15) / 16 * 16) * Y / ((Y + 3) / 4 * 4);
+  const double least = X % 32 != 0 ? (Cin >= 64 && Cin != 80 ? 0.48 : 0.53) : Cin >= 96 && Cout <= 48 ? 0.6 : 2.0;
+  return fill >= least * fill_fwd ? TY : 0;
+}
+
 template <int TY, int NP>
 void conv_fwd_lds(const bf16* x, int Z, int Y, int X, int Cin, const bf16* w, int Kpad, int Cout, const float* bias,
                   int epi, float slope, const bf16* act, bf16* ob, float* of, int cstore, hipStream_t s) {
-  const int tiles = ((X + 31) / 32) * ((Y + TY - 1) / TY);
-  const int zper = std::max(2, (int)((long)Z * tiles / 512));
+  const int zper = conv_planes(Z, Y, X, TY);
   const dim3 g((X + 31) / 32, (Y + TY - 1) / TY, (Z + zper - 1) / zper), b(64 * TY);
   // the weights join the planes where they fit
   const size_t planes = conv_lds(TY, Cin, Kpad), wl = (size_t)Cout * (2 * Kpad + 16);
-  const bool in_lds = planes + wl <= 160 * 1024;
+  const bool in_lds = planes + wl <= CONV_LDS;
   const size_t lds = in_lds ? planes + wl : planes;
   hipEvent_t e0, e1;
   emmi::timing::kernel_events(emmi::timing::CONV, 54.0 * Cin * Cout * (double)Z * Y * X, &e0, &e1);
   auto go = [&](auto kernel) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, CONV_LDS);
     if (e0) hipExtLaunchKernelGGL(kernel, g, b, lds, s, e0, e1, 0, x, Z, Y, X, Cin, w, Kpad, bias, epi, slope, act, ob, of, cstore, zper);
     else hipLaunchKernelGGL(kernel, g, b, lds, s, x, Z, Y, X, Cin, w, Kpad, bias, epi, slope, act, ob, of, cstore, zper);
   };
@@ -873,25 +917,23 @@ extern "C" {
 
 int emmi_x0_kpad(int cin) { return (27 * cin + 31) / 32 * 32; }
 
+int emmi_x0_conv_route(int Z, int Y, int X, int Cin, int Cout) {
+  if (Cin % 16 || Cout % 16 || Cout > 128 || Cin <= 0 || Cout <= 0 || X <= 0 || Y <= 0 || Z <= 0) return -1;
+  return conv_rows(Z, Y, X, Cin, emmi_x0_kpad(Cin), Cout);
+}
+
 int emmi_x0_conv_fwd(const void* x, int Z, int Y, int X, int Cin, const void* w, int Cout, const float* bias, int epi,
                      float slope, const void* act, void* out_bf16, float* out_f32, int cout_store, void* stream) {
   if (Cin % 16 || Cout % 16 || Cout > 128 || Cin <= 0 || X <= 0 || Y <= 0 || Z <= 0) return -1;
   const int Kpad = emmi_x0_kpad(Cin);
   const bf16* xb = (const bf16*)x;
   const bf16* wb = (const bf16*)w;
-  // Rows of 32 voxels and more, in planes of at least eight rows, from LDS: eight
-  // rows where the planes of the tile fit it, four for more channels (up to 112)
-  if (X >= 32 && Y >= 8 && (long)Y * X * Cin < (1L << 31)) {
-    if (Cin <= 64 && conv_lds(8, Cin, Kpad) <= 160 * 1024) {
-      conv_fwd_lds<8, 6>(xb, Z, Y, X, Cin, wb, Kpad, Cout, bias, epi, slope, (const bf16*)act, (bf16*)out_bf16, out_f32, cout_store, S(stream));
-      return hipGetLastError() == hipSuccess ? 0 : -1;
-    }
-    if (Cin <= 112 && conv_lds(4, Cin, Kpad) <= 160 * 1024) {
-      conv_fwd_lds<4, 12>(xb, Z, Y, X, Cin, wb, Kpad, Cout, bias, epi, slope, (const bf16*)act, (bf16*)out_bf16, out_f32, cout_store, S(stream));
-      return hipGetLastError() == hipSuccess ? 0 : -1;
-    }
-  }
-  if (X % 64 == 0) conv_fwd_mt<4>(xb, Z, Y, X, Cin, wb, Kpad, Cout, bias, epi, slope, (const bf16*)act, (bf16*)out_bf16, out_f32, cout_store, S(stream));
+  const int TY = conv_rows(Z, Y, X, Cin, Kpad, Cout);
+  if (TY == 8)
+    conv_fwd_lds<8, 6>(xb, Z, Y, X, Cin, wb, Kpad, Cout, bias, epi, slope, (const bf16*)act, (bf16*)out_bf16, out_f32, cout_store, S(stream));
+  else if (TY == 4)
+    conv_fwd_lds<4, 12>(xb, Z, Y, X, Cin, wb, Kpad, Cout, bias, epi, slope, (const bf16*)act, (bf16*)out_bf16, out_f32, cout_store, S(stream));
+  else if (X % 64 == 0) conv_fwd_mt<4>(xb, Z, Y, X, Cin, wb, Kpad, Cout, bias, epi, slope, (const bf16*)act, (bf16*)out_bf16, out_f32, cout_store, S(stream));
   else if (X % 32 == 0) conv_fwd_mt<2>(xb, Z, Y, X, Cin, wb, Kpad, Cout, bias, epi, slope, (const bf16*)act, (bf16*)out_bf16, out_f32, cout_store, S(stream));
   else conv_fwd_mt<1>(xb, Z, Y, X, Cin, wb, Kpad, Cout, bias, epi, slope, (const bf16*)act, (bf16*)out_bf16, out_f32, cout_store, S(stream));
   return hipGetLastError() == hipSuccess ? 0 : -1;

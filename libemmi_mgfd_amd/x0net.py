@@ -49,6 +49,7 @@ def _lib():
     vp, i, f, d, l = C.c_void_p, C.c_int, C.c_float, C.c_double, C.c_long
     sig = {
         "emmi_x0_kpad": (i, [i]),
+        "emmi_x0_conv_route": (i, [i, i, i, i, i]),
         "emmi_x0_conv_fwd": (i, [vp, i, i, i, i, vp, i, vp, i, f, vp, vp, vp, i, vp]),
         "emmi_x0_conv_dw": (i, [vp, vp, i, i, i, i, i, vp, i, vp, vp, vp]),
         "emmi_x0_prep_weights": (i, [vp, i, i, vp, vp, vp]),

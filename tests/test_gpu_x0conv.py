@@ -114,3 +114,39 @@ def test_outputs_at_any_element_offset(shape):
             assert float(ob[nv * co + off]) == 7.0 and (off == 0 or float(ob[0]) == 7.0)
             outs.append(ob[off:off + nv * co].clone())
         assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("shape,ci,co", [((600, 16, 64), 16, 16), ((600, 16, 64), 48, 16), ((300, 20, 45), 16, 48),
+                                         ((600, 16, 64), 96, 32), ((80, 80, 80), 64, 64), ((40, 39, 41), 48, 48)],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_planes_of_a_march_equal_those_of_a_slab(shape, ci, co):
+    """Blocks that march through several planes (the ring of three planes in LDS
+    turns more than once) against slabs of the same input, one plane per block
+    or the gathering kernel: the same sums in the same order, bit for bit."""
+    from libemmi_mgfd_amd import x0net
+    Z, Y, X = shape
+    pl = Y * X
+    L = x0net._lib()
+    assert L.emmi_x0_conv_route(Z, Y, X, ci, co) > 0
+    gen = torch.Generator(device="cuda").manual_seed(ci + co)
+    x = torch.randn((Z * pl, ci), generator=gen, device="cuda").to(torch.bfloat16)
+    w = torch.randn((co, 27 * ci), generator=gen, device="cuda") / np.sqrt(27 * ci)
+    bias = torch.randn(co, generator=gen, device="cuda")
+    wf = torch.empty((co, x0net.kpad(ci)), dtype=torch.bfloat16, device="cuda")
+    wt = torch.empty((ci, x0net.kpad(co)), dtype=torch.bfloat16, device="cuda")
+    assert L.emmi_x0_prep_weights(w.data_ptr(), ci, co, wf.data_ptr(), wt.data_ptr(), None) == 0
+
+    def conv(z0, nz):
+        out = torch.full((nz * pl, co), float("nan"), dtype=torch.bfloat16, device="cuda")
+        assert L.emmi_x0_conv_fwd(x.data_ptr() + 2 * ci * z0 * pl, nz, Y, X, ci, wf.data_ptr(), co, bias.data_ptr(), 0,
+                                  x0net.SLOPE, None, out.data_ptr(), None, 0, None) == 0
+        torch.cuda.synchronize()
+        return out.reshape(nz, pl, co)
+
+    print(f"conv {shape} {ci}->{co}", flush=True)
+    whole, n = conv(0, Z), 6
+    assert bool(torch.isfinite(whole).all())
+    for z0 in [*range(0, Z - n, 4), Z - n]:
+        part = conv(z0, n)
+        lo, hi = (0 if z0 == 0 else 1), (n if z0 == Z - n else n - 1)
+        assert torch.equal(whole[z0 + lo:z0 + hi], part[lo:hi]), z0
