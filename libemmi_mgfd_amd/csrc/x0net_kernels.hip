@@ -312,8 +312,10 @@ __global__ void __launch_bounds__(64 * TY) k_conv_fwd_lds(const bf16* __restrict
 // What bounds it: with one tap and one input tile per block, every tile was
 // stored element by element (16 two-byte LDS stores a voxel) for one matrix
 // instruction per wave between two barriers; here five loads and five LDS
-// stores serve nine.  48 -> 16 channels at 96^3: 48 -> 16 channels at 96^3: 560 -> 203 us (180 TFLOP/s).
-constexpr int DW_WAVES = 16, DW_CHUNK = 32;
+// stores serve nine.  48 -> 16 channels at 96^3: 560 -> 203 us (180 TFLOP/s).
+// On small slabs the last phase, which adds the waves' sums, weighs more than
+// the chunks: fewer waves there (conv_dw_waves).
+constexpr int DW_CHUNK = 32;
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 // transposed read of rows r0 .. r0 + 31 of a [voxel][16] tile: lane l receives
@@ -326,7 +328,7 @@ __device__ __forceinline__ bf16x8 read_tr(const bf16* tile, int r0, int lane) {
   return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-template <int NCI>
+template <int NCI, int DW_WAVES>
 __global__ void __launch_bounds__(64 * DW_WAVES) k_conv_dw(const bf16* __restrict__ x, const bf16* __restrict__ dy,
                                                            int Z, int Y, int X, int Cin, int Cout, int zslab,
                                                            float* __restrict__ part) {
@@ -888,6 +890,15 @@ int conv_rows(int Z, int Y, int X, int Cin, int Kpad, int Cout) {
   return fill >= least * fill_fwd ? TY : 0;
 }
 
+// waves of a k_conv_dw block by the voxels of a slab: with sixteen, most of them
+// have no chunk on a small slab, and two blocks fill a CU.  All launches of a
+// weight and bias gradient, with 16, 8 and 4 waves (one wave per tile and tap,
+// four per block, before): 64 -> 64 channels at 8^3 (slabs of 64 voxels) 21.5,
+// 17.5 and 16.3 us (16.4); at 12^3 (144) 29.2, 22.7 and 20.5 (23.2); at 31^3 (961)
+// 78.5, 56.7 and 53.2 (114.7); 16 -> 16 at 31^3 26.2, 23.3 and 24.5 (24.2), at 32^3
+// (2048) 20.0, 21.0 and 26.4 (23.7).
+int conv_dw_waves(long nv) { return nv <= 2 * DW_CHUNK ? 4 : nv <= 32 * DW_CHUNK ? 8 : 16; }
+
 template <int TY, int NP>
 void conv_fwd_lds(const bf16* x, int Z, int Y, int X, int Cin, const bf16* w, int Kpad, int Cout, const float* bias,
                   int epi, float slope, const bf16* act, bf16* ob, float* of, int cstore, hipStream_t s) {
@@ -944,9 +955,11 @@ int emmi_x0_conv_dw(const void* x, const void* dy, int Z, int Y, int X, int Cin,
   if (Cin % 16 || Cout % 16 || Cout > 256 || zslab < 1 || Z < 1 || Y < 1 || X < 1) return -1;
   if ((long)Z * Y * X >= (1L << 31)) return -1;   // the kernel indexes voxels in 32 bits
   const int nslab = (Z + zslab - 1) / zslab;
-  // input tiles per block: up to three
-  const int nci = Cin / 16, NCI = nci == 4 ? 2 : std::min(nci, 3);
-  const dim3 g(9 * ((nci + NCI - 1) / NCI) * (Cout / 16), nslab), b(64 * DW_WAVES);
+  // input tiles per block: up to three, one where single tiles do not fill the
+  // CUs (48 -> 16 channels at 8^3 14.4 and 13.0 us)
+  const int nci = Cin / 16, NCI = 9L * nci * (Cout / 16) * nslab <= 256 ? 1 : nci == 4 ? 2 : std::min(nci, 3);
+  const int waves = conv_dw_waves((long)std::min(zslab, Z) * Y * X);
+  const dim3 g(9 * ((nci + NCI - 1) / NCI) * (Cout / 16), nslab), b(64 * waves);
   hipEvent_t e0, e1;
   emmi::timing::kernel_events(emmi::timing::CONV_DW, 54.0 * Cin * Cout * (double)Z * Y * X, &e0, &e1);
   auto go = [&](auto kernel) {
@@ -954,9 +967,14 @@ int emmi_x0_conv_dw(const void* x, const void* dy, int Z, int Y, int X, int Cin,
                                   Cout, zslab, part);
     else hipLaunchKernelGGL(kernel, g, b, 0, S(stream), (const bf16*)x, (const bf16*)dy, Z, Y, X, Cin, Cout, zslab, part);
   };
-  if (NCI == 1) go(k_conv_dw<1>);
-  else if (NCI == 2) go(k_conv_dw<2>);
-  else go(k_conv_dw<3>);
+#define CASE(W)                             \
+  case W:                                   \
+    if (NCI == 1) go(k_conv_dw<1, W>);      \
+    else if (NCI == 2) go(k_conv_dw<2, W>); \
+    else go(k_conv_dw<3, W>);               \
+    break;
+  switch (waves) { CASE(4) CASE(8) CASE(16) }
+#undef CASE
   const long n = 27L * Cin * Cout;
   hipLaunchKernelGGL(k_reduce_slabs, dim3(blocks(n, 256)), dim3(256), 0, S(stream), part, nslab, n, dw);
   if (db) {

@@ -5,7 +5,8 @@ LDS and, for many channels, in memory, with four rows instead of eight, and the
 one that gathers from memory (narrower grids, 128 channels); partial tiles along
 every axis, single planes and rows; the weight gradient with one, two and three
 input tiles per block, groups that the channels do not fill, chunks across row
-and plane ends, and a slab shorter than the others.
+and plane ends, a slab shorter than the others, and blocks of four, eight and
+sixteen waves (slabs of up to 64, up to 1024 and of more voxels).
 
 Tolerances: products of BF16 values are exact in FP32 and sums of K = 27 Cin
 terms (or of all voxels, for the weight gradient) round at 2^-24 each, so 1e-5
@@ -18,7 +19,7 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(1, 8, 32), (3, 9, 33), (2, 16, 40), (5, 8, 64), (4, 11, 95), (1, 13, 47), (6, 7, 32), (5, 9, 31), (2, 1, 40), (3, 2, 5), (1, 1, 1)]
+SHAPES = [(1, 8, 32), (3, 9, 33), (3, 17, 33), (2, 16, 40), (5, 8, 64), (4, 11, 95), (1, 13, 47), (6, 7, 32), (5, 9, 31), (2, 1, 40), (3, 2, 5), (1, 1, 1)]
 CHANNELS = [(16, 16), (32, 48), (48, 16), (64, 64), (80, 32), (112, 48), (128, 16), (16, 128)]
 
 
