@@ -38,8 +38,8 @@
 #include <cstdint>
 #include <map>
 #include <mutex>
-#include <set>
-#include <utility>
+#include <stdexcept>
+#include "dynamic_lds.h"
 #include "stencil.h"
 #include "timing.h"
 
@@ -1258,12 +1258,11 @@ __global__ void __launch_bounds__(128) k_line_solve(LinePack<T> P) {
 // FP32, three 245 -> 225 and 280 -> 196; 96 nodes, FP32, eight 370 -> 248 and
 // 330 -> 218; 64 nodes, FP64, one 37 -> 24; 16 nodes 12.5 -> 9.5; one line of 96
 // nodes, eight right-hand sides 26 -> 16.
-constexpr int M_LDS = 160 * 1024;          // LDS of a CU
 // LDS of a line: 2 T edges (1 complex), 2 T - 1 node vectors (4 complex) and
 // room for one more, which the last step's read of the node after next meets
 __host__ __device__ __forceinline__ int line_m_bytes(int n) { return 160 * HalfOrder(n).T; }
-static int line_m_lpb(int n) { return 8 * line_m_bytes(n) <= M_LDS ? 8 : 2; }
-static bool line_m_fits(int n) { return 2 * line_m_bytes(n) <= M_LDS; }
+static int line_m_lpb(int n) { return 8 * line_m_bytes(n) <= CU_LDS ? 8 : 2; }
+static bool line_m_fits(int n) { return 2 * line_m_bytes(n) <= CU_LDS; }
 // lines whose records are in memory: lines of a block, nodes in flight per half
 constexpr int LONG_LPB = 8, LONG_RING = 8;
 
@@ -1974,20 +1973,11 @@ static void launch_timed(K kernel, dim3 g, dim3 b, hipStream_t s, int cls, Bytes
   else hipLaunchKernelGGL(kernel, g, b, 0, s, args...);
 }
 
-// the same with dynamic LDS (more than the default 64 KiB is enabled once per
-// kernel and device)
+// the same with dynamic LDS
 template <typename K, typename... Args>
 static void launch_lds(K kernel, dim3 g, dim3 b, size_t lds, hipStream_t s, int cls, Bytes bytes, Args... args) {
-  if (lds > 64 * 1024) {
-    static std::mutex mu;
-    static std::set<std::pair<const void*, int>> done;
-    int dev = 0;
-    (void)hipGetDevice(&dev);
-    std::lock_guard<std::mutex> lk(mu);
-    const void* fn = reinterpret_cast<const void*>(kernel);
-    if (done.insert({fn, dev}).second)
-      (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, M_LDS);
-  }
+  if (lds > 64 * 1024 && allow_lds(reinterpret_cast<const void*>(kernel)) != hipSuccess)
+    throw std::runtime_error("a line kernel was refused its LDS");
   hipEvent_t e0, e1;
   timing::kernel_events(cls, bytes.comp, &e0, &e1, bytes.layout);
   if (e0) hipExtLaunchKernelGGL(kernel, g, b, lds, s, e0, e1, 0, args...);

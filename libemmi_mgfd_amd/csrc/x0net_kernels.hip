@@ -20,6 +20,7 @@
 #include <algorithm>
 #include <cmath>
 
+#include "dynamic_lds.h"
 #include "emmi_mgfd.h"
 #include "timing.h"
 
@@ -842,8 +843,6 @@ void conv_fwd_mt(const bf16* x, int Z, int Y, int X, int Cin, const bf16* w, int
   }
 }
 
-constexpr size_t CONV_LDS = 160 * 1024;   // of a CU
-
 // LDS bytes of k_conv_fwd_lds for rows TY
 size_t conv_lds(int TY, int Cin, int Kpad) {
   return 3 * (size_t)((TY + 2) * 34) * (2 * Cin + 16) + (3 * (Kpad / 8) * sizeof(int) + 15) / 16 * 16;
@@ -877,9 +876,9 @@ int conv_planes(int Z, int Y, int X, int TY) {
 //    more into up to 48 (112 -> 48 at 96^3 932 and 807).
 int conv_rows(int Z, int Y, int X, int Cin, int Kpad, int Cout) {
   if (X < 32 || Y < 8 || Cin > 112 || (long)Y * X * Cin >= (1L << 31)) return 0;
-  const int TY = Cin <= 64 && conv_lds(8, Cin, Kpad) <= CONV_LDS ? 8 : 4;
-  if (conv_lds(TY, Cin, Kpad) > CONV_LDS) return 0;
-  if (Cout == 16 || conv_lds(TY, Cin, Kpad) + (size_t)Cout * (2 * Kpad + 16) <= CONV_LDS) return TY;
+  const int TY = Cin <= 64 && conv_lds(8, Cin, Kpad) <= (size_t)emmi::CU_LDS ? 8 : 4;
+  if (conv_lds(TY, Cin, Kpad) > (size_t)emmi::CU_LDS) return 0;
+  if (Cout == 16 || conv_lds(TY, Cin, Kpad) + (size_t)Cout * (2 * Kpad + 16) <= (size_t)emmi::CU_LDS) return TY;
   const int tx = (X + 31) / 32, ty = (Y + TY - 1) / TY, zper = conv_planes(Z, Y, X, TY);
   if (zper == 1) return TY == 4 && Cout <= 48 ? TY : 0;
   const double rounds = (double)(((long)tx * ty * ((Z + zper - 1) / zper) + 255) / 256);
@@ -900,26 +899,28 @@ int conv_rows(int Z, int Y, int X, int Cin, int Kpad, int Cout) {
 int conv_dw_waves(long nv) { return nv <= 2 * DW_CHUNK ? 4 : nv <= 32 * DW_CHUNK ? 8 : 16; }
 
 template <int TY, int NP>
-void conv_fwd_lds(const bf16* x, int Z, int Y, int X, int Cin, const bf16* w, int Kpad, int Cout, const float* bias,
+bool conv_fwd_lds(const bf16* x, int Z, int Y, int X, int Cin, const bf16* w, int Kpad, int Cout, const float* bias,
                   int epi, float slope, const bf16* act, bf16* ob, float* of, int cstore, hipStream_t s) {
   const int zper = conv_planes(Z, Y, X, TY);
   const dim3 g((X + 31) / 32, (Y + TY - 1) / TY, (Z + zper - 1) / zper), b(64 * TY);
   // the weights join the planes where they fit
   const size_t planes = conv_lds(TY, Cin, Kpad), wl = (size_t)Cout * (2 * Kpad + 16);
-  const bool in_lds = planes + wl <= CONV_LDS;
+  const bool in_lds = planes + wl <= (size_t)emmi::CU_LDS;
   const size_t lds = in_lds ? planes + wl : planes;
   hipEvent_t e0, e1;
   emmi::timing::kernel_events(emmi::timing::CONV, 54.0 * Cin * Cout * (double)Z * Y * X, &e0, &e1);
   auto go = [&](auto kernel) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, CONV_LDS);
+    if (lds > 64 * 1024 && emmi::allow_lds(reinterpret_cast<const void*>(kernel)) != hipSuccess) return false;
     if (e0) hipExtLaunchKernelGGL(kernel, g, b, lds, s, e0, e1, 0, x, Z, Y, X, Cin, w, Kpad, bias, epi, slope, act, ob, of, cstore, zper);
     else hipLaunchKernelGGL(kernel, g, b, lds, s, x, Z, Y, X, Cin, w, Kpad, bias, epi, slope, act, ob, of, cstore, zper);
+    return true;
   };
   switch (Cout / 16) {
-#define CASE(NT) case NT: if (in_lds) go(k_conv_fwd_lds<NT, TY, NP, true>); else go(k_conv_fwd_lds<NT, TY, NP, false>); break;
+#define CASE(NT) case NT: return in_lds ? go(k_conv_fwd_lds<NT, TY, NP, true>) : go(k_conv_fwd_lds<NT, TY, NP, false>);
     CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
 #undef CASE
   }
+  return true;
 }
 
 }  // namespace
@@ -940,14 +941,15 @@ int emmi_x0_conv_fwd(const void* x, int Z, int Y, int X, int Cin, const void* w,
   const bf16* xb = (const bf16*)x;
   const bf16* wb = (const bf16*)w;
   const int TY = conv_rows(Z, Y, X, Cin, Kpad, Cout);
+  bool ok = true;
   if (TY == 8)
-    conv_fwd_lds<8, 6>(xb, Z, Y, X, Cin, wb, Kpad, Cout, bias, epi, slope, (const bf16*)act, (bf16*)out_bf16, out_f32, cout_store, S(stream));
+    ok = conv_fwd_lds<8, 6>(xb, Z, Y, X, Cin, wb, Kpad, Cout, bias, epi, slope, (const bf16*)act, (bf16*)out_bf16, out_f32, cout_store, S(stream));
   else if (TY == 4)
-    conv_fwd_lds<4, 12>(xb, Z, Y, X, Cin, wb, Kpad, Cout, bias, epi, slope, (const bf16*)act, (bf16*)out_bf16, out_f32, cout_store, S(stream));
+    ok = conv_fwd_lds<4, 12>(xb, Z, Y, X, Cin, wb, Kpad, Cout, bias, epi, slope, (const bf16*)act, (bf16*)out_bf16, out_f32, cout_store, S(stream));
   else if (X % 64 == 0) conv_fwd_mt<4>(xb, Z, Y, X, Cin, wb, Kpad, Cout, bias, epi, slope, (const bf16*)act, (bf16*)out_bf16, out_f32, cout_store, S(stream));
   else if (X % 32 == 0) conv_fwd_mt<2>(xb, Z, Y, X, Cin, wb, Kpad, Cout, bias, epi, slope, (const bf16*)act, (bf16*)out_bf16, out_f32, cout_store, S(stream));
   else conv_fwd_mt<1>(xb, Z, Y, X, Cin, wb, Kpad, Cout, bias, epi, slope, (const bf16*)act, (bf16*)out_bf16, out_f32, cout_store, S(stream));
-  return hipGetLastError() == hipSuccess ? 0 : -1;
+  return ok && hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 int emmi_x0_conv_dw(const void* x, const void* dy, int Z, int Y, int X, int Cin, int Cout, float* part, int zslab,
