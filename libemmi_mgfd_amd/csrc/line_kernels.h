@@ -77,6 +77,11 @@ enum LineRoute { LINE_ROUTE_ONE_LANE = 0, LINE_ROUTE_MATRIX = 1, LINE_ROUTE_MATR
 LineRoute line_route(int esize, int axis, int njobs, const int* cells, const long* lines, bool one_lane);
 // the route under the current mode, without the autotuner's table
 LineRoute line_route_now(int esize, int axis, int njobs, const int* cells, const long* lines);
+// whether a launch over lines of a level of n cells along an axis, for up to
+// LINE_PACK_MAX right-hand sides, can need line records in memory (LineJob::scr)
+// under the current mode and the autotuner's table.  A pack without them keeps
+// to the LDS where its lines fit it, and is refused otherwise.
+bool line_needs_scratch(int esize, const int* n, int axis);
 
 // Autotuning: a launch shape (value size of the cycle precision, axis, line
 // length, lines per job, jobs per pack) and the substitution choice measured

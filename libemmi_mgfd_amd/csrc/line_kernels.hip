@@ -1938,6 +1938,23 @@ int line_choices(int* out, double* us, int maxn) {
   return i;
 }
 
+bool line_needs_scratch(int esize, const int* n, int axis) {
+  {
+    std::lock_guard<std::mutex> g(g_tuned_mu);
+    for (const auto& kv : g_tuned)
+      if (kv.second.choice == LINE_ONE_LANE) return true;
+  }
+  for (int colour = 0; colour < 4; colour++) {
+    int nlo, nhi, cells[LINE_PACK_MAX];
+    long lines[LINE_PACK_MAX];
+    line_colour_counts(n, axis, colour, &nlo, &nhi);
+    std::fill(cells, cells + LINE_PACK_MAX, n[axis]);
+    std::fill(lines, lines + LINE_PACK_MAX, (long)nlo * nhi);
+    if (line_route_now(esize, axis, LINE_PACK_MAX, cells, lines) != LINE_ROUTE_MATRIX) return true;
+  }
+  return false;
+}
+
 static size_t chunks_of(int values, size_t esize) {
   const size_t v = 16 / esize;
   return (values + v - 1) / v;
@@ -2075,7 +2092,10 @@ static void launch_pack(const LinePack<T>& P, int axis, bool factor, hipStream_t
   }
   if (choice == LINE_RULE && g_line_kernel == 0) choice = tuned_choice(line_shape(P, axis));
   const bool one_lane = choice == LINE_ONE_LANE || (choice == LINE_RULE && g_line_kernel == 1);
-  const LineRoute route = line_route(sizeof(T), axis, P.njobs, cells, lines, one_lane);
+  bool scr = true;
+  for (int j = 0; j < P.njobs; j++) scr = scr && P.job[j].scr;
+  const LineRoute route = line_route(sizeof(T), axis, P.njobs, cells, lines, one_lane && scr);
+  if (route != LINE_ROUTE_MATRIX && !scr) throw std::runtime_error("a line sweep without its records in memory");
   if (route != LINE_ROUTE_ONE_LANE) {
     const bool mem = route == LINE_ROUTE_MATRIX_MEM;
     launch_line_m<T>(P, axis, mem, maxl, maxna, s, Bytes{comp, rhs_bytes + solve_bytes - (mem ? 0.0 : 2.0 * rec_bytes)});

@@ -112,7 +112,7 @@ struct Slot {
   void* f64 = nullptr;
   void* r64 = nullptr;               // FP64 mode: r[0]; FP32-storage cycles: blend_guess scratch (lazy)
   std::vector<LineFactors> facs;     // [(pattern*lmax + level)*3 + axis]; level 0 under pattern 0
-  void* lscr = nullptr;              // right-hand side / substitution records of the line solves
+  void* lscr = nullptr;              // line records in memory (lazy: line_scratch)
   double* partial = nullptr;         // residual-norm partial sums
   double rnorm0 = 0;
   SolveStats* st = nullptr;
@@ -223,6 +223,9 @@ class Solver {
   // (the next cycle's right-hand side); with `add` each slot's pending FP32
   // correction u[0] is added to u64 first.
   void norms(const std::vector<int>& which, bool add, std::vector<double>& out);
+  // line records in memory of slots 0..n-1, allocated where a sweep can need
+  // them (outside graph capture) or at once
+  void line_scratch(int n, bool always = false);
 
   int n_[3];
   long nc0_;

@@ -280,7 +280,6 @@ void Solver::init(int n1, int n2, int n3, int nmed, const float* const* x1, cons
       S.r64 = nullptr;   // scratch of blend_guess only, allocated there on first use
     }
     S.facs.assign((size_t)npat_ * lmax_ * 3, LineFactors());
-    S.lscr = dalloc(std::max<size_t>(16, lscr_bytes_), owned_);
     S.partial = (double*)dalloc(sizeof(double) * residual_blocks_max(n_), owned_);
   }
   dnorm_ = (double*)dalloc(sizeof(double) * nslots, owned_);
@@ -294,6 +293,15 @@ Solver::~Solver() {
   drop_graphs();
   owned_.release();
   if (hnorm_) hipHostFree(hnorm_);
+}
+
+void Solver::line_scratch(int n, bool always) {
+  const int esize = p_.precision == 0 ? 8 : 4;
+  for (int c = 0; c < npat_ && !always; c++)
+    for (int lev = 0; lev < lmax_; lev++)
+      for (int a = 0; a < 3; a++) always = always || line_needs_scratch(esize, dims_[c][lev].data(), a);
+  for (int k = 0; k < n && always; k++)
+    if (!slots_[k].lscr) slots_[k].lscr = dalloc(std::max<size_t>(16, lscr_bytes_), owned_);
 }
 
 void Solver::set_omega(int slot, float omega) {
@@ -421,6 +429,7 @@ LineFactors& Solver::factors(Slot& S, int pat, int lev, int axis) {
 
 template <typename T>
 void Solver::line_sweep_on(int pat, int lev, int axis, int iter, void* u, const void* f) {
+  line_scratch(1);
   Slot& S = slots_[0];
   const LineFactors& F = factors<T>(S, pat, lev, axis);
   const DevLevel<T>& L = hier<T>(S.med).pat[pat][lev];
@@ -512,6 +521,7 @@ void Solver::smooth(int pat, int lev, int iter) {
 template <typename T>
 int Solver::autotune_t(int reps) {
   if (reps < 1) reps = 1;
+  line_scratch(nslots(), true);
   std::vector<int> all(slots_.size());
   for (size_t k = 0; k < slots_.size(); k++) all[k] = (int)k;
   hipEvent_t e0, e1;
@@ -934,6 +944,7 @@ int Solver::solve_batch(int n, const void* const* b, void* const* x, void* const
                         SolveStats* st) {
   if (n < 1 || n > nslots()) throw std::runtime_error("batch size out of range of the solver's slots");
   const long nv = 3 * nc0_;
+  line_scratch(n);
   // The launch-error check at the end of the solve reads the thread's last
   // HIP error; clear what calls outside the solver left there (unchecked
   // frees and queries of other objects) so that it reports this solve's.
