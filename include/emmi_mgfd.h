@@ -392,10 +392,13 @@ int emmi_memcpy_d2h(void *dst, const void *src, size_t bytes);
 int emmi_memcpy_d2d(void *dst, const void *src, size_t bytes);
 int emmi_device_sync(void);
 /* Line-substitution kernel of the following launches (no counterpart in the
- * reference; for tests and tuning): 0 the matrix-core kernel (default; the
- * autotuner's table is consulted), 1 one lane per line half, 2 to 4 the
- * matrix-core kernel without the table.  All solve the same line systems
- * exactly.  Graphs a solver captured earlier keep the kernels they captured.  Returns the previous mode, or -1 for an unknown mode. */
+ * reference; for tests and tuning): 0 the matrix-core kernels (default; the
+ * autotuner's table is consulted), 1 one lane per line half, 2 and 4 the
+ * matrix-core kernels without the table, 3 the same with every residual record
+ * built node by node (the same sweep, bit for bit).  Colours of many long lines
+ * take one lane per line half in every mode (emmi_line_route).  All solve the
+ * same line systems exactly.  Graphs a solver captured earlier keep the kernels
+ * they captured.  Returns the previous mode, or -1 for an unknown mode. */
 int emmi_set_line_kernel(int mode);
 /* the substitution that a launch over njobs jobs (1 to 16) along an axis takes
  * in the current mode (without the autotuner's table), job j having lines[j]

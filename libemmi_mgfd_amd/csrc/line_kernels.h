@@ -64,9 +64,9 @@ inline void line_job_colour(LineJob<T>& J, int a, int colour) {
 
 // substitution kernel of later launches: 0 the matrix-core kernel (or the
 // autotuner's choice where its table has the
-// launch's shape), 1 the one-lane kernel, 2, 3, 4 as 0 without the table
-// (they named kernels that the matrix-core one replaced); returns the previous
-// mode or -1
+// launch's shape), 1 the one-lane kernel, 2 and 4 as 0 without the table, 3 the
+// same with every residual record built node by node; returns the previous mode
+// or -1
 int set_line_kernel(int mode);
 
 // The substitution that a launch takes.  The matrix-core kernels lay out their

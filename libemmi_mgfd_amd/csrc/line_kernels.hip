@@ -2005,8 +2005,9 @@ static void launch_lds(K kernel, dim3 g, dim3 b, size_t lds, hipStream_t s, int 
 // ring by the length of a half
 template <typename T, int A>
 static void launch_line_m_axis(const LinePack<T>& P, bool mem, int maxl, int maxna, hipStream_t s, Bytes by) {
+  const bool by_node = g_line_kernel == 3;   // residual records node by node (for tests)
   if (mem) {
-    const int run = A == 0 || maxl < 64 ? 1 : 8;
+    const int run = A == 0 || maxl < 64 || by_node ? 1 : 8;
     auto blocks = [&](long n, int per) { return dim3((unsigned)((n + per - 1) / per), P.njobs); };
     launch_timed(k_line_long_rhs<T, A>, blocks((long)maxl * ((maxna + run - 1) / run), 256), dim3(256), s, timing::LINE_RHS,
                  Bytes{0.0, 0.0}, P, run);
@@ -2023,7 +2024,7 @@ static void launch_line_m_axis(const LinePack<T>& P, bool mem, int maxl, int max
   // leave most threads of its block without a run (one line of 96 nodes: 23 us
   // marched, 16 node by node).
   if constexpr (A != 0) {
-    if (D == 8 && maxna >= 64 && maxl > 4) {
+    if (D == 8 && maxna >= 64 && maxl > 4 && !by_node) {
       if (lpb == 2) go(k_line_solve_m<T, A, 2, 8, M_MARCH>);
       else go(k_line_solve_m<T, A, 8, 8, M_MARCH>);
       return;
@@ -2032,7 +2033,7 @@ static void launch_line_m_axis(const LinePack<T>& P, bool mem, int maxl, int max
   if (lpb == 2) {
     if (D == 8) go(k_line_solve_m<T, A, 2, 8, M_NODES>);
     else go(k_line_solve_m<T, A, 2, 4, M_NODES>);
-  } else if (maxna <= 32 && D < 8 && (long)g.x * P.njobs <= 256) {
+  } else if (maxna <= 32 && D < 8 && (long)g.x * P.njobs <= 256 && !by_node) {
     // at most a block per CU (the look-ahead takes the registers of a second:
     // solves of one slot 64^3 10.3 -> 10.1 ms, 12x10x16 13.1 -> 12.8; eight slots
     // on 96^3 without this limit 55.6 -> 56.4)

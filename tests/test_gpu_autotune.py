@@ -1,10 +1,9 @@
 """The line-sweep autotuner (emmi_solver_autotune; no counterpart in the
 reference, which has one smoother implementation).
 
-For each launch shape of a solve the autotuner times the three substitution
-kernels (one lane per line half; four lanes with the right-hand sides in the
-same launch; four lanes with a separate right-hand-side launch) and records
-the fastest in a process-wide table that later launches of that shape use.
+For each launch shape of a solve the autotuner times the substitution kernels
+(one lane per line half; matrix cores) and records the fastest in a process-wide
+table that later launches of that shape use.
 Checked here on the 64^3 survey (six levels, every shape class of the line
 sweeps) with three right-hand sides batched:
 

@@ -41,7 +41,7 @@ def solve_config2(precision, tol, survey=None):
     return sc, s, sts
 
 
-@pytest.fixture(params=[0, 1, 2], ids=["auto", "one_lane", "quad_lane"])
+@pytest.fixture(params=[0, 1, 3], ids=["auto", "one_lane", "matrix_by_node"])
 def line_kernel(request):
     L = native.lib()
     prev = L.emmi_set_line_kernel(request.param)
@@ -50,8 +50,7 @@ def line_kernel(request):
 
 
 def test_config2_mixed_matches_fp64_at_bench_tolerance():
-    """FP32-storage cycles (one-lane substitution on the two finest levels,
-    quad-lane below) against the FP64 solve at the benchmark's tolerance:
+    """FP32-storage cycles against the FP64 solve at the benchmark's tolerance:
     the signal channels agree within 1e-5."""
     print("config2 batched solves, precision 1 and 0, tol 1e-6", flush=True)
     sc1, s, st1 = solve_config2(1, 1e-6)

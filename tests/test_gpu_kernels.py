@@ -24,10 +24,10 @@ def tiny():
     return s, g, n, L0
 
 
-@pytest.fixture(params=[1, 2], ids=["one_lane", "quad_lane"])
+@pytest.fixture(params=[1, 2], ids=["one_lane", "matrix"])
 def line_kernel(request):
-    """Runs a test with each line-substitution kernel (one lane or four lanes
-    per line half), whatever the line count would select."""
+    """Runs a test with each line-substitution kernel (one lane per line half,
+    matrix cores), whatever the autotuner's table holds."""
     from libemmi_mgfd_amd import native
     L = native.lib()
     prev = L.emmi_set_line_kernel(request.param)
@@ -176,7 +176,7 @@ def test_line_gs_fp32_air_finite(tiny, line_kernel):
 @pytest.mark.parametrize("precision,tol", [(0, 1e-12), (1, 1e-6)])
 @pytest.mark.parametrize("axis", [0, 1, 2])
 def test_line_kernels_agree(tiny, axis, precision, tol):
-    """The one-lane and quad-lane substitutions solve the same line systems
+    """The one-lane and matrix-core substitutions solve the same line systems
     exactly: on well-conditioned blocks they agree to rounding (FP64) or to
     the FP32 rounding of the stored records and vectors."""
     from libemmi_mgfd_amd import native
@@ -193,20 +193,22 @@ def test_line_kernels_agree(tiny, axis, precision, tol):
             outs.append(S.check_op(1, 0, 0, axis, 1, random_field(n, 21), random_field(n, 22)))
     finally:
         L.emmi_set_line_kernel(prev)
-    print("one-lane vs quad-lane rel", rel(outs[1], outs[0]))
+    print("one-lane vs matrix-core rel", rel(outs[1], outs[0]))
     assert rel(outs[1], outs[0]) < tol
 
 
-@pytest.mark.parametrize("n", [(128, 128, 64), (64, 96, 48)], ids=["128x128x64", "64x96x48"])
+@pytest.mark.parametrize("n", [(128, 128, 64), (64, 96, 48), (20, 12, 14), (6, 4, 10), (12, 10, 280), (10, 22, 1030)],
+                         ids=lambda n: "x".join(map(str, n)))
 @pytest.mark.parametrize("precision", [0, 1])
 def test_line_rhs_march_matches_node_records(precision, n):
-    """The fused quad-lane launch builds its lines' right-hand sides by
+    """Lines of 64 nodes and more along y and z build their residual records by
     marching along them (values shared by neighbouring nodes carried in
-    registers); the separate right-hand-side launch builds each node on its
-    own.  Both evaluate every operator row with the same arithmetic, so a
-    sweep gives the same result to the last bit.  Lines of 128, 96, 64 and 48
-    nodes (records in LDS and in memory; the march on the 64- and 128-node
-    lines along y and z), with an air layer and a layered earth."""
+    registers), short ones row by row where that fills a block better; mode 3
+    builds every record node by node.  All evaluate every operator row with
+    the same arithmetic, so a sweep gives the same result to the last bit.
+    Lines of 128, 96, 64 and 48 nodes, short ones (a thread per node; a thread
+    per row), lines of two-line blocks and lines whose records are in memory,
+    with an air layer and a layered earth."""
     from libemmi_mgfd_amd import native
     rng = np.random.default_rng(11)
     xs = [np.cumsum(np.r_[0.0, rng.uniform(20.0, 80.0, m)]).astype(np.float32) for m in n]
@@ -219,7 +221,7 @@ def test_line_rhs_march_matches_node_records(precision, n):
     prev = L.emmi_set_line_kernel(3)
     try:
         for axis in range(3):
-            print(f"line sweep {n} precision {precision} axis {axis}: fused vs separate records", flush=True)
+            print(f"line sweep {n} precision {precision} axis {axis}: node by node vs by the rule", flush=True)
             outs = []
             for mode in (3, 4):
                 L.emmi_set_line_kernel(mode)
