@@ -2031,8 +2031,7 @@ static void launch_line_m_axis(const LinePack<T>& P, bool mem, int maxl, int max
     }
   }
   if (lpb == 2) {
-    if (D == 8) go(k_line_solve_m<T, A, 2, 8, M_NODES>);
-    else go(k_line_solve_m<T, A, 2, 4, M_NODES>);
+    go(k_line_solve_m<T, A, 2, 8, M_NODES>);   // (more than 256 nodes: groups of eight)
   } else if (maxna <= 32 && D < 8 && (long)g.x * P.njobs <= 256 && !by_node) {
     // at most a block per CU (the look-ahead takes the registers of a second:
     // solves of one slot 64^3 10.3 -> 10.1 ms, 12x10x16 13.1 -> 12.8; eight slots
