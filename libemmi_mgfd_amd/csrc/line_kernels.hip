@@ -2033,9 +2033,12 @@ static void launch_line_m_axis(const LinePack<T>& P, bool mem, int maxl, int max
   if (lpb == 2) {
     go(k_line_solve_m<T, A, 2, 8, M_NODES>);   // (more than 256 nodes: groups of eight)
   } else if (maxna <= 32 && D < 8 && (long)g.x * P.njobs <= 256 && !by_node) {
-    // at most a block per CU (the look-ahead takes the registers of a second:
-    // solves of one slot 64^3 10.3 -> 10.1 ms, 12x10x16 13.1 -> 12.8; eight slots
-    // on 96^3 without this limit 55.6 -> 56.4)
+    // at most a block per CU: the look-ahead costs FP32 launches along y and z
+    // their third wave per SIMD (163 -> 197 to 220 registers; 192 x 192 lines of 4
+    // nodes 11.6 -> 13.1 us, of 12 22.2 -> 25.6; FP64 and x keep two, 14.9 -> 13.1).
+    // Within the limit, node by node -> ahead: 64 x 64 lines of 4 nodes FP64
+    // 5.9 -> 5.3 us, FP32 6.3 -> 5.5, of 6 6.7 -> 6.1 and 6.9 -> 6.2, of 8 6.4 ->
+    // 6.7 and 6.6 -> 6.8, of 12 to 28 within 3%
     if (D == 4) go(k_line_solve_m<T, A, 8, 4, M_SHORT>);
     else go(k_line_solve_m<T, A, 8, 2, M_SHORT>);
   } else {
@@ -2055,7 +2058,7 @@ template <typename T>
 static void launch_pack(const LinePack<T>& P, int axis, bool factor, hipStream_t s, int choice = LINE_RULE) {
   int maxl = 0;
   long maxnodes = 0;
-  double rhs_bytes = 0, solve_bytes = 0, rec_bytes = 0, comp = 0;
+  double rhs_bytes = 0, solve_bytes = 0, rec_bytes = 0, scr_bytes = 0, comp = 0;
   const double es = sizeof(typename cvec<T>::type), cs = sizeof(T);
   for (int j = 0; j < P.njobs; j++) {
     // compulsory bytes of one colour: a quarter of a full sweep's
@@ -2068,11 +2071,13 @@ static void launch_pack(const LinePack<T>& P, int axis, bool factor, hipStream_t
     if (nl * na > maxnodes) maxnodes = nl * na;
     const double rows = (double)nl * (5.0 * na - 4.0);
     // right-hand sides: the colour's rows read f and sigma-bar once, u is
-    // read once over the level, the records are written once
-    rhs_bytes += rows * (es + cs) + 3.0 * (double)P.job[j].L.nc * es + (double)nl * na * SREC * sizeof(ScrRec<T>);
-    // substitution: records and factors read once, the rows of u read and written
-    solve_bytes += (double)nl * na * (SREC * sizeof(ScrRec<T>) + FREC * sizeof(FacRec<T>)) + rows * 2.0 * es;
+    // read once over the level
+    rhs_bytes += rows * (es + cs) + 3.0 * (double)P.job[j].L.nc * es;
+    // substitution: factors read by both passes, the rows of u read and written
+    solve_bytes += (double)nl * na * 2.0 * FREC * sizeof(FacRec<T>) + rows * 2.0 * es;
+    // records in memory: written, read by both passes, z written by the first
     rec_bytes += (double)nl * na * SREC * sizeof(ScrRec<T>);
+    scr_bytes += (double)nl * na * (2.0 * SREC + 8.0) * sizeof(ScrRec<T>);
   }
   if (maxl == 0 || P.njobs == 0) return;
   int maxna = 0, cells[LINE_PACK_MAX];
@@ -2098,9 +2103,11 @@ static void launch_pack(const LinePack<T>& P, int axis, bool factor, hipStream_t
   if (route != LINE_ROUTE_MATRIX && !scr) throw std::runtime_error("a line sweep without its records in memory");
   if (route != LINE_ROUTE_ONE_LANE) {
     const bool mem = route == LINE_ROUTE_MATRIX_MEM;
-    launch_line_m<T>(P, axis, mem, maxl, maxna, s, Bytes{comp, rhs_bytes + solve_bytes - (mem ? 0.0 : 2.0 * rec_bytes)});
+    launch_line_m<T>(P, axis, mem, maxl, maxna, s, Bytes{comp, rhs_bytes + solve_bytes + (mem ? rec_bytes + scr_bytes : 0.0)});
     return;
   }
+  rhs_bytes += rec_bytes;
+  solve_bytes += scr_bytes;
   if (axis == 0) {
     int maxn = 0;
     for (int j = 0; j < P.njobs; j++) maxn = std::max(maxn, P.job[j].L.n[0]);
